@@ -20,7 +20,7 @@
 //  iteration; the stop test is the true FP64 residual.
 //
 //  All scalars live on the device; reductions are two-level and
-//  deterministic (per-block partials, the last block sums them in a fixed
+//  deterministic (per-block partials, a one-block kernel sums them in a fixed
 //  order), so iterations need no host round trip.  The host only polls the
 //  'done' flag once per batch of iterations; a batch can be captured once in
 //  a hipGraph and replayed.
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(TPB) void k_cg_update64(int64_t n, double *__restri
                                                      const double *__restrict__ q,
                                                      const double *__restrict__ diag,
                                                      SolveScalars *sc, double *hist,
-                                                     double *partials, unsigned *counter) {
+                                                     double *partials) {
   if (sc->done) return;
   const double alpha = sc->alpha;
   double rr = 0., rz = 0.;
@@ -466,8 +466,7 @@ __global__ __launch_bounds__(TPB) void k_cg_init64(int64_t n, const double *__re
                                                    double *__restrict__ x, double *__restrict__ r,
                                                    double *__restrict__ z, double *__restrict__ p,
                                                    const double *__restrict__ diag,
-                                                   SolveScalars *sc, double *partials,
-                                                   unsigned *counter) {
+                                                   SolveScalars *sc, double *partials) {
   double bb = 0., rz = 0.;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
@@ -483,15 +482,19 @@ __global__ __launch_bounds__(TPB) void k_cg_init64(int64_t n, const double *__re
       rz += bi * zi;
     }
   }
-  double v[2] = {bb, rz}, tot[2];
-  if (reduce_last<2>(v, partials, counter, tot) && threadIdx.x == 0) {
-    double normb = sqrt(tot[0]);
+  double v[2] = {bb, rz};
+  block_partials<2>(v, partials);
+}
+__global__ void k_fin_cg_init64(SolveScalars *sc, const double *partials, int nblk) {
+  const double bb = sum_partials(partials, 0, nblk), rz = sum_partials(partials, 1, nblk);
+  if (threadIdx.x == 0) {
+    double normb = sqrt(bb);
     double resid = normb == 0. ? 0. : 1.0;
     if (normb == 0.) normb = 1.;
     sc->normb = normb;
     sc->resid = resid;
     sc->iter = 0;
-    sc->rho = tot[1];
+    sc->rho = rz;
     sc->beta = 0.;
     sc->done = resid <= sc->tol ? 1 : 0;
   }
@@ -504,8 +507,7 @@ __global__ __launch_bounds__(TPB) void k_cg_restart64(int64_t n, const double *_
                                                       const double *__restrict__ r,
                                                       double *__restrict__ z, double *__restrict__ p,
                                                       const double *__restrict__ diag,
-                                                      SolveScalars *sc, double *partials,
-                                                      unsigned *counter) {
+                                                      SolveScalars *sc, double *partials) {
   double ff = 0., rr = 0., rz = 0.;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
@@ -517,14 +519,19 @@ __global__ __launch_bounds__(TPB) void k_cg_restart64(int64_t n, const double *_
     rr += ri * ri;
     rz += ri * zi;
   }
-  double v[3] = {ff, rr, rz}, tot[3];
-  if (reduce_last<3>(v, partials, counter, tot) && threadIdx.x == 0) {
-    double normb = sqrt(tot[0]);
+  double v[3] = {ff, rr, rz};
+  block_partials<3>(v, partials);
+}
+__global__ void k_fin_cg_restart64(SolveScalars *sc, const double *partials, int nblk) {
+  const double ff = sum_partials(partials, 0, nblk), rr = sum_partials(partials, 1, nblk),
+               rz = sum_partials(partials, 2, nblk);
+  if (threadIdx.x == 0) {
+    double normb = sqrt(ff);
     if (normb == 0.) normb = 1.;
-    const double resid = sqrt(tot[1]) / normb;
+    const double resid = sqrt(rr) / normb;
     sc->normb = normb;
     sc->resid = resid;
-    sc->rho = tot[2];
+    sc->rho = rz;
     sc->beta = 0.;
     sc->done = resid <= sc->tol ? 1 : 0;
   }
@@ -537,8 +544,7 @@ __global__ __launch_bounds__(TPB) void k_residual64(int64_t nb, const int64_t *_
                                                     const double *__restrict__ v,
                                                     const double *__restrict__ u,
                                                     const double *__restrict__ f,
-                                                    double *__restrict__ r, double *out,
-                                                    double *partials, unsigned *counter) {
+                                                    double *__restrict__ r, double *partials) {
   const int sub = threadIdx.x % BSR_L;
   int64_t lo, hi;
   int xi, xg;
@@ -563,17 +569,23 @@ __global__ __launch_bounds__(TPB) void k_residual64(int64_t nb, const int64_t *_
       ff += f[i] * f[i];
     }
   }
-  double vv[2] = {rr, ff}, tot[2];
-  if (reduce_last<2>(vv, partials, counter, tot) && threadIdx.x == 0) {
-    out[0] = tot[0];
-    out[1] = tot[1];
+  double vv[2] = {rr, ff};
+  block_partials<2>(vv, partials);
+}
+// out = (|r|^2, |f|^2) from the residual's partials (one block; |r|^2 twice
+// when only slot 0 was written)
+__global__ void k_fin_residual64(const double *partials, int nblk, int nslot, double *out) {
+  const double rr = sum_partials(partials, 0, nblk);
+  const double ff = nslot > 1 ? sum_partials(partials, 1, nblk) : rr;
+  if (threadIdx.x == 0) {
+    out[0] = rr;
+    out[1] = ff;
   }
 }
 
 // the residual of u = 0: r = f, out = (|f|^2, |f|^2)
 __global__ __launch_bounds__(TPB) void k_residual_zero(int64_t n, const double *__restrict__ f,
-                                                       double *__restrict__ r, double *out,
-                                                       double *partials, unsigned *counter) {
+                                                       double *__restrict__ r, double *partials) {
   double ff = 0.;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -581,11 +593,8 @@ __global__ __launch_bounds__(TPB) void k_residual_zero(int64_t n, const double *
     r[i] = v;
     ff += v * v;
   }
-  double vv[1] = {ff}, tot[1];
-  if (reduce_last<1>(vv, partials, counter, tot) && threadIdx.x == 0) {
-    out[0] = tot[0];
-    out[1] = tot[0];
-  }
+  double vv[1] = {ff};
+  block_partials<1>(vv, partials);
 }
 
 __global__ void k_axpby64(int64_t n, double alpha, const double *__restrict__ x, double beta,
@@ -621,6 +630,10 @@ static int ensure_reduce(Ctx &c) {
 }
 int ensure_reduce_pub(Ctx &c) { return ensure_reduce(c); }
 
+static void fin_residual64(Ctx &c, const double *partials, int nblk, int nslot, double *out) {
+  hipLaunchKernelGGL(k_fin_residual64, dim3(1), dim3(TPB), 0, c.stream, partials, nblk, nslot, out);
+}
+
 int launch_multadd_upper(Ctx &c, const double *x, const double *y, double *z, double alpha,
                          double beta) {
   if (!c.full_valid) PZG_TRY(launch_expand_full(c));
@@ -642,8 +655,8 @@ int true_residual(Ctx &c, const double *u, double *rel) {
   DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(bsr_grid(c.nb)), dim3(TPB), 0,
                                        c.stream, c.nb, c.d_fbia.as<int64_t>(),
                                        c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), u,
-                                       c.d_f.as<double>(), nullptr, c.d_res2.as<double>(),
-                                       c.d_partials.as<double>(), c.d_counter.as<unsigned>()));
+                                       c.d_f.as<double>(), nullptr, c.d_partials.as<double>()));
+  fin_residual64(c, c.d_partials.as<double>(), bsr_grid(c.nb), 2, c.d_res2.as<double>());
   PZG_HIP(hipGetLastError());
   double h[2];
   PZG_HIP(hipMemcpyAsync(h, c.d_res2.p, sizeof(h), hipMemcpyDeviceToHost, c.stream));
@@ -655,12 +668,10 @@ int true_residual(Ctx &c, const double *u, double *rel) {
 // ---- allocation-free true residual ---------------------------------------
 // Fixed device scratch of pzg_true_residual_noalloc, one copy per GPU, held
 // until the process ends: the reduction partials (2 x MAXBLK doubles, one
-// slot per workgroup of the capped residual grid), the two sums and the
-// arrival counter.  32.8 KB whatever the system size, because the residual
+// slot per workgroup of the capped residual grid) and the two sums.  32.8 KB whatever the system size, because the residual
 // kernel strides over block rows with at most MAXBLK workgroups.
 constexpr int NOALLOC_PART = 2 * MAXBLK;           // partials, doubles
 constexpr int NOALLOC_OUT = NOALLOC_PART;          // |r|^2, |f|^2
-constexpr int NOALLOC_CNT = NOALLOC_PART + 4;      // counter (as unsigned)
 constexpr int NOALLOC_WORDS = NOALLOC_PART + 8;
 static __device__ __align__(256) double scratch[NOALLOC_WORDS];
 
@@ -687,11 +698,6 @@ int noalloc_scratch_setup(int device) {
   return PZG_OK;
 }
 
-__global__ void k_noalloc_clear(double *s) {
-  if (threadIdx.x < 2) s[NOALLOC_OUT + threadIdx.x] = 0.;
-  if (threadIdx.x == 0) *reinterpret_cast<unsigned *>(s + NOALLOC_CNT) = 0u;
-}
-
 // The residual of true_residual on the full block CSR already on the device,
 // reducing in the per-device scratch: no allocation of any kind.
 int true_residual_noalloc(Ctx &c, double *rel) {
@@ -711,12 +717,11 @@ int true_residual_noalloc(Ctx &c, double *rel) {
               " workgroups exceeds the scratch's " + std::to_string(NOALLOC_PART / 2));
     return PZG_EINVAL;
   }
-  hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(64), 0, c.stream, s);
   DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(grid), dim3(TPB), 0, c.stream, c.nb,
                                        c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
                                        c.d_fa.as<double>(), c.d_u.as<double>(),
-                                       c.d_f.as<double>(), nullptr, s + NOALLOC_OUT, s,
-                                       reinterpret_cast<unsigned *>(s + NOALLOC_CNT)));
+                                       c.d_f.as<double>(), nullptr, s));
+  fin_residual64(c, s, grid, 2, s + NOALLOC_OUT);
   PZG_HIP(hipGetLastError());
   double h[2];
   PZG_HIP(hipMemcpyAsync(h, s + NOALLOC_OUT, sizeof(h), hipMemcpyDeviceToHost, c.stream));
@@ -761,7 +766,6 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
   for (DevBuf *b : {&c.d_z, &c.d_p, &c.d_q}) PZG_TRY(dev_alloc(*b, n * sizeof(double)));
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
-  unsigned *cnt = c.d_counter.as<unsigned>();
   const int gv = grid_for(n, TPB), gs = bsr_grid(c.nb);
   for (int round = 0; round < 4 && rel > prm.tol && iters < prm.max_iter; round++) {
     SolveScalars hs;
@@ -772,7 +776,8 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
     PZG_HIP(hipMemcpyAsync(c.d_scal.p, &hs, sizeof(hs), hipMemcpyHostToDevice, c.stream));
     hipLaunchKernelGGL(k_cg_restart64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_f.as<double>(),
                        c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
-                       c.d_diag.as<double>(), sc, part, cnt);
+                       c.d_diag.as<double>(), sc, part);
+    hipLaunchKernelGGL(k_fin_cg_restart64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
     PZG_HIP(hipGetLastError());
     auto iter = [&]() {
       hipLaunchKernelGGL(k_p_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_z.as<double>(),
@@ -784,8 +789,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
       hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
       hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
                          c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
-                         c.d_q.as<double>(), c.d_diag.as<double>(), sc, (double *)nullptr, part,
-                         cnt);
+                         c.d_q.as<double>(), c.d_diag.as<double>(), sc, (double *)nullptr, part);
       hipLaunchKernelGGL(k_fin_cg64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv,
                          (double *)nullptr);
     };
@@ -797,7 +801,8 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
     DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(gs), dim3(TPB), 0, c.stream, c.nb,
                                          c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
                                          c.d_fa.as<double>(), c.d_u.as<double>(), c.d_f.as<double>(),
-                                         c.d_r.as<double>(), c.d_res2.as<double>(), part, cnt));
+                                         c.d_r.as<double>(), part));
+    fin_residual64(c, part, gs, 2, c.d_res2.as<double>());
     PZG_HIP(hipGetLastError());
     double h[2];
     PZG_HIP(hipMemcpyAsync(h, c.d_res2.p, sizeof(h), hipMemcpyDeviceToHost, c.stream));
@@ -821,7 +826,6 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
   PZG_HIP(hipEventRecord(c.ev0, c.stream));
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
-  unsigned *cnt = c.d_counter.as<unsigned>();
   const int gv = grid_for(n, TPB);
   // EJacobi (reference default) or the connect-block Jacobi of
   // BuildPreconditioner(EBlockJacobi): blocks of one connect's nstate
@@ -878,7 +882,8 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
   const double *dg = block ? nullptr : c.d_diag.as<double>();
   hipLaunchKernelGGL(k_cg_init64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_f.as<double>(),
                      c.d_u.as<double>(), c.d_r.as<double>(), c.d_z.as<double>(),
-                     c.d_p.as<double>(), dg, sc, part, cnt);
+                     c.d_p.as<double>(), dg, sc, part);
+  hipLaunchKernelGGL(k_fin_cg_init64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
   auto vbj_apply = [&](const SolveScalars *s2) {
     hipLaunchKernelGGL(k_vbj_apply64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_vbj_eqb.as<int32_t>(),
                        c.d_vbj_pos.as<int64_t>(), c.d_vbj_m.as<int32_t>(), c.d_vbj_off.as<int64_t>(),
@@ -906,8 +911,7 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
     hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
     hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
                        c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
-                       c.d_q.as<double>(), dg, sc, (double *)nullptr, part,
-                       cnt);
+                       c.d_q.as<double>(), dg, sc, (double *)nullptr, part);
     if (vblock)
       vbj_apply(sc);
     else if (block)
@@ -1001,8 +1005,7 @@ __global__ __launch_bounds__(TPB) void k_fcg_update(int64_t nb, float *__restric
                                                     const float *__restrict__ p,
                                                     const float *__restrict__ q,
                                                     const float *__restrict__ binv,
-                                                    SolveScalars *sc, double *partials,
-                                                    unsigned *counter) {
+                                                    SolveScalars *sc, double *partials) {
   if (sc->done) return;
   const float alpha = (float)sc->alpha;
   double rr = 0., zq = 0.;
@@ -1077,8 +1080,7 @@ __global__ __launch_bounds__(TPB) void k_fcg_init(int64_t nb, const double *__re
                                                   float *__restrict__ x, float *__restrict__ r,
                                                   float *__restrict__ z, float *__restrict__ p,
                                                   const float *__restrict__ binv,
-                                                  SolveScalars *sc, double *partials,
-                                                  unsigned *counter) {
+                                                  SolveScalars *sc, double *partials) {
   double bb = 0.;
   int64_t A = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
@@ -1101,9 +1103,13 @@ __global__ __launch_bounds__(TPB) void k_fcg_init(int64_t nb, const double *__re
       p[A * BS + k] = s;
     }
   }
-  double vv[1] = {bb}, tot[1];
-  if (reduce_last<1>(vv, partials, counter, tot) && threadIdx.x == 0) {
-    double nbv = sqrt(tot[0]);
+  double vv[1] = {bb};
+  block_partials<1>(vv, partials);
+}
+__global__ void k_fin_fcg_init(SolveScalars *sc, const double *partials, int nblk) {
+  const double bb = sum_partials(partials, 0, nblk);
+  if (threadIdx.x == 0) {
+    double nbv = sqrt(bb);
     sc->normb = nbv > 0. ? nbv : 1.;
     sc->rlast = nbv;
     sc->resid = nbv > 0. ? 1. : 0.;
@@ -1126,9 +1132,7 @@ __global__ void k_ir_update(int64_t n, float *__restrict__ y, const double *__re
 // direction p is kept
 __global__ __launch_bounds__(TPB) void k_fcg_reset(int64_t n, const double *__restrict__ r64,
                                                    const double *__restrict__ dis,
-                                                   float *__restrict__ r, double delta,
-                                                   SolveScalars *sc, double *partials,
-                                                   unsigned *counter) {
+                                                   float *__restrict__ r, double *partials) {
   double bb = 0.;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
@@ -1137,9 +1141,13 @@ __global__ __launch_bounds__(TPB) void k_fcg_reset(int64_t n, const double *__re
     r[i] = v;
     bb += (double)v * v;
   }
-  double vv[1] = {bb}, tot[1];
-  if (reduce_last<1>(vv, partials, counter, tot) && threadIdx.x == 0) {
-    sc->rlast = sqrt(tot[0]);
+  double vv[1] = {bb};
+  block_partials<1>(vv, partials);
+}
+__global__ void k_fin_fcg_reset(SolveScalars *sc, const double *partials, int nblk, double delta) {
+  const double bb = sum_partials(partials, 0, nblk);
+  if (threadIdx.x == 0) {
+    sc->rlast = sqrt(bb);
     sc->delta = delta;
     sc->done = 0;
   }
@@ -1188,7 +1196,6 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
   double *out = c.d_res2.as<double>();
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
-  unsigned *cnt = c.d_counter.as<unsigned>();
   const int gv = grid_for(n, TPB), gb = grid_for(nb, TPB), gs = bsr_grid(nb);
   PZG_HIP(hipEventRecord(c.ev0, c.stream));
   hipLaunchKernelGGL(k_axpby64, dim3(gv), dim3(TPB), 0, c.stream, n, 0.0, c.d_f.as<double>(), 0.0,
@@ -1202,12 +1209,12 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
   auto true_res = [&](bool u_zero = false) -> int {
     if (u_zero)  // the starting guess: no product needed
       hipLaunchKernelGGL(k_residual_zero, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_f.as<double>(),
-                         c.d_r.as<double>(), out, part, cnt);
+                         c.d_r.as<double>(), part);
     else
       hipLaunchKernelGGL(k_residual64<BS>, dim3(bsr_grid(nb)), dim3(TPB), 0, c.stream, nb,
                          c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
-                         c.d_u.as<double>(), c.d_f.as<double>(), c.d_r.as<double>(), out,
-                         part, cnt);
+                         c.d_u.as<double>(), c.d_f.as<double>(), c.d_r.as<double>(), part);
+    fin_residual64(c, part, u_zero ? gv : bsr_grid(nb), u_zero ? 1 : 2, out);
     double h[2];
     PZG_HIP(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, c.stream));
     PZG_HIP(hipStreamSynchronize(c.stream));
@@ -1325,7 +1332,8 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
       hipLaunchKernelGGL(k_fcg_init<BS>, dim3(gb), dim3(TPB), 0, c.stream, nb, c.d_r.as<double>(),
                          c.d_dinvsqrt.as<double>(), c.d_xs.as<float>(), c.d_rs.as<float>(),
                          c.d_zs.as<float>(), c.d_ps.as<float>(),
-                         multigrid ? (const float *)nullptr : c.d_bjinv.as<float>(), sc, part, cnt);
+                         multigrid ? (const float *)nullptr : c.d_bjinv.as<float>(), sc, part);
+      hipLaunchKernelGGL(k_fin_fcg_init, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb);
       PZG_HIP(hipGetLastError());
       if (pen_rows) PZG_TRY(pen_zero32(c, c.d_rs.as<float>()));
       if (multigrid)
@@ -1347,8 +1355,7 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
       hipLaunchKernelGGL(k_fin_fcg_alpha, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, ga);
       hipLaunchKernelGGL(k_fcg_update<BS>, dim3(gb), dim3(TPB), 0, c.stream, nb,
                          c.d_xs.as<float>(), c.d_rs.as<float>(), c.d_zs.as<float>(),
-                         c.d_ps.as<float>(), c.d_qs.as<float>(), c.d_bjinv.as<float>(), sc, part,
-                         cnt);
+                         c.d_ps.as<float>(), c.d_qs.as<float>(), c.d_bjinv.as<float>(), sc, part);
       // S couples the penalty rows to the others (at the 1/sqrt(big) level):
       // keep their residual at zero rather than let it drift
       if (pen_rows) (void)pen_zero32(c, c.d_rs.as<float>());
@@ -1399,7 +1406,8 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
     prev_rel = rel;
     if (hs.done == 3 || prm.refine == 0) { restart = true; continue; }
     hipLaunchKernelGGL(k_fcg_reset, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_r.as<double>(),
-                       c.d_dinvsqrt.as<double>(), c.d_rs.as<float>(), next_delta(), sc, part, cnt);
+                       c.d_dinvsqrt.as<double>(), c.d_rs.as<float>(), part);
+    hipLaunchKernelGGL(k_fin_fcg_reset, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv, next_delta());
     PZG_HIP(hipGetLastError());
     if (pen_rows) PZG_TRY(pen_zero32(c, c.d_rs.as<float>()));
   }
