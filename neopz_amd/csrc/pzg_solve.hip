@@ -1032,23 +1032,30 @@ __global__ __launch_bounds__(TPB) void k_fcg_update(int64_t nb, float *__restric
   block_partials<2>(vv, partials);
 }
 
-// stop tests on |r|; beta = -(z.q)/(p.q)   (one block; slot 1 may have been
-// rewritten by the learned preconditioner's prolongation)
-__global__ void k_fin_fcg_beta(SolveScalars *sc, const double *partials, int nblk) {
+// stop tests on |r| (what & 1), beta = -(z.q)/(p.q) (what & 2)   (one block;
+// slot 1 may have been rewritten by the preconditioner).  Under the multigrid
+// cycle of a restarted FCG the stop test runs alone before the cycle (what =
+// 1, update due = 5: no kernel of this iteration is left to run), since the
+// restart recomputes z: the last cycle of every refinement step is not run
+// (3 of 23 cycles on a 256^2 Darcy solve, 3 of 87 at 48^3, 3 of 38 at 64^3
+// with the learned smoother).
+__global__ void k_fin_fcg_beta(SolveScalars *sc, const double *partials, int nblk, int what) {
   if (sc->done) return;
-  double rr = sum_partials(partials, 0, nblk);
-  double zq = sum_partials(partials, 1, nblk);
+  double rr = what & 1 ? sum_partials(partials, 0, nblk) : 0.;
+  double zq = what & 2 ? sum_partials(partials, 1, nblk) : 0.;
   if (threadIdx.x == 0) {
-    int64_t it = sc->iter + 1;
-    sc->iter = it;
-    double rn = sqrt(rr);
-    double resid = rn / sc->normb;
-    // divergence guard: leave the loop, the host restarts from the true residual
-    if (!(resid == resid) || resid > 1e3) sc->done = 3;
-    else if (rn < sc->delta * sc->rlast) sc->done = 4;
-    else if (it >= sc->maxit) sc->done = 2;
-    sc->resid = resid;
-    sc->beta = -zq / sc->pq;
+    if (what & 1) {
+      int64_t it = sc->iter + 1;
+      sc->iter = it;
+      double rn = sqrt(rr);
+      double resid = rn / sc->normb;
+      // divergence guard: leave the loop, the host restarts from the true residual
+      if (!(resid == resid) || resid > 1e3) sc->done = 3;
+      else if (rn < sc->delta * sc->rlast) sc->done = what & 2 ? 4 : 5;
+      else if (it >= sc->maxit) sc->done = 2;
+      sc->resid = resid;
+    }
+    if (what & 2) sc->beta = -zq / sc->pq;
   }
 }
 
@@ -1359,10 +1366,13 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
       // S couples the penalty rows to the others (at the 1/sqrt(big) level):
       // keep their residual at zero rather than let it drift
       if (pen_rows) (void)pen_zero32(c, c.d_rs.as<float>());
+      const bool early = multigrid && prm.refine == 0;
+      if (early)
+        hipLaunchKernelGGL(k_fin_fcg_beta, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb, 1);
       if (multigrid)
         (void)mg_apply(c, c.d_rs.as<float>(), c.d_zs.as<float>(), nullptr, c.d_qs.as<float>(), sc, part);
       if (vbj) vbj_apply(c.d_zs.as<float>(), nullptr, c.d_qs.as<float>());
-      hipLaunchKernelGGL(k_fin_fcg_beta, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb);
+      hipLaunchKernelGGL(k_fin_fcg_beta, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb, early ? 2 : 3);
       hipLaunchKernelGGL(k_p_update32, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_zs.as<float>(),
                          c.d_ps.as<float>(), sc, use_mf ? c.d_mf_dis.as<float>() : nullptr,
                          use_mf ? c.d_mf_pt.as<float>() : nullptr);
