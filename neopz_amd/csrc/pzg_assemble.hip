@@ -1785,7 +1785,8 @@ __global__ void k_nlow(int64_t nb, const int64_t *__restrict__ fbia, const int64
 // nlow[A] = number of lower blocks of block row A (= rank of its diagonal block)
 
 
-// Row-gather form of the expansion: one wavefront per block row A writes the
+// Row-gather form of the expansion: one wavefront per block row A (of the nb
+// first, or of the list rows) writes the
 // row's storage in order (coalesced), each lane one value.  Upper blocks
 // come from row A's scalar rows, lower blocks (A, B), B < A, from the upper
 // block (B, A) in row B (lowsrc: its index among the upper blocks).  SCALED:
@@ -1797,10 +1798,12 @@ __global__ __launch_bounds__(256) void k_bsr_gather(int64_t nb, const int64_t *_
                                                     const int64_t *__restrict__ fbia,
                                                     const int32_t *__restrict__ fbja,
                                                     const int32_t *__restrict__ lowsrc,
-                                                    const double *__restrict__ dis, T *__restrict__ v) {
-  const int64_t A = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+                                                    const double *__restrict__ dis, T *__restrict__ v,
+                                                    const int32_t *__restrict__ rows) {
+  const int64_t w = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
-  if (A >= nb) return;
+  if (w >= nb) return;
+  const int64_t A = rows ? rows[w] : w;
   constexpr int BB = BS * BS;
   const int64_t b0 = fbia[A], u0 = ubia[A];
   const int n = (int)(fbia[A + 1] - b0), nl = n - 1 - (int)(ubia[A + 1] - u0);
@@ -1883,30 +1886,37 @@ static int ensure_lowsrc(Ctx &c) {
   return PZG_OK;
 }
 
-int launch_expand_full(Ctx &c) {
+static int expand_rows(Ctx &c, const int32_t *rows, int64_t nrows) {
   const int bs = c.bs;
   PZG_TRY(dev_alloc(c.d_fa, sizeof(double) * c.nbf * bs * bs));
   PZG_TRY(ensure_lowsrc(c));
-  const int64_t threads = c.nb * 64;
+  const int64_t threads = nrows * 64;
   const dim3 g((unsigned)((threads + TPB - 1) / TPB));
   if (bs == 3)
-    hipLaunchKernelGGL((k_bsr_gather<3, double, false>), g, dim3(TPB), 0, c.stream, c.nb, c.d_ia.as<int64_t>(),
+    hipLaunchKernelGGL((k_bsr_gather<3, double, false>), g, dim3(TPB), 0, c.stream, nrows, c.d_ia.as<int64_t>(),
                        c.d_a.as<double>(), c.d_ubia.as<int64_t>(), c.d_fbia.as<int64_t>(),
                        c.d_fbja.as<int32_t>(), c.d_lowsrc.as<int32_t>(), (const double *)nullptr,
-                       c.d_fa.as<double>());
+                       c.d_fa.as<double>(), rows);
   else if (bs == 1)
-    hipLaunchKernelGGL((k_bsr_gather<1, double, false>), g, dim3(TPB), 0, c.stream, c.nb, c.d_ia.as<int64_t>(),
+    hipLaunchKernelGGL((k_bsr_gather<1, double, false>), g, dim3(TPB), 0, c.stream, nrows, c.d_ia.as<int64_t>(),
                        c.d_a.as<double>(), c.d_ubia.as<int64_t>(), c.d_fbia.as<int64_t>(),
                        c.d_fbja.as<int32_t>(), c.d_lowsrc.as<int32_t>(), (const double *)nullptr,
-                       c.d_fa.as<double>());
+                       c.d_fa.as<double>(), rows);
   else {
     set_error("block CSR: unsupported block size");
     return PZG_EUNSUP;
   }
   PZG_HIP(hipGetLastError());
+  return PZG_OK;
+}
+int launch_expand_full(Ctx &c) {
+  PZG_TRY(expand_rows(c, nullptr, c.nb));
   PZG_HIP(hipStreamSynchronize(c.stream));
   c.full_valid = true;
   return PZG_OK;
+}
+int launch_expand_rows(Ctx &c, const int32_t *d_rows, int64_t nrows) {
+  return nrows > 0 ? expand_rows(c, d_rows, nrows) : PZG_OK;
 }
 
 // --------------------------------------------------------------------------
@@ -2027,7 +2037,7 @@ int launch_build_bsr(Ctx &c, bool values) {
       hipLaunchKernelGGL((k_bsr_gather<3, float, true>), dim3((threads + TPB - 1) / TPB), dim3(TPB), 0, c.stream,
                          c.nb, c.d_ia.as<int64_t>(), c.d_a.as<double>(), c.d_ubia.as<int64_t>(),
                          c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_lowsrc.as<int32_t>(),
-                         c.d_dinvsqrt.as<double>(), c.d_bsr.as<float>());
+                         c.d_dinvsqrt.as<double>(), c.d_bsr.as<float>(), (const int32_t *)nullptr);
   } else if (bs == 1) {
     hipLaunchKernelGGL(k_bsr_diag<1>, dim3((c.nb + TPB - 1) / TPB), dim3(TPB), 0, c.stream, c.nb,
                        c.nbf, c.d_ia.as<int64_t>(), c.d_a.as<double>(), nl.as<int32_t>(),
@@ -2036,7 +2046,7 @@ int launch_build_bsr(Ctx &c, bool values) {
       hipLaunchKernelGGL((k_bsr_gather<1, float, true>), dim3((threads + TPB - 1) / TPB), dim3(TPB), 0, c.stream,
                          c.nb, c.d_ia.as<int64_t>(), c.d_a.as<double>(), c.d_ubia.as<int64_t>(),
                          c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_lowsrc.as<int32_t>(),
-                         c.d_dinvsqrt.as<double>(), c.d_bsr.as<float>());
+                         c.d_dinvsqrt.as<double>(), c.d_bsr.as<float>(), (const int32_t *)nullptr);
   } else {
     dev_free(nl);
     set_error("block CSR: unsupported block size");

@@ -60,7 +60,7 @@ static void free_all(Ctx &c) {
                     &c.d_fa, &c.d_bsr, &c.d_dinvsqrt, &c.d_bjinv, &c.d_xyz, &c.d_vnodes,
                     &c.d_vconn, &c.d_vcoef, &c.d_bnodes, &c.d_bconn, &c.d_bcid, &c.d_bctype,
                     &c.d_bcval, &c.d_bccoef, &c.d_bcvec, &c.d_aidx, &c.d_bumps, &c.d_vmap, &c.d_bmap, &c.d_tvol,
-                    &c.d_tbc, &c.d_vcolor_list, &c.d_vol_R, &c.d_blk_iptr, &c.d_blk_inc, &c.d_blk_kref, &c.d_vbj_pos, &c.d_vbj_m, &c.d_vbj_off, &c.d_vbj_eqb, &c.d_vbjinv64, &c.d_vbjinv32, &c.d_bcolor_list, &c.d_x, &c.d_r, &c.d_z,
+                    &c.d_tbc, &c.d_vcolor_list, &c.d_vol_R, &c.d_blk_iptr, &c.d_blk_inc, &c.d_blk_kref, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab, &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_vbj_pos, &c.d_vbj_m, &c.d_vbj_off, &c.d_vbj_eqb, &c.d_vbjinv64, &c.d_vbjinv32, &c.d_bcolor_list, &c.d_x, &c.d_r, &c.d_z,
                     &c.d_p, &c.d_p2, &c.d_q, &c.d_u, &c.d_f, &c.d_w, &c.d_xs, &c.d_rs,
                     &c.d_zs, &c.d_ps, &c.d_ps2, &c.d_qs, &c.d_bs, &c.d_scal, &c.d_partials,
                     &c.d_counter, &c.d_res2, &c.d_les_th, &c.d_les_m, &c.d_les_v, &c.d_les_g,
@@ -345,6 +345,9 @@ static int blk_setup(Ctx &c, const std::vector<double> &R) {
   PZG_TRY(dev_upload(c.d_blk_kref, K.data(), K.size(), s));
   PZG_TRY(dev_upload(c.d_blk_iptr, iptr.data(), iptr.size(), s));
   PZG_TRY(dev_upload(c.d_blk_inc, inc.data(), inc.size(), s));
+  c.blk_kref.swap(K);
+  c.blk_full = iptr[c.nb] == c.nvol * NSH;
+  for (int sh = 0; sh < NSH; sh++) c.blk_full &= T.shape_side[sh] == sh;
   c.blk_asm = true;
   c.blk_grid = 0;
   return PZG_OK;
@@ -1075,7 +1078,7 @@ static int struct_create(Ctx &c) {
   // colour: the assembly integrates them from the rule's reference Gram
   // matrices (k_vol_aff); single-rule quad/hex meshes only
   c.vcolor_aff.clear();
-  c.blk_asm = false;
+  c.blk_asm = c.blk_full = c.kf_struct = false;
   c.aff_on = !(std::getenv("PZG_NO_AFFINE") && std::getenv("PZG_NO_AFFINE")[0] == '1');
   if (c.vol_rules.size() == 1 && !c.hp_simplex && c.vol_etype != PZG_TET &&
       ((c.dim == 3 && c.vol_ncorner == 8) || (c.dim == 2 && c.vol_ncorner == 4))) {
@@ -1140,7 +1143,7 @@ static int struct_create(Ctx &c) {
   c.kel_added = false;
   c.mf_ready = c.mf_vals_valid = false;
   c.les_tile_ready = c.les_tile_ok = false;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   c.has_solution = c.f_valid = false;
   return PZG_OK;
 }
@@ -1254,7 +1257,7 @@ int pzg_set_equation_filter(pzg_ctx *ctx, int64_t nactive, const int64_t *active
   c.has_solution = c.f_valid = false;
   c.mf_ready = c.mf_vals_valid = false;
   c.les_tile_ready = c.les_tile_ok = false;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   mg_free(c);
   return PZG_OK;
 }
@@ -1304,7 +1307,7 @@ int pzg_assemble(pzg_ctx *ctx) {
   PZG_TRY(launch_diag(c));
   c.assembled = true;
   c.kel_added = false;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   c.has_solution = c.f_valid = false;
   return PZG_OK;
 }
@@ -1478,7 +1481,7 @@ int pzg_csr_set(pzg_ctx *ctx, int64_t neq, const int64_t *ia, const int64_t *ja,
   c.mf_ready = c.mf_vals_valid = false;
   c.les_tile_ready = c.les_tile_ok = false;
   c.assembled = true;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   c.has_solution = c.f_valid = false;
   return PZG_OK;
 }
@@ -1543,7 +1546,7 @@ int pzg_add_kel_batch(pzg_ctx *ctx, int64_t nel, int32_t ne, const int64_t *dest
   dev_free(d_list);
   c.assembled = true;
   c.kel_added = true;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   c.mg_ready = c.pen_ready = false;  // both are built from K
   return rc;
 }
@@ -1869,7 +1872,6 @@ int pzg_mg_apply(pzg_ctx *ctx, int32_t op, int32_t degree, double range, const d
     return PZG_ESTATE;
   }
   const int64_t n = c.neq;
-  if (!c.full_valid) PZG_TRY(launch_expand_full(c));
   if (!c.bsr_valid) PZG_TRY(launch_build_bsr(c));
   if (op == PZG_INNER_MATFREE) PZG_TRY(mf_prepare(c));
   PZG_TRY(ensure_reduce_pub(c));
@@ -1912,7 +1914,7 @@ int pzg_mesh_set_coef(pzg_ctx *ctx, const double *vol_coef) {
   PZG_TRY(dev_upload(c.d_vcoef, c.vol_coef.data(), c.vol_coef.size(), c.stream));
   PZG_HIP(hipStreamSynchronize(c.stream));
   c.assembled = false;
-  c.full_valid = c.bsr_valid = c.scal_valid = false;
+  c.full_valid = c.bsr_valid = c.scal_valid = c.kf_valid = false;
   c.has_solution = c.f_valid = false;
   return PZG_OK;
 }

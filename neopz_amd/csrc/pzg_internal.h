@@ -243,6 +243,14 @@ struct Ctx {
   bool blk_asm = false;
   int blk_grid = 0;
   DevBuf d_blk_iptr, d_blk_inc, d_blk_kref;
+  bool blk_full = false;          // every shape of every element is active
+  std::vector<double> blk_kref;   // the coefficient-1 element matrix
+  // FP64 products from the element matrix (pzg_matfree64.hip): mesh part,
+  // validity for the assembled system, entries dropped by AddKel for every
+  // element (-1: tables not uploaded)
+  bool kf_struct = false, kf_valid = false;
+  int64_t kf_nface = 0, kf_ndrop = -1;
+  DevBuf d_kf_blk, d_kf_ye, d_kf_tab, d_kf_bblk, d_kf_bm, d_kf_pidx, d_kf_pptr, d_kf_psrc;
   int64_t nb = 0;  // active blocks
 
   // constrained connects (hanging sides): dependencies per connect, and the
@@ -407,6 +415,8 @@ int launch_diag(Ctx &c);
 // decouples the inactive equations of the equation filter (mesh numbering)
 int launch_filter_mask(Ctx &c);
 int launch_expand_full(Ctx &c);
+// the listed block rows of the full block CSR only (full_valid stays as it is)
+int launch_expand_rows(Ctx &c, const int32_t *d_rows, int64_t nrows);
 // equation-level full CSR (device arrays, any may be null; ia without ia[neq])
 int launch_full_csr(Ctx &c, int64_t *d_ia, int64_t *d_ja, double *d_a);
 // D^-1/2 and the block-Jacobi inverses of S; values: also the FP32 block CSR of S
@@ -466,6 +476,19 @@ inline bool mf_available(const Ctx &c) {
          !c.filt &&
          c.vol_rules.size() == 1 && c.bc_rules.size() <= 1 && c.vol_etype != PZG_TET && c.bc_mf_ok;
 }
+// FP64 products with K from the coefficient-1 element matrix
+// (pzg_matfree64.hip).  kf_prepare: *ok when they stand for the block CSR's on
+// the assembled system.  kf_apply: KF_AXPBY out = alpha K x + beta f (f may be
+// null), KF_DOT out = K x with x.(K x) in partials slot 0, KF_RESIDUAL out =
+// f - K x (out may be null) with |out|^2, |f|^2 in slots 0 and 1; partials of
+// kf_rows_grid blocks.
+enum { KF_AXPBY = 0, KF_DOT = 1, KF_RESIDUAL = 2 };
+constexpr int64_t KF_SPLIT_TILES = 4096;  // fewer element tiles of 16: three wavefronts per tile
+bool kf_usable(const Ctx &c);
+int kf_prepare(Ctx &c, bool *ok);
+int kf_rows_grid(const Ctx &c);
+int kf_apply(Ctx &c, int mode, const double *x, const double *f, double alpha, double beta, double *out,
+             const SolveScalars *sc, double *partials);
 int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info);
 int solve_mixed(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info);
 int true_residual(Ctx &c, const double *u, double *rel);

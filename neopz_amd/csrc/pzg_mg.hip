@@ -9,7 +9,7 @@
 // the trilinear ones, edge/face/interior functions vanish at the vertices)
 // make it the span of the vertex functions, so its prolongation is the
 // injection of vertex values and its Galerkin operator P^T K P is the
-// vertex-vertex part K_vv of the assembled K, read from the FP64 block CSR.
+// vertex-vertex part K_vv of the assembled K, read from its upper CSR.
 // In level 0's scaled unknowns the transfer carries D^1/2 at the vertex
 // equations.  Level 1 is stored in lattice order as a 27-point block
 // stencil.  Levels 2.. halve the lattice with trilinear prolongation and the
@@ -326,41 +326,55 @@ __global__ __launch_bounds__(TPB) void k_mg_finish(int64_t nb, const float *__re
 }
 
 // ---- set-up kernels --------------------------------------------------------------
-// level 1 stencil from the FP64 full block CSR (values at bsr_pos): block
-// (vmap[v], vmap[w]) for the lattice neighbour w of v in direction s (zero
-// off the lattice or when the row does not hold the column).  One wavefront
-// per vertex v scans its block row once: vinv maps a block to its vertex (-1
-// for the other connects); the directions found are gathered in a mask so
-// that the zero entries and the found ones are written by disjoint stores.
+// level 1 stencil from the assembled upper CSR: block (vmap[v], vmap[w]) for
+// the lattice neighbour w of v in direction s, its transpose at w in the
+// opposite direction.  One wavefront per vertex v scans the upper blocks of
+// its block row once: vinv maps a block to its vertex (-1 for the other
+// connects).  A must hold zeros (directions off the lattice or without a
+// stored block).  Reads half of the rows that a scan of the full block CSR
+// reads, and that format is not needed for the cycle.
 template <int BS>
 __global__ void k_mg_l1(Dims D, int64_t nn, const int32_t *__restrict__ vmap, const int32_t *__restrict__ vinv,
-                        const int64_t *__restrict__ fbia, const int32_t *__restrict__ fbja,
-                        const double *__restrict__ fa, float *__restrict__ A) {
+                        const int64_t *__restrict__ ia, const double *__restrict__ a,
+                        const int64_t *__restrict__ ubia, const int32_t *__restrict__ ubja,
+                        float *__restrict__ A) {
   constexpr int BB = BS * BS;
   const int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   if (v >= nn) return;
+  const int64_t row = vmap[v];
+  if (row < 0) return;
   int i, j, k;
   node_ijk(D, v, i, j, k);
-  const int64_t row = vmap[v];
-  const int64_t b0 = row >= 0 ? fbia[row] : 0, nr = row >= 0 ? fbia[row + 1] - b0 : 0;
-  int found = 0;
-  for (int64_t q = lane; q < nr; q += 64) {
-    const int32_t w = vinv[fbja[b0 + q]];
+  int64_t ra[BS];
+#pragma unroll
+  for (int e = 0; e < BS; e++) ra[e] = ia[row * BS + e];
+  if (lane < BB) {
+    const int p = lane / BS, q = lane % BS, lo = p < q ? p : q, hi = p < q ? q : p;
+    A[((int64_t)13 * BB + lane) * nn + v] = (float)a[ia[row * BS + lo] + (hi - lo)];
+  }
+  const int64_t u0 = ubia[row], nu = ubia[row + 1] - u0;
+  for (int64_t q = lane; q < nu; q += 64) {
+    const int32_t w = vinv[ubja[u0 + q]];
     if (w < 0) continue;
     int ii, jj, kk;
     node_ijk(D, w, ii, jj, kk);
     const int di = ii - i, dj = jj - j, dk = kk - k;
     if (di < -1 || di > 1 || dj < -1 || dj > 1 || dk < -1 || dk > 1) continue;
     const int sd = (di + 1) + 3 * (dj + 1) + 9 * (dk + 1);
-    found |= 1 << sd;
-    for (int e = 0; e < BB; e++) A[((int64_t)sd * BB + e) * nn + v] = (float)fa[bsr_pos<BB>(b0, nr, q, e)];
+#pragma unroll
+    for (int e = 0; e < BS; e++)
+#pragma unroll
+      for (int f = 0; f < BS; f++) {
+        const float x = (float)a[ra[e] + (BS - e) + q * BS + f];
+        A[((int64_t)sd * BB + e * BS + f) * nn + v] = x;
+        A[((int64_t)(26 - sd) * BB + f * BS + e) * nn + w] = x;
+      }
   }
-  for (int o = 32; o > 0; o >>= 1) found |= __shfl_xor(found, o, 64);
-  for (int t = lane; t < 27 * BB; t += 64) {
-    const int sd = t / BB;
-    if (!((found >> sd) & 1)) A[(int64_t)t * nn + v] = 0.f;
-  }
+}
+__global__ void k_mg_zero(int64_t n, float *__restrict__ x) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    x[i] = 0.f;
 }
 
 // Galerkin product A_c = P^T A_f P for trilinear P, one thread per coarse
@@ -911,9 +925,11 @@ int setup_impl(Ctx &c) {
   const int64_t nn1 = c.mg[0].nn;
   hipLaunchKernelGGL(k_mg_dsq<BS>, dim3(gridx(nn1)), dim3(TPB), 0, c.stream, nn1, c.d_mg_vmap.as<int32_t>(),
                      c.d_dinvsqrt.as<double>(), c.d_mg_dsq.as<float>());
+  hipLaunchKernelGGL(k_mg_zero, dim3(gridr(27 * BS * BS * nn1)), dim3(TPB), 0, c.stream, 27 * BS * BS * nn1,
+                     c.mg[0].A.as<float>());
   hipLaunchKernelGGL(k_mg_l1<BS>, dim3(gridx(64 * nn1)), dim3(TPB), 0, c.stream, dims_of(c.mg[0]), nn1,
-                     c.d_mg_vmap.as<int32_t>(), c.d_mg_vinv.as<int32_t>(), c.d_fbia.as<int64_t>(),
-                     c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), c.mg[0].A.as<float>());
+                     c.d_mg_vmap.as<int32_t>(), c.d_mg_vinv.as<int32_t>(), c.d_ia.as<int64_t>(),
+                     c.d_a.as<double>(), c.d_ubia.as<int64_t>(), c.d_ubja.as<int32_t>(), c.mg[0].A.as<float>());
   PZG_HIP(hipGetLastError());
   for (size_t k = 1; k < c.mg.size(); k++) {
     hipLaunchKernelGGL(k_mg_rap<BS>, dim3(gridx(27 * BS * BS * c.mg[k].nn)), dim3(TPB), 0, c.stream, dims_of(c.mg[k]),

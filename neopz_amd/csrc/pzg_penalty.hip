@@ -59,7 +59,8 @@ __global__ void k_pen_count(int64_t np, int bs, const int64_t *__restrict__ idx,
 }
 
 // K_pp in CSR over the penalty numbering (columns ascending: blocks ascend
-// along the full block row and the numbering follows the equations)
+// along the full block row and the numbering follows the equations); the
+// pattern alone when fa is null
 template <int BS>
 __global__ void k_pen_fill(int64_t np, const int64_t *__restrict__ idx, const int64_t *__restrict__ fbia,
                            const int32_t *__restrict__ fbja, const double *__restrict__ fa,
@@ -76,7 +77,7 @@ __global__ void k_pen_fill(int64_t np, const int64_t *__restrict__ idx, const in
       const int32_t pj = pmap[(int64_t)fbja[b0 + q] * BS + l];
       if (pj < 0) continue;
       ja[o] = pj;
-      a[o] = fa[bsr_pos<BS * BS>(b0, n, q, ci * BS + l)];
+      if (fa) a[o] = fa[bsr_pos<BS * BS>(b0, n, q, ci * BS + l)];
       o++;
     }
 }
@@ -369,6 +370,7 @@ static int pen_fill(Ctx &c);
 // K_pp's CSR pattern, the Schwarz sets of the penalized boundary elements with
 // the CSR position of every entry of their dense blocks, and the row -> slot
 // gather.
+static int pen_fill(Ctx &c, const double *fa);
 static int pen_structure(Ctx &c) {
   const int bs = c.bs;
   std::vector<int64_t> idx;
@@ -411,7 +413,7 @@ static int pen_structure(Ctx &c) {
   PZG_TRY(dev_upload(c.d_pen_ia, ia.data(), ia.size(), s));
   PZG_TRY(dev_alloc(c.d_pen_ja, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
   PZG_TRY(dev_alloc(c.d_pen_a, sizeof(double) * std::max<int64_t>(nnz, 1)));
-  PZG_TRY(pen_fill(c));
+  PZG_TRY(pen_fill(c, nullptr));
   std::vector<int32_t> ja(std::max<int64_t>(nnz, 1));
   PZG_HIP(hipMemcpyAsync(ja.data(), c.d_pen_ja.p, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, s));
   PZG_HIP(hipStreamSynchronize(s));
@@ -510,18 +512,18 @@ static int pen_structure(Ctx &c) {
   return PZG_OK;
 }
 
-// K_pp values of the current assembly (pattern of pen_structure)
-static int pen_fill(Ctx &c) {
+// K_pp pattern and, with fa, the values of the current assembly
+static int pen_fill(Ctx &c, const double *fa) {
   const int64_t np = c.pen_n;
   const int g1 = (int)((np + TPB - 1) / TPB);
   if (c.bs == 3)
     hipLaunchKernelGGL(k_pen_fill<3>, dim3(g1), dim3(TPB), 0, c.stream, np, c.d_pen_idx.as<int64_t>(),
-                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
+                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), fa,
                        c.d_pen_pmap.as<int32_t>(), c.d_pen_ia.as<int64_t>(), c.d_pen_ja.as<int32_t>(),
                        c.d_pen_a.as<double>());
   else
     hipLaunchKernelGGL(k_pen_fill<1>, dim3(g1), dim3(TPB), 0, c.stream, np, c.d_pen_idx.as<int64_t>(),
-                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
+                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), fa,
                        c.d_pen_pmap.as<int32_t>(), c.d_pen_ia.as<int64_t>(), c.d_pen_ja.as<int32_t>(),
                        c.d_pen_a.as<double>());
   PZG_HIP(hipGetLastError());
@@ -530,26 +532,26 @@ static int pen_fill(Ctx &c) {
 
 // The penalty block of the current assembly: structure once per mesh, then
 // K_pp and the Schwarz inverses on the device.  Needs les_prepare (penalty
-// flags) and the full block CSR of the current assembly.
+// flags); of the full block CSR it uses the rows that the penalized columns
+// reach, and expands those when the whole is not there.
 int pen_setup(Ctx &c) {
   c.pen_ready = false;
-  if (!c.les_graph || (int64_t)c.les_pen.size() != c.neq || !c.full_valid) {
-    set_error("penalty rows: learned element graph or full block CSR missing");
+  if (!c.les_graph || (int64_t)c.les_pen.size() != c.neq) {
+    set_error("penalty rows: learned element graph missing");
     return PZG_ESTATE;
   }
   if (c.bs != 1 && c.bs != 3) {
     set_error("penalty rows: nstate must be 1 or 3");
     return PZG_EUNSUP;
   }
-  if (!c.pen_struct) {
-    PZG_TRY(pen_structure(c));
-  } else if (c.pen_n > 0) {
-    PZG_TRY(pen_fill(c));
-  }
+  if (!c.pen_struct) PZG_TRY(pen_structure(c));
   if (c.pen_n == 0) {
     c.pen_ready = true;
     return PZG_OK;
   }
+  // (the penalized rows are among them: every row holds its diagonal block)
+  if (!c.full_valid) PZG_TRY(launch_expand_rows(c, c.d_pen_arow.as<int32_t>(), c.pen_narow));
+  PZG_TRY(pen_fill(c, c.d_fa.as<double>()));
   int *fail = reinterpret_cast<int *>(reinterpret_cast<char *>(c.d_pen_scal.p) + sizeof(PenScal));
   hipLaunchKernelGGL(k_pen_zero_int, dim3(1), dim3(1), 0, c.stream, fail);
   hipLaunchKernelGGL(k_pen_inv, dim3((unsigned)c.pen_nset), dim3(64), 0, c.stream, c.d_pen_sptr.as<int64_t>(),

@@ -276,23 +276,21 @@ __global__ void k_bj_rho64(SolveScalars *sc, const double *partials, int nblk) {
   if (threadIdx.x == 0) sc->rho = rz;
 }
 
-// inverse of each diagonal block of the FP64 full block CSR (cofactors for
-// 3 x 3, the reciprocal for 1 x 1); a singular block sets *fail
+// inverse of each diagonal block of K (the first entries of the block's rows
+// in the upper CSR; cofactors for 3 x 3, the reciprocal for 1 x 1); a singular
+// block sets *fail
 template <int BS>
-__global__ void k_bj_inv64(int64_t nb, const int64_t *__restrict__ fbia, const int32_t *__restrict__ fbja,
-                           const double *__restrict__ fa, double *__restrict__ binv, int *fail) {
+__global__ void k_bj_inv64(int64_t nb, const int64_t *__restrict__ ia, const double *__restrict__ v,
+                           double *__restrict__ binv, int *fail) {
   const int64_t A = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (A >= nb) return;
-  const int64_t b0 = fbia[A], n = fbia[A + 1] - b0;
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t m = (lo + hi) / 2;
-    if (fbja[b0 + m] < A) lo = m + 1;
-    else hi = m;
-  }
   double a[BS * BS];
 #pragma unroll
-  for (int k = 0; k < BS * BS; k++) a[k] = fa[bsr_pos<BS * BS>(b0, n, lo, k)];
+  for (int k = 0; k < BS; k++) {
+    const int64_t q = ia[A * BS + k];
+#pragma unroll
+    for (int l = k; l < BS; l++) a[k * BS + l] = a[l * BS + k] = v[q + (l - k)];
+  }
   static_assert(BS == 1 || BS == 3, "connect blocks of 1 or 3 equations");
   double *o = binv + A * BS * BS;
   if (BS == 1) {
@@ -636,6 +634,9 @@ static void fin_residual64(Ctx &c, const double *partials, int nblk, int nslot, 
 
 int launch_multadd_upper(Ctx &c, const double *x, const double *y, double *z, double alpha,
                          double beta) {
+  bool kf = false;
+  PZG_TRY(kf_prepare(c, &kf));
+  if (kf) return kf_apply(c, KF_AXPBY, x, y, alpha, beta, z, nullptr, nullptr);
   if (!c.full_valid) PZG_TRY(launch_expand_full(c));
   PZG_TRY(launch_spmv64(c, x, z));
   int64_t n = c.neq;
@@ -645,19 +646,38 @@ int launch_multadd_upper(Ctx &c, const double *x, const double *y, double *z, do
   return PZG_OK;
 }
 
+// r = f - K u (r may be null) and out = (|r|^2, |f|^2), by the element
+// products when they are prepared (kf_prepare) and the block CSR otherwise
+static int launch_residual64(Ctx &c, const double *u, double *r, double *partials, double *out) {
+  if (c.kf_valid) {
+    PZG_TRY(kf_apply(c, KF_RESIDUAL, u, c.d_f.as<double>(), 1., 0., r, nullptr, partials));
+    fin_residual64(c, partials, kf_rows_grid(c), 2, out);
+  } else {
+    DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(bsr_grid(c.nb)), dim3(TPB), 0, c.stream, c.nb,
+                                         c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), u,
+                                         c.d_f.as<double>(), r, partials));
+    fin_residual64(c, partials, bsr_grid(c.nb), 2, out);
+  }
+  PZG_HIP(hipGetLastError());
+  return PZG_OK;
+}
+
+// the FP64 operator of the assembled system: element products or block CSR
+static int prepare_k64(Ctx &c) {
+  bool kf = false;
+  PZG_TRY(kf_prepare(c, &kf));
+  if (!kf && !c.full_valid) PZG_TRY(launch_expand_full(c));
+  return PZG_OK;
+}
+
 int true_residual(Ctx &c, const double *u, double *rel) {
   if (!c.f_valid || !c.d_f.p || !u) {  // never launch on a missing load or solution
     set_error("true residual: no load or solution of the current system on the device");
     return PZG_ESTATE;
   }
-  if (!c.full_valid) PZG_TRY(launch_expand_full(c));
+  PZG_TRY(prepare_k64(c));
   PZG_TRY(ensure_reduce(c));
-  DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(bsr_grid(c.nb)), dim3(TPB), 0,
-                                       c.stream, c.nb, c.d_fbia.as<int64_t>(),
-                                       c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), u,
-                                       c.d_f.as<double>(), nullptr, c.d_partials.as<double>()));
-  fin_residual64(c, c.d_partials.as<double>(), bsr_grid(c.nb), 2, c.d_res2.as<double>());
-  PZG_HIP(hipGetLastError());
+  PZG_TRY(launch_residual64(c, u, nullptr, c.d_partials.as<double>(), c.d_res2.as<double>()));
   double h[2];
   PZG_HIP(hipMemcpyAsync(h, c.d_res2.p, sizeof(h), hipMemcpyDeviceToHost, c.stream));
   PZG_HIP(hipStreamSynchronize(c.stream));
@@ -698,11 +718,11 @@ int noalloc_scratch_setup(int device) {
   return PZG_OK;
 }
 
-// The residual of true_residual on the full block CSR already on the device,
-// reducing in the per-device scratch: no allocation of any kind.
+// The residual of true_residual on the FP64 operator already on the device
+// (element products or full block CSR), reducing in the per-device scratch: no allocation of any kind.
 int true_residual_noalloc(Ctx &c, double *rel) {
-  if (!c.full_valid || !c.d_fbia.p || !c.f_valid || !c.d_f.p) {
-    set_error("pzg_true_residual_noalloc: no full block CSR or load of the current system on the "
+  if (!(c.kf_valid || (c.full_valid && c.d_fbia.p)) || !c.f_valid || !c.d_f.p) {
+    set_error("pzg_true_residual_noalloc: no FP64 operator or load of the current system on the "
               "device (call a solve or pzg_true_residual after assembling first)");
     return PZG_ESTATE;
   }
@@ -711,18 +731,13 @@ int true_residual_noalloc(Ctx &c, double *rel) {
     set_error("pzg_true_residual_noalloc: scratch of this device not set up");
     return PZG_ESTATE;
   }
-  const int grid = bsr_grid(c.nb);
+  const int grid = c.kf_valid ? kf_rows_grid(c) : bsr_grid(c.nb);
   if (grid > NOALLOC_PART / 2) {
     set_error("pzg_true_residual_noalloc: residual grid of " + std::to_string(grid) +
               " workgroups exceeds the scratch's " + std::to_string(NOALLOC_PART / 2));
     return PZG_EINVAL;
   }
-  DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(grid), dim3(TPB), 0, c.stream, c.nb,
-                                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
-                                       c.d_fa.as<double>(), c.d_u.as<double>(),
-                                       c.d_f.as<double>(), nullptr, s));
-  fin_residual64(c, s, grid, 2, s + NOALLOC_OUT);
-  PZG_HIP(hipGetLastError());
+  PZG_TRY(launch_residual64(c, c.d_u.as<double>(), nullptr, s, s + NOALLOC_OUT));
   double h[2];
   PZG_HIP(hipMemcpyAsync(h, s + NOALLOC_OUT, sizeof(h), hipMemcpyDeviceToHost, c.stream));
   PZG_HIP(hipStreamSynchronize(c.stream));
@@ -755,6 +770,18 @@ static int run_batches(Ctx &c, int batch, bool use_graph, F enqueue_iter, SolveS
   return PZG_OK;
 }
 
+// q = K p with the partials of p.q in slot 0; the number of partials
+static int pq64_grid(const Ctx &c) { return c.kf_valid ? kf_rows_grid(c) : bsr_grid(c.nb); }
+static void launch_pq64(Ctx &c, SolveScalars *sc, double *part) {
+  if (c.kf_valid) {
+    (void)kf_apply(c, KF_DOT, c.d_p.as<double>(), nullptr, 1., 0., c.d_q.as<double>(), sc, part);
+    return;
+  }
+  DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_spmv64_pq<BS>, dim3(bsr_grid(c.nb)), dim3(TPB), 0, c.stream, c.nb,
+                                       c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
+                                       c.d_p.as<double>(), c.d_q.as<double>(), sc, part));
+}
+
 // FP64 Jacobi-PCG iterations (the EJacobi CG<> of solve_pcg64) continued from
 // the current solution u, whose true residual f - K u is in d_r: the mixed
 // solver's fallback when the FP32 iterations stall.  Runs until the
@@ -766,7 +793,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
   for (DevBuf *b : {&c.d_z, &c.d_p, &c.d_q}) PZG_TRY(dev_alloc(*b, n * sizeof(double)));
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
-  const int gv = grid_for(n, TPB), gs = bsr_grid(c.nb);
+  const int gv = grid_for(n, TPB), gs = pq64_grid(c);
   for (int round = 0; round < 4 && rel > prm.tol && iters < prm.max_iter; round++) {
     SolveScalars hs;
     std::memset(&hs, 0, sizeof(hs));
@@ -782,10 +809,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
     auto iter = [&]() {
       hipLaunchKernelGGL(k_p_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_z.as<double>(),
                          c.d_p.as<double>(), sc);
-      DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_spmv64_pq<BS>, dim3(gs), dim3(TPB), 0, c.stream, c.nb,
-                                           c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
-                                           c.d_fa.as<double>(), c.d_p.as<double>(),
-                                           c.d_q.as<double>(), sc, part));
+      launch_pq64(c, sc, part);
       hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
       hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
                          c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
@@ -798,12 +822,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
     if (!hs.done) PZG_TRY(run_batches(c, prm.check_every > 0 ? prm.check_every : 50, prm.use_graph != 0, iter, hs));
     iters = hs.iter;
     // true residual into d_r (the next round restarts from it)
-    DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_residual64<BS>, dim3(gs), dim3(TPB), 0, c.stream, c.nb,
-                                         c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
-                                         c.d_fa.as<double>(), c.d_u.as<double>(), c.d_f.as<double>(),
-                                         c.d_r.as<double>(), part));
-    fin_residual64(c, part, gs, 2, c.d_res2.as<double>());
-    PZG_HIP(hipGetLastError());
+    PZG_TRY(launch_residual64(c, c.d_u.as<double>(), c.d_r.as<double>(), part, c.d_res2.as<double>()));
     double h[2];
     PZG_HIP(hipMemcpyAsync(h, c.d_res2.p, sizeof(h), hipMemcpyDeviceToHost, c.stream));
     PZG_HIP(hipStreamSynchronize(c.stream));
@@ -815,7 +834,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
 
 int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
   const int64_t n = c.neq;
-  if (!c.full_valid) PZG_TRY(launch_expand_full(c));
+  PZG_TRY(prepare_k64(c));
   PZG_TRY(ensure_reduce(c));
   for (DevBuf *b : {&c.d_u, &c.d_r, &c.d_z, &c.d_p, &c.d_q}) PZG_TRY(dev_alloc(*b, n * sizeof(double)));
   SolveScalars hs;
@@ -869,8 +888,8 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
     int *fail = reinterpret_cast<int *>(c.d_counter.as<unsigned>() + 8);
     PZG_HIP(hipMemsetAsync(fail, 0, sizeof(int), c.stream));
     DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_bj_inv64<BS>, dim3((unsigned)((c.nb + TPB - 1) / TPB)), dim3(TPB), 0,
-                                         c.stream, c.nb, c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
-                                         c.d_fa.as<double>(), c.d_bjinv64.as<double>(), fail));
+                                         c.stream, c.nb, c.d_ia.as<int64_t>(), c.d_a.as<double>(),
+                                         c.d_bjinv64.as<double>(), fail));
     int hf = 0;
     PZG_HIP(hipMemcpyAsync(&hf, fail, sizeof(int), hipMemcpyDeviceToHost, c.stream));
     PZG_HIP(hipStreamSynchronize(c.stream));
@@ -900,14 +919,11 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
     hipLaunchKernelGGL(k_bj_rho64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
   }
   PZG_HIP(hipGetLastError());
-  const int gs = bsr_grid(c.nb);
+  const int gs = pq64_grid(c);
   auto iter = [&]() {
     hipLaunchKernelGGL(k_p_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_z.as<double>(),
                        c.d_p.as<double>(), sc);
-    DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_spmv64_pq<BS>, dim3(gs), dim3(TPB), 0, c.stream, c.nb,
-                                         c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(),
-                                         c.d_fa.as<double>(), c.d_p.as<double>(),
-                                         c.d_q.as<double>(), sc, part));
+    launch_pq64(c, sc, part);
     hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
     hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
                        c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
@@ -1175,7 +1191,7 @@ constexpr int64_t MG_INNER_CAP = 2000;  // FP32 iterations per refinement step, 
 template <int BS>
 static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
   const int64_t n = c.neq, nb = c.nb;
-  if (!c.full_valid) PZG_TRY(launch_expand_full(c));
+  PZG_TRY(prepare_k64(c));
   // operator of the FP32 iterations
   bool use_mf = false;
   if (prm.inner_op == PZG_INNER_MATFREE) {
@@ -1218,10 +1234,8 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
       hipLaunchKernelGGL(k_residual_zero, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_f.as<double>(),
                          c.d_r.as<double>(), part);
     else
-      hipLaunchKernelGGL(k_residual64<BS>, dim3(bsr_grid(nb)), dim3(TPB), 0, c.stream, nb,
-                         c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
-                         c.d_u.as<double>(), c.d_f.as<double>(), c.d_r.as<double>(), part);
-    fin_residual64(c, part, u_zero ? gv : bsr_grid(nb), u_zero ? 1 : 2, out);
+      PZG_TRY(launch_residual64(c, c.d_u.as<double>(), c.d_r.as<double>(), part, out));
+    if (u_zero) fin_residual64(c, part, gv, 1, out);
     double h[2];
     PZG_HIP(hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, c.stream));
     PZG_HIP(hipStreamSynchronize(c.stream));
