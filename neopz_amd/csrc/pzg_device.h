@@ -43,9 +43,38 @@ __device__ inline void xcd_slab(int64_t n, int64_t &lo, int64_t &hi, int &i, int
 constexpr int MAXBLK = 2048;  // partial-sum slots per reduction
 constexpr int NSLOT = 4;
 
-__device__ inline double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Cross-lane moves inside a row of 16 lanes by DPP (no LDS round trip: a
+// __shfl of a double is two ds_bpermute of some 60 cycles each).
+template <int CTRL> __device__ inline float dpp_move(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ inline double dpp_move(double v) {
+  const int64_t b = __builtin_bit_cast(int64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffff), CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (int64_t)((uint64_t)hi << 32 | lo));
+}
+// sum over the row of 16 lanes in each of its lanes (row_ror 8, 4, 2, 1: the
+// additions of an xor butterfly)
+template <class T> __device__ inline T row16_sum(T v) {
+  v += dpp_move<0x128>(v);
+  v += dpp_move<0x124>(v);
+  v += dpp_move<0x122>(v);
+  v += dpp_move<0x121>(v);
   return v;
+}
+__device__ inline double lane_value(double v, int lane) {
+  const int64_t b = __builtin_bit_cast(int64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(b & 0xffffffff), lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __builtin_bit_cast(double, (int64_t)((uint64_t)hi << 32 | lo));
+}
+
+// sum over the wavefront (every lane active) in every lane
+__device__ inline double wave_sum(double v) {
+  v = row16_sum(v);
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 // Sum of v over the block; result valid in thread 0.

@@ -78,6 +78,9 @@ static void free_all(Ctx &c) {
                     &c.cv.d_ef, &c.cb.d_cel, &c.cb.d_cslot, &c.cb.d_T, &c.cb.d_blk, &c.cb.d_n,
                     &c.cb.d_ek, &c.cb.d_ef};
   for (DevBuf *b : bufs) dev_free(*b);
+  if (c.solve_graph) (void)hipGraphExecDestroy(c.solve_graph);
+  c.solve_graph = nullptr;
+  c.solve_key.clear();
   mg_free(c);
 }
 

@@ -152,16 +152,22 @@ __host__ __device__ inline int64_t bsr_pos(int64_t b0, int64_t n, int64_t i, int
   return (b0 + j) * BB + (int64_t)k * m + (i - j);
 }
 
-// Device-side scalar state of an iterative solve.
+// Device-side scalar state of an iterative solve.  Two copies: a kernel reads
+// one and its first workgroup writes the other (sc[0]: written by the update,
+// read by the direction; sc[1]: the reverse), so every workgroup can form the
+// scalars of a step from the partial sums itself.
 struct SolveScalars {
-  double rho, rho_old, pq, alpha, beta, rr, normb, resid, tol, pr, zq;
+  double rho, pq, alpha, beta, rr, normb, resid, tol, pr, zq;
   double rlast;   // mixed: scaled residual norm at the last reliable update
   double delta;   // mixed: reduction of the recursive residual that triggers an update
   int64_t iter, maxit;
   // done: 0 running, 1 tol, 2 maxit, 3 divergence, 4 update due (set by the
   // iteration's last reduction; its completion kernels still run), 5 update
   // due (completion kernels already ran)
-  int32_t done, pad;
+  // pend (state of the search direction): 0 p is ready; bit 0 the stop test,
+  // bit 1 beta still to be formed from the update's partials; bit 2 beta is
+  // known, p not yet updated
+  int32_t done, pend;
 };
 
 // A lattice level of the multigrid preconditioner (pzg_mg.hip): n[0] x n[1] x
@@ -310,6 +316,10 @@ struct Ctx {
   DevBuf d_scal, d_partials, d_counter;
   DevBuf d_res2;  // |r|^2, |f|^2 of the FP64 true residual
   int reduce_blocks = 1024;
+  // captured batch of the last CG/FCG iteration, reused while every pointer,
+  // size and launch shape in it (solve_key) is the same
+  hipGraphExec_t solve_graph = nullptr;
+  std::vector<uint64_t> solve_key;
   bool has_solution = false;
   bool f_valid = false;  // d_f holds the load of the current system (set by a solve)
 

@@ -63,12 +63,13 @@ static int grid_for(int64_t n, int per_block) {
 #endif
 constexpr int BSR_L = PZG_BSR_L;
 constexpr int BSR_U = PZG_BSR_U;
-static_assert(BSR_L == BSR_CHUNK, "lanes per block row must match the value chunks");
+static_assert(BSR_L == BSR_CHUNK && BSR_L == 16, "a block row is a row of 16 lanes, as the value chunks are");
 
-template <class T, int BS>
-__device__ inline void bsr_row(int64_t A, const int64_t *__restrict__ bia,
-                               const int32_t *__restrict__ bja, const T *__restrict__ v,
-                               const T *__restrict__ x, int sub, T (&out)[BS]) {
+// xf(i): entry i of the vector.
+template <class T, int BS, class X>
+__device__ inline void bsr_row_f(int64_t A, const int64_t *__restrict__ bia,
+                                 const int32_t *__restrict__ bja, const T *__restrict__ v,
+                                 X xf, int sub, T (&out)[BS]) {
   constexpr int BB = BS * BS;
   T acc[BS];
   for (int k = 0; k < BS; k++) acc[k] = T(0);
@@ -95,7 +96,7 @@ __device__ inline void bsr_row(int64_t A, const int64_t *__restrict__ bia,
 #pragma unroll
     for (int u = 0; u < BSR_U; u++)
 #pragma unroll
-      for (int l = 0; l < BS; l++) xv[u][l] = x[col[u] * BS + l];
+      for (int l = 0; l < BS; l++) xv[u][l] = xf(col[u] * BS + l);
 #pragma unroll
     for (int u = 0; u < BSR_U; u++)
 #pragma unroll
@@ -105,10 +106,15 @@ __device__ inline void bsr_row(int64_t A, const int64_t *__restrict__ bia,
   }
 #pragma unroll
   for (int k = 0; k < BS; k++) {
-    T s = acc[k];
-    for (int o = BSR_L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, BSR_L);
-    out[k] = s;
+    out[k] = row16_sum(acc[k]);
   }
+}
+
+template <class T, int BS>
+__device__ inline void bsr_row(int64_t A, const int64_t *__restrict__ bia,
+                               const int32_t *__restrict__ bja, const T *__restrict__ v,
+                               const T *__restrict__ x, int sub, T (&out)[BS]) {
+  bsr_row_f<T, BS>(A, bia, bja, v, [x](int64_t i) { return x[i]; }, sub, out);
 }
 
 // lane 'sub' (< BS) of a row group picks component sub of out
@@ -147,13 +153,210 @@ __global__ __launch_bounds__(TPB) void k_spmv_bsr(int64_t nb, const int64_t *__r
   }
 }
 
+// Sums of NV partial slots, the same bits in every workgroup and thread: each
+// workgroup of a step forms the scalars it needs itself, which replaces the
+// one-block kernel between two steps (3 to 5 us each on the device, as much as
+// a step of a small system).  The step kernels run at most CG_MAXBLK
+// workgroups, so the slots stay short.
+constexpr int CG_MAXBLK = 512;
+template <int NV>
+__device__ inline void sum_slots(const double *partials, const int (&slot)[NV], const int (&cnt)[NV],
+                                 double (&tot)[NV]) {
+  __shared__ double sm[NV][16];
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    double s = 0.;
+    for (int b = threadIdx.x; b < cnt[k]; b += blockDim.x) s += partials[slot[k] * MAXBLK + b];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) sm[k][w] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    tot[k] = 0.;
+    for (int j = 0; j < nw; j++) tot[k] += sm[k][j];
+  }
+}
+
+// this workgroup's sums of v into slots 0 .. NV-1 (any workgroup size up to
+// 1024)
+template <int NV>
+__device__ inline void store_slots(const double (&v)[NV], double *partials) {
+  __shared__ double sm[NV][16];
+  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    const double s = wave_sum(v[k]);
+    if ((threadIdx.x & 63) == 0) sm[k][w] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV) {
+    double s = 0.;
+    for (int j = 0; j < nw; j++) s += sm[threadIdx.x][j];
+    partials[threadIdx.x * MAXBLK + blockIdx.x] = s;
+  }
+}
+
+// Workgroup size and grid of the step kernels over n items: 256 threads on
+// small systems (latency), 1024 beyond 2 workgroups of 256 per CU so that
+// CG_MAXBLK workgroups still fill every wavefront slot.
+struct CgGrid {
+  int tpb, blocks;
+};
+static CgGrid cg_grid(int64_t n) {
+  CgGrid g;
+  g.tpb = n > (int64_t)CG_MAXBLK * 256 ? 1024 : 256;
+  g.blocks = (int)std::max<int64_t>(1, std::min<int64_t>((n + g.tpb - 1) / g.tpb, CG_MAXBLK));
+  return g;
+}
+
+// Scalars of the next direction from state A and the update's partials (slots
+// 0 and 1): stop test, beta; the new state in B (first workgroup).  Returns
+// false when the iteration has stopped and p must not change; *upd: p is to be
+// updated with *beta.  FCG: beta = -(z.q)/(p.q) and the tests of the mixed
+// solver's FP32 iteration; else beta = (r.z)/rho and the reference's tests.
+// (Fields are read and written one by one: a struct copy per thread is kept
+// in memory by the compiler and cost 14 us a launch at 350k equations.)
+template <bool FCG>
+__device__ inline bool next_direction(const SolveScalars *A, SolveScalars *B, const double *partials, int n0,
+                                      int n1, double *beta, bool *upd) {
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  int done = A->done;
+  const int pend = A->pend;
+  double bt = A->beta, rho = A->rho, resid = A->resid;
+  int64_t iter = A->iter;
+  if (!done && (pend & 3)) {
+    const int slot[2] = {0, 1}, cnt[2] = {pend & 1 ? n0 : 0, pend & 2 ? n1 : 0};
+    double t[2];
+    sum_slots<2>(partials, slot, cnt, t);
+    if (pend & 1) {
+      iter++;
+      resid = sqrt(t[0]) / A->normb;
+      if (FCG) {
+        // divergence guard: leave the loop, the host restarts from the true residual
+        if (!(resid == resid) || resid > 1e3) done = 3;
+        else if (sqrt(t[0]) < A->delta * A->rlast) done = 4;
+        else if (iter >= A->maxit) done = 2;
+      } else {
+        if (resid <= A->tol) done = 1;
+        else if (iter >= A->maxit) done = 2;
+      }
+    }
+    if (pend & 2) {
+      if (FCG) {
+        bt = -t[1] / A->pq;
+      } else {
+        bt = t[1] / rho;
+        rho = t[1];
+      }
+    }
+  } else if (done) {
+    if (first) {
+      B->done = done;
+      B->pend = pend;
+      B->iter = iter;
+      B->resid = resid;
+      B->rho = rho;
+      B->beta = bt;
+      B->pq = A->pq;
+    }
+    return false;
+  }
+  if (first) {
+    B->done = done;
+    B->pend = 0;
+    B->iter = iter;
+    B->resid = resid;
+    B->rho = rho;
+    B->beta = bt;
+    B->pq = A->pq;
+  }
+  *beta = bt;
+  *upd = pend != 0;
+  // an update request (4) of the FCG still completes its direction
+  return !done || (FCG && done == 4);
+}
+
+// the update's side of the exchange: state A after a step that ran (pend = 3)
+// or after one that found the iteration stopped
+__device__ inline void close_step(SolveScalars *A, const SolveScalars *B, double pq, int pend) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    A->iter = B->iter;
+    A->resid = B->resid;
+    A->rho = B->rho;
+    A->beta = B->beta;
+    A->pq = pq;
+    A->pend = pend;
+    A->done = B->done;
+  }
+}
+
+// end of a batch: the pending test and beta into A (one block), for the host
+// and the next batch's first direction
+template <bool FCG>
+__global__ __launch_bounds__(TPB) void k_cg_close(SolveScalars *A, SolveScalars *B, const double *partials, int n0,
+                                                  int n1) {
+  double beta;
+  bool upd;
+  if (A->done || A->pend == 0) return;
+  (void)next_direction<FCG>(A, B, partials, n0, n1, &beta, &upd);
+  __syncthreads();
+  close_step(A, B, B->pq, 4);
+}
+
+// PCG64 with the direction formed inside the product: p = z + beta p_old,
+// q = K p, partials of p.q (slot 2).  Every gather reads z and p_old and forms
+// its entry; the row's own entries go to p_new.
+template <int BS>
+__global__ __launch_bounds__(TPB) void k_pcg_step64(int64_t nb, const int64_t *__restrict__ bia,
+                                                    const int32_t *__restrict__ bja,
+                                                    const double *__restrict__ v,
+                                                    const double *__restrict__ z,
+                                                    const double *__restrict__ p_old,
+                                                    double *__restrict__ p_new, double *__restrict__ q,
+                                                    const SolveScalars *A, SolveScalars *B, double *partials,
+                                                    int n0, int n1) {
+  double beta;
+  bool upd;
+  if (!next_direction<false>(A, B, partials, n0, n1, &beta, &upd)) return;
+  const int sub = threadIdx.x % BSR_L;
+  constexpr int RPB = TPB / BSR_L;
+  double acc = 0.;
+  auto dir = [=](int64_t i) { return upd ? beta * p_old[i] + z[i] : p_old[i]; };
+  for (int64_t R = (int64_t)blockIdx.x * RPB + threadIdx.x / BSR_L; R < nb; R += (int64_t)gridDim.x * RPB) {
+    double out[BS];
+    bsr_row_f<double, BS>(R, bia, bja, v, dir, sub, out);
+    if (sub < BS) {
+      const int64_t i = R * BS + sub;
+      const double qi = pick<double, BS>(out, sub), pi = dir(i);
+      q[i] = qi;
+      p_new[i] = pi;
+      acc += qi * pi;
+    }
+  }
+  double vv[1] = {acc};
+  store_slots<1>(vv, partials + 2 * MAXBLK);
+}
+
+// PCG64 direction alone: p = z + beta p
+__global__ __launch_bounds__(1024) void k_pcg_dir64(int64_t n, const double *__restrict__ z,
+                                                    double *__restrict__ p, const SolveScalars *A,
+                                                    SolveScalars *B, const double *partials, int n0, int n1) {
+  double beta;
+  bool upd;
+  if (!next_direction<false>(A, B, partials, n0, n1, &beta, &upd) || !upd) return;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = beta * p[i] + z[i];
+}
+
 // PCG64: q = K p and per-block partial sums of p.q (slot 0)
 template <int BS>
 __global__ __launch_bounds__(TPB) void k_spmv64_pq(int64_t nb, const int64_t *__restrict__ bia,
                                                    const int32_t *__restrict__ bja,
                                                    const double *__restrict__ v,
                                                    const double *__restrict__ p,
-                                                   double *__restrict__ q, SolveScalars *sc,
+                                                   double *__restrict__ q, const SolveScalars *sc,
                                                    double *partials) {
   if (sc->done) return;
   const int sub = threadIdx.x % BSR_L;
@@ -189,67 +392,76 @@ static int bsr_grid(int64_t nb) {
   return (int)std::max<int64_t>(g, 1);
 }
 
-// alpha = rho / (p.q)   (one block)
-__global__ void k_fin_alpha64(SolveScalars *sc, const double *partials, int nblk) {
-  if (sc->done) return;
-  double pq = sum_partials(partials, 0, nblk);
-  if (threadIdx.x == 0) {
-    sc->pq = pq;
-    sc->alpha = sc->rho / pq;
+// x += alpha p; r -= alpha q; partials of r.r (slot 0); preconditioner PRE: 0
+// point Jacobi z = r / diag, 1 the connect blocks z = Binv r (BS equations
+// each; TPZBlockDiagonal with ELU blocks, the preconditioner
+// TPZAnalysis::BuildPreconditioner(EBlockJacobi, true) returns,
+// Analysis/TPZAnalysis.cpp:1062-1070), both with r.z in slot 1; 2 left to
+// k_vbj_apply64.  alpha = rho / (p.q) from the product's partials (slot 2).
+template <int BS, int PRE>
+__global__ __launch_bounds__(1024) void k_cg_update64(int64_t nb, double *__restrict__ x,
+                                                      double *__restrict__ r,
+                                                      double *__restrict__ z,
+                                                      const double *__restrict__ p,
+                                                      const double *__restrict__ q,
+                                                      const double *__restrict__ pre,
+                                                      SolveScalars *A, const SolveScalars *B,
+                                                      double *partials, int npq) {
+  if (B->done) {
+    close_step(A, B, B->pq, 0);
+    return;
   }
-}
-
-// p = z + beta p  (p = z on the first iteration)
-__global__ void k_p_update64(int64_t n, const double *__restrict__ z, double *__restrict__ p,
-                             const SolveScalars *sc) {
-  if (sc->done) return;
-  const double beta = sc->iter == 0 ? 0. : sc->beta;
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t st = (int64_t)gridDim.x * blockDim.x;
-  if (sc->iter == 0)
-    for (; i < n; i += st) p[i] = z[i];
-  else
-    for (; i < n; i += st) p[i] = beta * p[i] + z[i];
-}
-
-// x += alpha p; r -= alpha q; resid = |r|/|b|; z = r/diag; beta = (r.z)/rho
-__global__ __launch_bounds__(TPB) void k_cg_update64(int64_t n, double *__restrict__ x,
-                                                     double *__restrict__ r,
-                                                     double *__restrict__ z,
-                                                     const double *__restrict__ p,
-                                                     const double *__restrict__ q,
-                                                     const double *__restrict__ diag,
-                                                     SolveScalars *sc, double *hist,
-                                                     double *partials) {
-  if (sc->done) return;
-  const double alpha = sc->alpha;
+  const int slot[1] = {2}, cnt[1] = {npq};
+  double pq[1];
+  sum_slots<1>(partials, slot, cnt, pq);
+  const double alpha = B->rho / pq[0];
   double rr = 0., rz = 0.;
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t st = (int64_t)gridDim.x * blockDim.x;
-  for (; i < n; i += st) {
-    x[i] += alpha * p[i];
-    double ri = r[i] + (-alpha) * q[i];
-    r[i] = ri;
-    rr += ri * ri;
-    if (diag) {  // point Jacobi; the block form follows in k_bj_apply64
-      double zi = ri / diag[i];
-      z[i] = zi;
-      rz += ri * zi;
+  for (int64_t R = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; R < nb; R += (int64_t)gridDim.x * blockDim.x) {
+    double rv[BS];
+#pragma unroll
+    for (int k = 0; k < BS; k++) {
+      const int64_t i = R * BS + k;
+      x[i] += alpha * p[i];
+      rv[k] = r[i] + (-alpha) * q[i];
+      r[i] = rv[k];
+      rr += rv[k] * rv[k];
+    }
+    if (PRE == 0) {
+#pragma unroll
+      for (int k = 0; k < BS; k++) {
+        const int64_t i = R * BS + k;
+        const double zi = rv[k] / pre[i];
+        z[i] = zi;
+        rz += rv[k] * zi;
+      }
+    } else if (PRE == 1) {
+      const double *bi = pre + R * BS * BS;
+#pragma unroll
+      for (int k = 0; k < BS; k++) {
+        double t = 0.;
+#pragma unroll
+        for (int l = 0; l < BS; l++) t += bi[k * BS + l] * rv[l];
+        z[R * BS + k] = t;
+        rz += rv[k] * t;
+      }
     }
   }
-  double v[2] = {rr, rz};
-  block_partials<2>(v, partials);
+  if (PRE == 2) {
+    double v[1] = {rr};
+    store_slots<1>(v, partials);
+  } else {
+    double v[2] = {rr, rz};
+    store_slots<2>(v, partials);
+  }
+  close_step(A, B, pq[0], 3);
 }
 
-// Connect-block Jacobi (TPZBlockDiagonal with ELU blocks, the preconditioner
-// TPZAnalysis::BuildPreconditioner(EBlockJacobi, true) returns,
-// Analysis/TPZAnalysis.cpp:1062-1070): z = Binv r per block row, r.z into
-// partials slot 1 (same grid as k_cg_update64).
+// Connect-block Jacobi of the first residual: p = z = Binv r per block row,
+// r.z into partials slot 1.
 template <int BS>
 __global__ __launch_bounds__(TPB) void k_bj_apply64(int64_t nb, const double *__restrict__ binv,
                                                     const double *__restrict__ r, double *__restrict__ z,
-                                                    const SolveScalars *sc, double *partials) {
-  if (sc && sc->done) return;
+                                                    double *__restrict__ p, double *partials) {
   double rz = 0.;
   for (int64_t A = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; A < nb; A += (int64_t)gridDim.x * blockDim.x) {
     double rv[BS];
@@ -262,6 +474,7 @@ __global__ __launch_bounds__(TPB) void k_bj_apply64(int64_t nb, const double *__
 #pragma unroll
       for (int l = 0; l < BS; l++) s += bi[k * BS + l] * rv[l];
       z[A * BS + k] = s;
+      p[A * BS + k] = s;
       rz += rv[k] * s;
     }
   }
@@ -293,7 +506,7 @@ __global__ void k_bj_inv64(int64_t nb, const int64_t *__restrict__ ia, const dou
   }
   static_assert(BS == 1 || BS == 3, "connect blocks of 1 or 3 equations");
   double *o = binv + A * BS * BS;
-  if (BS == 1) {
+  if constexpr (BS == 1) {
     if (a[0] == 0.) atomicExch(fail, 1);
     o[0] = 1. / a[0];
   } else {
@@ -372,24 +585,26 @@ __global__ __launch_bounds__(256) void k_vbj_inv64(int64_t nblk, const int64_t *
 }
 
 // z = Binv r on the blocks (one thread per equation), r.z into partials
-// slot 1 (same grid as k_cg_update64)
+// slot 1; p = z too when p is given (the first residual)
 __global__ __launch_bounds__(TPB) void k_vbj_apply64(int64_t n, const int32_t *__restrict__ eqb,
                                                      const int64_t *__restrict__ bpos,
                                                      const int32_t *__restrict__ bm,
                                                      const int64_t *__restrict__ boff,
                                                      const double *__restrict__ binv,
                                                      const double *__restrict__ r, double *__restrict__ z,
-                                                     const SolveScalars *sc, double *partials) {
+                                                     double *__restrict__ p, const SolveScalars *sc,
+                                                     double *partials) {
   if (sc && sc->done) return;
   double rz = 0.;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int32_t b = eqb[i];
-    const int64_t p = bpos[b];
+    const int64_t b0 = bpos[b];
     const int m = bm[b];
-    const double *row = binv + boff[b] + (i - p) * m;
+    const double *row = binv + boff[b] + (i - b0) * m;
     double s = 0.;
-    for (int c = 0; c < m; c++) s += row[c] * r[p + c];
+    for (int c = 0; c < m; c++) s += row[c] * r[b0 + c];
     z[i] = s;
+    if (p) p[i] = s;
     rz += r[i] * s;
   }
   __shared__ double sm[TPB / 64];
@@ -440,26 +655,7 @@ __global__ __launch_bounds__(TPB) void k_vbj_apply32(int64_t n, const int32_t *_
   if (threadIdx.x == 0) partials[1 * MAXBLK + blockIdx.x] = t;
 }
 
-// resid = |r|/|b|; stop tests; beta = (r.z)/rho   (one block)
-__global__ void k_fin_cg64(SolveScalars *sc, const double *partials, int nblk, double *hist) {
-  if (sc->done) return;
-  double rr = sum_partials(partials, 0, nblk);
-  double rz = sum_partials(partials, 1, nblk);
-  if (threadIdx.x == 0) {
-    int64_t it = sc->iter + 1;
-    sc->iter = it;
-    double resid = sqrt(rr) / sc->normb;
-    sc->resid = resid;
-    if (hist) hist[it - 1] = resid;
-    if (resid <= sc->tol) sc->done = 1;
-    else if (it >= sc->maxit) sc->done = 2;
-    sc->beta = rz / sc->rho;
-    sc->rho_old = sc->rho;
-    sc->rho = rz;
-  }
-}
-
-// x = 0; r = b; z = r/diag; rho = r.z; normb = |b|
+// x = 0; r = b; p = z = r/diag (with diag); rho = r.z; normb = |b|
 __global__ __launch_bounds__(TPB) void k_cg_init64(int64_t n, const double *__restrict__ b,
                                                    double *__restrict__ x, double *__restrict__ r,
                                                    double *__restrict__ z, double *__restrict__ p,
@@ -472,11 +668,11 @@ __global__ __launch_bounds__(TPB) void k_cg_init64(int64_t n, const double *__re
     double bi = b[i];
     x[i] = 0.;
     r[i] = bi;
-    p[i] = 0.;
     bb += bi * bi;
     if (diag) {
       double zi = bi / diag[i];
       z[i] = zi;
+      p[i] = zi;
       rz += bi * zi;
     }
   }
@@ -499,8 +695,8 @@ __global__ void k_fin_cg_init64(SolveScalars *sc, const double *partials, int nb
 }
 
 // Continuation from the current x with its residual r = f - K x already in
-// r (CG<> with fromCurrent, Solvers/LinearSolvers/cg.h:29-132): z = r/diag,
-// p = 0, rho = r.z, normb = |f|, resid = |r|/|f|.
+// r (CG<> with fromCurrent, Solvers/LinearSolvers/cg.h:29-132): p = z = r/diag,
+// rho = r.z, normb = |f|, resid = |r|/|f|.
 __global__ __launch_bounds__(TPB) void k_cg_restart64(int64_t n, const double *__restrict__ f,
                                                       const double *__restrict__ r,
                                                       double *__restrict__ z, double *__restrict__ p,
@@ -511,7 +707,7 @@ __global__ __launch_bounds__(TPB) void k_cg_restart64(int64_t n, const double *_
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
   for (; i < n; i += st) {
     const double fi = f[i], ri = r[i], zi = ri / diag[i];
-    p[i] = 0.;
+    p[i] = zi;
     z[i] = zi;
     ff += fi * fi;
     rr += ri * ri;
@@ -593,6 +789,148 @@ __global__ __launch_bounds__(TPB) void k_residual_zero(int64_t n, const double *
   }
   double vv[1] = {ff};
   block_partials<1>(vv, partials);
+}
+
+// ---- small systems: CG in one workgroup ------------------------------------
+// The whole iteration of a system whose block CSR and vectors fit in one CU's
+// LDS runs in one workgroup: matrix, p, q, r, x and the preconditioner in LDS,
+// three barriers an iteration, no launch in between.  Bound by LDS latency:
+// 3.2 us an iteration at 289 equations (Poisson 8^2 p = 2, solve 0.27 ms
+// against 3.3 ms of launches).  A launch runs at most CG_SMALL_IT iterations and
+// leaves its state (x, r, p, scalars) in memory, where the next one resumes.
+constexpr int CG_SMALL_TPB = 1024;
+constexpr int CG_SMALL_IT = 2000;
+constexpr int64_t CG_SMALL_LDS = 158 * 1024;  // of the CU's 160 KB; the rest is the reductions'
+
+template <int BS>
+static int64_t cg_small_lds(int64_t nb, int64_t nbf, bool block) {
+  const int64_t n = nb * BS;
+  return 8 * (nbf * BS * BS + n * (4 + (block ? BS : 1))) + 4 * (nbf + nb + 1);
+}
+
+// L lanes (a power of two <= 16) per scalar row in the product; vector steps
+// one thread per block row.
+template <int BS, bool BLOCK>
+__global__ __launch_bounds__(CG_SMALL_TPB) void k_cg_small(int nb, int nbf, int L,
+                                                           const int64_t *__restrict__ bia,
+                                                           const int32_t *__restrict__ bja,
+                                                           const double *__restrict__ v,
+                                                           const double *__restrict__ pre,
+                                                           double *__restrict__ xg, double *__restrict__ rg,
+                                                           double *__restrict__ pg, SolveScalars *sc) {
+  constexpr int BB = BS * BS;
+  extern __shared__ double lds[];
+  __shared__ double sm[3][CG_SMALL_TPB / 64];
+  if (sc->done) return;
+  const int n = nb * BS, tid = threadIdx.x, w = tid >> 6;
+  double *sv = lds, *p = sv + (int64_t)nbf * BB, *q = p + n, *r = q + n, *x = r + n, *m = x + n;
+  int32_t *cj = reinterpret_cast<int32_t *>(m + (int64_t)n * (BLOCK ? BS : 1)), *ci = cj + nbf;
+  for (int i = tid; i < nbf * BB; i += CG_SMALL_TPB) sv[i] = v[i];
+  for (int i = tid; i < nbf; i += CG_SMALL_TPB) cj[i] = bja[i];
+  for (int i = tid; i <= nb; i += CG_SMALL_TPB) ci[i] = (int32_t)bia[i];
+  for (int i = tid; i < n; i += CG_SMALL_TPB) {
+    p[i] = pg[i];
+    r[i] = rg[i];
+    x[i] = xg[i];
+  }
+  for (int i = tid; i < n * (BLOCK ? BS : 1); i += CG_SMALL_TPB) m[i] = pre[i];
+  // total of one value per thread in every thread (slot k of sm; a slot is
+  // written again only after another barrier)
+  auto total = [&](double s, int k) {
+    s = wave_sum(s);
+    if ((tid & 63) == 0) sm[k][w] = s;
+  };
+  auto read = [&](int k) {
+    double t = 0.;
+    for (int j = 0; j < CG_SMALL_TPB / 64; j++) t += sm[k][j];
+    return t;
+  };
+  const double normb = sc->normb, tol = sc->tol;
+  double rho = sc->rho, beta = sc->beta, resid = sc->resid;
+  int64_t it = sc->iter;
+  const int64_t maxit = sc->maxit;
+  int done = 0;
+  const int sub = tid & (L - 1), grp = tid / L, ngrp = CG_SMALL_TPB / L;
+  __syncthreads();
+  for (int k = 0; k < CG_SMALL_IT && !done; k++) {
+    double pq = 0.;
+    for (int i0 = 0; i0 < n; i0 += ngrp) {  // every lane of a wavefront runs the same passes
+      const int i = i0 + grp, A = i / BS, c = i - A * BS;
+      double s = 0.;
+      if (i < n) {
+        const int b0 = ci[A], nn = ci[A + 1] - b0;
+        for (int j = sub; j < nn; j += L) {
+          const int j0 = BS == 1 ? j : j / BSR_CHUNK * BSR_CHUNK;
+          const int mc = BS == 1 ? 1 : (nn - j0 < BSR_CHUNK ? nn - j0 : BSR_CHUNK);
+          const double *vp = sv + (b0 + j0) * BB + (j - j0);
+          const double *pp = p + cj[b0 + j] * BS;
+#pragma unroll
+          for (int l = 0; l < BS; l++) s += vp[(c * BS + l) * mc] * pp[l];
+        }
+      }
+      for (int o = L >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (i < n && sub == 0) {
+        q[i] = s;
+        pq += s * p[i];
+      }
+    }
+    total(pq, 0);
+    __syncthreads();
+    const double alpha = rho / read(0);
+    double rr = 0., rz = 0.;
+    for (int A = tid; A < nb; A += CG_SMALL_TPB) {
+      double rv[BS];
+#pragma unroll
+      for (int a = 0; a < BS; a++) {
+        const int i = A * BS + a;
+        x[i] += alpha * p[i];
+        rv[a] = r[i] + (-alpha) * q[i];
+        r[i] = rv[a];
+        rr += rv[a] * rv[a];
+      }
+#pragma unroll
+      for (int a = 0; a < BS; a++) {
+        const int i = A * BS + a;
+        double z = 0.;
+        if (BLOCK) {
+#pragma unroll
+          for (int l = 0; l < BS; l++) z += m[(A * BS + a) * BS + l] * rv[l];
+        } else {
+          z = rv[a] / m[i];
+        }
+        q[i] = z;
+        rz += rv[a] * z;
+      }
+    }
+    total(rr, 1);
+    total(rz, 2);
+    __syncthreads();
+    it++;
+    resid = sqrt(read(1)) / normb;
+    if (resid <= tol) done = 1;
+    else if (it >= maxit) done = 2;
+    const double t = read(2);
+    beta = t / rho;
+    rho = t;
+    if (!done)
+      for (int A = tid; A < nb; A += CG_SMALL_TPB)
+#pragma unroll
+        for (int a = 0; a < BS; a++) p[A * BS + a] = beta * p[A * BS + a] + q[A * BS + a];
+    __syncthreads();
+  }
+  for (int i = tid; i < n; i += CG_SMALL_TPB) {
+    pg[i] = p[i];
+    rg[i] = r[i];
+    xg[i] = x[i];
+  }
+  if (tid == 0) {
+    sc->iter = it;
+    sc->resid = resid;
+    sc->beta = beta;
+    sc->rho = rho;
+    sc->pend = 0;
+    sc->done = done;
+  }
 }
 
 __global__ void k_axpby64(int64_t n, double alpha, const double *__restrict__ x, double beta,
@@ -745,41 +1083,156 @@ int true_residual_noalloc(Ctx &c, double *rel) {
   return PZG_OK;
 }
 
-// Runs 'batch' iterations of the given enqueue function, optionally through a
-// captured hipGraph, until the device 'done' flag is set.
+// Runs batches of the given enqueue function, optionally through a captured
+// hipGraph, until the device 'done' flag is set.  key: everything the captured
+// launches hold (pointers, sizes, launch shapes); the context keeps the last
+// graph and reuses it while the key is the same (capture and instantiation of
+// 100 iterations cost 0.5 to 1.5 ms a solve).  An empty key: used here only.
 template <class F>
-static int run_batches(Ctx &c, int batch, bool use_graph, F enqueue_iter, SolveScalars &hs) {
+static int run_batches(Ctx &c, bool use_graph, std::vector<uint64_t> key, F enqueue, SolveScalars &hs) {
   hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
-  if (use_graph) {
+  const bool keep = !key.empty();
+  if (use_graph && keep && c.solve_graph && c.solve_key == key) exec = c.solve_graph;
+  if (use_graph && !exec) {
+    hipGraph_t graph = nullptr;
     PZG_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < batch; k++) enqueue_iter();
+    enqueue();
     PZG_HIP(hipStreamEndCapture(c.stream, &graph));
-    PZG_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) {
+      set_error(std::string("pzg_solve: hipGraphInstantiate: ") + hipGetErrorString(e));
+      return PZG_EHIP;
+    }
+    if (keep) {
+      if (c.solve_graph) (void)hipGraphExecDestroy(c.solve_graph);
+      c.solve_graph = exec;
+      c.solve_key.swap(key);
+    }
   }
+  int rc = PZG_OK;
   for (;;) {
-    if (use_graph) PZG_HIP(hipGraphLaunch(exec, c.stream));
-    else
-      for (int k = 0; k < batch; k++) enqueue_iter();
-    PZG_HIP(hipMemcpyAsync(&hs, c.d_scal.p, sizeof(SolveScalars), hipMemcpyDeviceToHost, c.stream));
-    PZG_HIP(hipStreamSynchronize(c.stream));
+    hipError_t e = hipSuccess;
+    if (use_graph) e = hipGraphLaunch(exec, c.stream);
+    else enqueue();
+    if (e == hipSuccess) e = hipMemcpyAsync(&hs, c.d_scal.p, sizeof(SolveScalars), hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    if (e != hipSuccess) {
+      set_error(std::string("pzg_solve: iteration batch: ") + hipGetErrorString(e));
+      rc = PZG_EHIP;
+      break;
+    }
     if (hs.done) break;
   }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  return PZG_OK;
+  if (exec && !keep) (void)hipGraphExecDestroy(exec);
+  return rc;
 }
 
-// q = K p with the partials of p.q in slot 0; the number of partials
+// q = K p with the partials of p.q in slot 2; the number of partials
 static int pq64_grid(const Ctx &c) { return c.kf_valid ? kf_rows_grid(c) : bsr_grid(c.nb); }
 static void launch_pq64(Ctx &c, SolveScalars *sc, double *part) {
   if (c.kf_valid) {
-    (void)kf_apply(c, KF_DOT, c.d_p.as<double>(), nullptr, 1., 0., c.d_q.as<double>(), sc, part);
+    (void)kf_apply(c, KF_DOT, c.d_p.as<double>(), nullptr, 1., 0., c.d_q.as<double>(), sc, part + 2 * MAXBLK);
     return;
   }
   DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_spmv64_pq<BS>, dim3(bsr_grid(c.nb)), dim3(TPB), 0, c.stream, c.nb,
                                        c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(),
-                                       c.d_p.as<double>(), c.d_q.as<double>(), sc, part));
+                                       c.d_p.as<double>(), c.d_q.as<double>(), sc, part + 2 * MAXBLK));
+}
+
+enum { PRE_JACOBI = 0, PRE_BLOCK = 1, PRE_VBLOCK = 2 };
+// Direction formed inside the product (two launches an iteration) up to this
+// many stored scalars, beyond as a launch of its own: the second gathered
+// vector costs more than the launch once the product is bound by its gathers.
+// Merged against apart, ms per solve: 263k scalars (Poisson 64^2 p = 2) 2.99 /
+// 3.29, 456k (elasticity 12^3 p = 1) 6.81 / 6.91, 920k (Poisson 120^2) 9.63 /
+// 7.78; FCG: 0.4M (elasticity hp 8^3) 8.42 / 8.57, 6M (hp 21^3) 29.0 / 25.9,
+// 21M (tetrahedra, orders to 5) 109 / 34.
+constexpr int64_t PCG_MERGE_NNZ = (int64_t)1 << 19;
+
+// Iterations of PCG64 from the state that the start kernels left (x = d_u,
+// r = d_r, p = z, scalars in d_scal) until tol, maxit; hs receives the scalars.
+template <int BS>
+static int pcg64_iterate(Ctx &c, const pzg_solve_params &prm, int pre, SolveScalars &hs) {
+  const int64_t n = c.neq, nb = c.nb;
+  SolveScalars *A = c.d_scal.as<SolveScalars>(), *B = A + 1;
+  double *part = c.d_partials.as<double>();
+  const double *m = pre == PRE_JACOBI ? c.d_diag.as<double>() : c.d_bjinv64.as<double>();
+  const int64_t lds = cg_small_lds<BS>(nb, c.nbf, pre == PRE_BLOCK);
+  if (!c.kf_valid && pre != PRE_VBLOCK && lds <= CG_SMALL_LDS) {
+    int L = 1;
+    while (L < 16 && n * L * 2 <= CG_SMALL_TPB) L *= 2;
+    const void *fn = pre == PRE_BLOCK ? (const void *)k_cg_small<BS, true> : (const void *)k_cg_small<BS, false>;
+    PZG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CG_SMALL_LDS));
+    do {
+      if (pre == PRE_BLOCK)
+        hipLaunchKernelGGL((k_cg_small<BS, true>), dim3(1), dim3(CG_SMALL_TPB), (size_t)lds, c.stream, (int)nb,
+                           (int)c.nbf, L, c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), m,
+                           c.d_u.as<double>(), c.d_r.as<double>(), c.d_p.as<double>(), A);
+      else
+        hipLaunchKernelGGL((k_cg_small<BS, false>), dim3(1), dim3(CG_SMALL_TPB), (size_t)lds, c.stream, (int)nb,
+                           (int)c.nbf, L, c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), m,
+                           c.d_u.as<double>(), c.d_r.as<double>(), c.d_p.as<double>(), A);
+      PZG_HIP(hipGetLastError());
+      PZG_HIP(hipMemcpyAsync(&hs, A, sizeof(hs), hipMemcpyDeviceToHost, c.stream));
+      PZG_HIP(hipStreamSynchronize(c.stream));
+    } while (!hs.done);
+    return PZG_OK;
+  }
+  const CgGrid gu = cg_grid(nb), gd = cg_grid(n);
+  const int gv = grid_for(n, TPB), gs = pq64_grid(c);
+  const int n1 = pre == PRE_VBLOCK ? gv : gu.blocks;
+  const bool merge = !c.kf_valid && c.nbf * BS * BS <= PCG_MERGE_NNZ;
+  if (merge) PZG_TRY(dev_alloc(c.d_p2, n * sizeof(double)));
+  const int gm = std::min(gs, CG_MAXBLK);
+  double *r = c.d_r.as<double>(), *z = c.d_z.as<double>(), *q = c.d_q.as<double>(), *x = c.d_u.as<double>();
+  auto step = [&](double *p_old, double *p_new) {
+    double *p = merge ? p_new : c.d_p.as<double>();
+    if (merge) {
+      hipLaunchKernelGGL(k_pcg_step64<BS>, dim3(gm), dim3(TPB), 0, c.stream, nb, c.d_fbia.as<int64_t>(),
+                         c.d_fbja.as<int32_t>(), c.d_fa.as<double>(), (const double *)z, (const double *)p_old, p_new,
+                         q, (const SolveScalars *)A, B, part, gu.blocks, n1);
+    } else {
+      hipLaunchKernelGGL(k_pcg_dir64, dim3(gd.blocks), dim3(gd.tpb), 0, c.stream, n, (const double *)z, p,
+                         (const SolveScalars *)A, B, (const double *)part, gu.blocks, n1);
+      launch_pq64(c, B, part);
+    }
+    const int npq = merge ? gm : gs;
+#define PZG_UPD(P)                                                                                               \
+  hipLaunchKernelGGL((k_cg_update64<BS, P>), dim3(gu.blocks), dim3(gu.tpb), 0, c.stream, nb, x, r, z,            \
+                     (const double *)p, (const double *)q, m, A, (const SolveScalars *)B, part, npq)
+    if (pre == PRE_JACOBI) PZG_UPD(0);
+    else if (pre == PRE_BLOCK) PZG_UPD(1);
+    else PZG_UPD(2);
+#undef PZG_UPD
+    if (pre == PRE_VBLOCK)
+      hipLaunchKernelGGL(k_vbj_apply64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_vbj_eqb.as<int32_t>(),
+                         c.d_vbj_pos.as<int64_t>(), c.d_vbj_m.as<int32_t>(), c.d_vbj_off.as<int64_t>(), m,
+                         (const double *)r, z, (double *)nullptr, (const SolveScalars *)A, part);
+  };
+  // an even number of iterations: the two direction buffers are back in place
+  const int batch = ((prm.check_every > 0 ? prm.check_every : 50) + 1) / 2 * 2;
+  auto enqueue = [&]() {
+    double *p0 = c.d_p.as<double>(), *p1 = merge ? c.d_p2.as<double>() : p0;
+    for (int k = 0; k < batch; k += 2) {
+      step(p0, p1);
+      step(p1, p0);
+    }
+    hipLaunchKernelGGL(k_cg_close<false>, dim3(1), dim3(TPB), 0, c.stream, A, B, (const double *)part, gu.blocks, n1);
+  };
+  std::vector<uint64_t> key = {64, BS, (uint64_t)pre, (uint64_t)batch, (uint64_t)n, (uint64_t)nb, (uint64_t)c.nbf,
+                               (uint64_t)merge, (uint64_t)c.kf_valid, (uint64_t)c.nvol, (uint64_t)c.kf_nface,
+                               (uint64_t)c.vol_coef.empty()};
+  double coef0 = c.material == PZG_MAT_ELAST3D ? c.E : c.scale;
+  uint64_t cb;
+  std::memcpy(&cb, &coef0, sizeof(cb));
+  key.push_back(cb);
+  for (const DevBuf *b : {&c.d_scal, &c.d_partials, &c.d_diag, &c.d_bjinv64, &c.d_r, &c.d_z, &c.d_q, &c.d_u, &c.d_p,
+                          &c.d_p2, &c.d_fbia, &c.d_fbja, &c.d_fa, &c.d_vbj_eqb, &c.d_vbj_pos, &c.d_vbj_m,
+                          &c.d_vbj_off, &c.d_blk_iptr, &c.d_blk_inc, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab,
+                          &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_vcoef})
+    key.push_back((uint64_t)(uintptr_t)b->p);
+  return run_batches(c, prm.use_graph != 0, key, enqueue, hs);
 }
 
 // FP64 Jacobi-PCG iterations (the EJacobi CG<> of solve_pcg64) continued from
@@ -793,7 +1246,7 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
   for (DevBuf *b : {&c.d_z, &c.d_p, &c.d_q}) PZG_TRY(dev_alloc(*b, n * sizeof(double)));
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
-  const int gv = grid_for(n, TPB), gs = pq64_grid(c);
+  const int gv = grid_for(n, TPB);
   for (int round = 0; round < 4 && rel > prm.tol && iters < prm.max_iter; round++) {
     SolveScalars hs;
     std::memset(&hs, 0, sizeof(hs));
@@ -806,20 +1259,13 @@ static int pcg64_continue(Ctx &c, const pzg_solve_params &prm, int64_t &iters, d
                        c.d_diag.as<double>(), sc, part);
     hipLaunchKernelGGL(k_fin_cg_restart64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
     PZG_HIP(hipGetLastError());
-    auto iter = [&]() {
-      hipLaunchKernelGGL(k_p_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_z.as<double>(),
-                         c.d_p.as<double>(), sc);
-      launch_pq64(c, sc, part);
-      hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
-      hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
-                         c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
-                         c.d_q.as<double>(), c.d_diag.as<double>(), sc, (double *)nullptr, part);
-      hipLaunchKernelGGL(k_fin_cg64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv,
-                         (double *)nullptr);
-    };
     PZG_HIP(hipMemcpyAsync(&hs, c.d_scal.p, sizeof(hs), hipMemcpyDeviceToHost, c.stream));
     PZG_HIP(hipStreamSynchronize(c.stream));
-    if (!hs.done) PZG_TRY(run_batches(c, prm.check_every > 0 ? prm.check_every : 50, prm.use_graph != 0, iter, hs));
+    if (!hs.done) {
+      int rc = PZG_OK;
+      DISPATCH_BS(c.bs, rc = pcg64_iterate<BS>(c, prm, PRE_JACOBI, hs));
+      PZG_TRY(rc);
+    }
     iters = hs.iter;
     // true residual into d_r (the next round restarts from it)
     PZG_TRY(launch_residual64(c, c.d_u.as<double>(), c.d_r.as<double>(), part, c.d_res2.as<double>()));
@@ -903,42 +1349,22 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
                      c.d_u.as<double>(), c.d_r.as<double>(), c.d_z.as<double>(),
                      c.d_p.as<double>(), dg, sc, part);
   hipLaunchKernelGGL(k_fin_cg_init64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
-  auto vbj_apply = [&](const SolveScalars *s2) {
+  if (vblock) {
     hipLaunchKernelGGL(k_vbj_apply64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_vbj_eqb.as<int32_t>(),
                        c.d_vbj_pos.as<int64_t>(), c.d_vbj_m.as<int32_t>(), c.d_vbj_off.as<int64_t>(),
                        (const double *)c.d_bjinv64.as<double>(), (const double *)c.d_r.as<double>(),
-                       c.d_z.as<double>(), s2, part);
-  };
-  if (vblock) {
-    vbj_apply(nullptr);
+                       c.d_z.as<double>(), c.d_p.as<double>(), (const SolveScalars *)nullptr, part);
     hipLaunchKernelGGL(k_bj_rho64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
   } else if (block) {
     DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_bj_apply64<BS>, dim3(gv), dim3(TPB), 0, c.stream, c.nb,
                                          c.d_bjinv64.as<double>(), c.d_r.as<double>(), c.d_z.as<double>(),
-                                         (const SolveScalars *)nullptr, part));
+                                         c.d_p.as<double>(), part));
     hipLaunchKernelGGL(k_bj_rho64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv);
   }
   PZG_HIP(hipGetLastError());
-  const int gs = pq64_grid(c);
-  auto iter = [&]() {
-    hipLaunchKernelGGL(k_p_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_z.as<double>(),
-                       c.d_p.as<double>(), sc);
-    launch_pq64(c, sc, part);
-    hipLaunchKernelGGL(k_fin_alpha64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gs);
-    hipLaunchKernelGGL(k_cg_update64, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_u.as<double>(),
-                       c.d_r.as<double>(), c.d_z.as<double>(), c.d_p.as<double>(),
-                       c.d_q.as<double>(), dg, sc, (double *)nullptr, part);
-    if (vblock)
-      vbj_apply(sc);
-    else if (block)
-      DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_bj_apply64<BS>, dim3(gv), dim3(TPB), 0, c.stream, c.nb,
-                                           c.d_bjinv64.as<double>(), c.d_r.as<double>(), c.d_z.as<double>(),
-                                           (const SolveScalars *)sc, part));
-    hipLaunchKernelGGL(k_fin_cg64, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gv,
-                       (double *)nullptr);
-  };
-  int batch = prm.check_every > 0 ? prm.check_every : 50;
-  PZG_TRY(run_batches(c, batch, prm.use_graph != 0, iter, hs));
+  int rc = PZG_OK;
+  DISPATCH_BS(c.bs, rc = pcg64_iterate<BS>(c, prm, vblock ? PRE_VBLOCK : block ? PRE_BLOCK : PRE_JACOBI, hs));
+  PZG_TRY(rc);
   PZG_HIP(hipEventRecord(c.ev1, c.stream));
   PZG_HIP(hipEventSynchronize(c.ev1));
   float ms = 0;
@@ -995,94 +1421,90 @@ __global__ __launch_bounds__(TPB) void k_fcg_spmv(int64_t nb, const int64_t *__r
   block_partials<2>(vv, partials);
 }
 
-// alpha = (p.r)/(p.q)   (one block).  A pending update request (4) raised by
-// the previous iteration becomes 5 here, so that the completion kernels of that
-// iteration (prolongation, p update), which run on 4, do not run again.
-__global__ void k_fin_fcg_alpha(SolveScalars *sc, const double *partials, int nblk) {
-  if (sc->done == 4) {
-    __syncthreads();
-    if (threadIdx.x == 0) sc->done = 5;
+// x += alpha p; r -= alpha q; rr (slot 0); with binv z = Binv r (block Jacobi)
+// and z.q (slot 1), else z is left to the preconditioner's own kernels.
+// alpha = (p.r)/(p.q) from the product's partials (slots 3 and 2).
+template <int BS>
+__global__ __launch_bounds__(1024) void k_fcg_update(int64_t nb, float *__restrict__ x,
+                                                     float *__restrict__ r, float *__restrict__ z,
+                                                     const float *__restrict__ p,
+                                                     const float *__restrict__ q,
+                                                     const float *__restrict__ binv,
+                                                     SolveScalars *A, const SolveScalars *B,
+                                                     double *partials, int npq) {
+  if (B->done) {
+    close_step(A, B, B->pq, 0);
     return;
   }
-  if (sc->done) return;
-  double pq = sum_partials(partials, 0, nblk);
-  double pr = sum_partials(partials, 1, nblk);
-  if (threadIdx.x == 0) {
-    sc->pq = pq;
-    sc->pr = pr;
-    sc->alpha = pr / pq;
-  }
-}
-
-// x += alpha p; r -= alpha q; z = Binv r (block Jacobi); rr, zq; beta = -zq/pq
-template <int BS>
-__global__ __launch_bounds__(TPB) void k_fcg_update(int64_t nb, float *__restrict__ x,
-                                                    float *__restrict__ r, float *__restrict__ z,
-                                                    const float *__restrict__ p,
-                                                    const float *__restrict__ q,
-                                                    const float *__restrict__ binv,
-                                                    SolveScalars *sc, double *partials) {
-  if (sc->done) return;
-  const float alpha = (float)sc->alpha;
+  const int slot[2] = {2, 3}, cnt[2] = {npq, npq};
+  double t[2];
+  sum_slots<2>(partials, slot, cnt, t);
+  const float alpha = (float)(t[1] / t[0]);
   double rr = 0., zq = 0.;
-  int64_t A = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t st = (int64_t)gridDim.x * blockDim.x;
-  for (; A < nb; A += st) {
-    float rv[BS];
+  for (int64_t R = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; R < nb; R += (int64_t)gridDim.x * blockDim.x) {
+    float rv[BS], qv[BS];
+#pragma unroll
     for (int k = 0; k < BS; k++) {
-      const int64_t i = A * BS + k;
+      const int64_t i = R * BS + k;
+      qv[k] = q[i];
       x[i] += alpha * p[i];
-      rv[k] = r[i] - alpha * q[i];
+      rv[k] = r[i] - alpha * qv[k];
       r[i] = rv[k];
       rr += (double)rv[k] * rv[k];
     }
-    const float *bi = binv + A * BS * BS;
+    if (!binv) continue;
+    const float *bi = binv + R * BS * BS;
+#pragma unroll
     for (int k = 0; k < BS; k++) {
-      float s = 0.f;
-      for (int l = 0; l < BS; l++) s += bi[k * BS + l] * rv[l];
-      z[A * BS + k] = s;
-      zq += (double)s * q[A * BS + k];
+      float u = 0.f;
+#pragma unroll
+      for (int l = 0; l < BS; l++) u += bi[k * BS + l] * rv[l];
+      z[R * BS + k] = u;
+      zq += (double)u * qv[k];
     }
   }
-  double vv[2] = {rr, zq};
-  block_partials<2>(vv, partials);
+  if (binv) {
+    double vv[2] = {rr, zq};
+    store_slots<2>(vv, partials);
+  } else {
+    double vv[1] = {rr};
+    store_slots<1>(vv, partials);
+  }
+  close_step(A, B, t[0], 3);
 }
 
-// stop tests on |r| (what & 1), beta = -(z.q)/(p.q) (what & 2)   (one block;
-// slot 1 may have been rewritten by the preconditioner).  Under the multigrid
-// cycle of a restarted FCG the stop test runs alone before the cycle (what =
-// 1, update due = 5: no kernel of this iteration is left to run), since the
-// restart recomputes z: the last cycle of every refinement step is not run
-// (3 of 23 cycles on a 256^2 Darcy solve, 3 of 87 at 48^3, 3 of 38 at 64^3
-// with the learned smoother).
-__global__ void k_fin_fcg_beta(SolveScalars *sc, const double *partials, int nblk, int what) {
+// Stop test on |r| before the multigrid cycle of a restarted FCG (one block;
+// update due = 5: no kernel of this iteration is left to run): the restart
+// recomputes z, so the last cycle of every refinement step is not run (3 of 23
+// cycles on a 256^2 Darcy solve, 3 of 87 at 48^3, 3 of 38 at 64^3 with the
+// learned smoother).
+__global__ void k_fin_fcg_stop(SolveScalars *sc, const double *partials, int nblk) {
   if (sc->done) return;
-  double rr = what & 1 ? sum_partials(partials, 0, nblk) : 0.;
-  double zq = what & 2 ? sum_partials(partials, 1, nblk) : 0.;
+  const double rr = sum_partials(partials, 0, nblk);
   if (threadIdx.x == 0) {
-    if (what & 1) {
-      int64_t it = sc->iter + 1;
-      sc->iter = it;
-      double rn = sqrt(rr);
-      double resid = rn / sc->normb;
-      // divergence guard: leave the loop, the host restarts from the true residual
-      if (!(resid == resid) || resid > 1e3) sc->done = 3;
-      else if (rn < sc->delta * sc->rlast) sc->done = what & 2 ? 4 : 5;
-      else if (it >= sc->maxit) sc->done = 2;
-      sc->resid = resid;
-    }
-    if (what & 2) sc->beta = -zq / sc->pq;
+    int64_t it = sc->iter + 1;
+    sc->iter = it;
+    double rn = sqrt(rr);
+    double resid = rn / sc->normb;
+    // divergence guard: leave the loop, the host restarts from the true residual
+    if (!(resid == resid) || resid > 1e3) sc->done = 3;
+    else if (rn < sc->delta * sc->rlast) sc->done = 5;
+    else if (it >= sc->maxit) sc->done = 2;
+    sc->resid = resid;
+    sc->pend = 2;
   }
 }
 
-// runs when the iteration completed normally (done 0) or completed and asked
-// for a reliable update (done 4)
-// p = z + beta p; with pt: also pt = D^-1/2 p (input of the matrix-free operator)
-__global__ void k_p_update32(int64_t n, const float *__restrict__ z, float *__restrict__ p,
-                             const SolveScalars *sc, const float *__restrict__ dis = nullptr,
-                             float *__restrict__ pt = nullptr) {
-  if (sc->done != 0 && sc->done != 4) return;
-  const float beta = (float)sc->beta;
+// p = z + beta p; with pt: also pt = D^-1/2 p (input of the matrix-free
+// operator).  An update request (4) still completes its direction.
+__global__ __launch_bounds__(1024) void k_fcg_dir32(int64_t n, const float *__restrict__ z, float *__restrict__ p,
+                                                    const float *__restrict__ dis, float *__restrict__ pt,
+                                                    const SolveScalars *A, SolveScalars *B, const double *partials,
+                                                    int n0, int n1) {
+  double bt;
+  bool upd;
+  if (!next_direction<true>(A, B, partials, n0, n1, &bt, &upd) || !upd) return;
+  const float beta = (float)bt;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t st = (int64_t)gridDim.x * blockDim.x;
   if (pt) {
@@ -1094,6 +1516,40 @@ __global__ void k_p_update32(int64_t n, const float *__restrict__ z, float *__re
   } else {
     for (; i < n; i += st) p[i] = z[i] + beta * p[i];
   }
+}
+
+// the stored operator with the direction formed inside the product (as
+// k_pcg_step64): p = z + beta p_old, q = S p, p.q and p.r (slots 2 and 3)
+template <int BS>
+__global__ __launch_bounds__(TPB) void k_fcg_step32(int64_t nb, const int64_t *__restrict__ bia,
+                                                    const int32_t *__restrict__ bja,
+                                                    const float *__restrict__ v, const float *__restrict__ z,
+                                                    const float *__restrict__ p_old, float *__restrict__ p_new,
+                                                    const float *__restrict__ r, float *__restrict__ q,
+                                                    const SolveScalars *A, SolveScalars *B, double *partials, int n0,
+                                                    int n1) {
+  double bt;
+  bool upd;
+  if (!next_direction<true>(A, B, partials, n0, n1, &bt, &upd)) return;
+  const float beta = (float)bt;
+  const int sub = threadIdx.x % BSR_L;
+  constexpr int RPB = TPB / BSR_L;
+  double pq = 0., pr = 0.;
+  auto dir = [=](int64_t i) { return upd ? z[i] + beta * p_old[i] : p_old[i]; };
+  for (int64_t R = (int64_t)blockIdx.x * RPB + threadIdx.x / BSR_L; R < nb; R += (int64_t)gridDim.x * RPB) {
+    float out[BS];
+    bsr_row_f<float, BS>(R, bia, bja, v, dir, sub, out);
+    if (sub < BS) {
+      const int64_t i = R * BS + sub;
+      const float o = pick<float, BS>(out, sub), pi = dir(i);
+      q[i] = o;
+      p_new[i] = pi;
+      pq += (double)o * pi;
+      pr += (double)pi * r[i];
+    }
+  }
+  double vv[2] = {pq, pr};
+  store_slots<2>(vv, partials + 2 * MAXBLK);
 }
 
 // b = D^-1/2 r64 (fp32); x = 0; r = b; z = Binv r; p = z; normb = |b|
@@ -1136,6 +1592,7 @@ __global__ void k_fin_fcg_init(SolveScalars *sc, const double *partials, int nbl
     sc->normb = nbv > 0. ? nbv : 1.;
     sc->rlast = nbv;
     sc->resid = nbv > 0. ? 1. : 0.;
+    sc->pend = 0;  // p = z follows from the start kernels
     sc->done = nbv > 0. ? 0 : 1;
   }
 }
@@ -1186,6 +1643,7 @@ int launch_spmv_bsr(Ctx &c, const float *x, float *y) {
   return PZG_OK;
 }
 
+constexpr int64_t FCG_MERGE_NNZ = PCG_MERGE_NNZ;
 constexpr int64_t MG_INNER_CAP = 2000;  // FP32 iterations per refinement step, multigrid paths
 
 template <int BS>
@@ -1220,6 +1678,15 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
   SolveScalars *sc = c.d_scal.as<SolveScalars>();
   double *part = c.d_partials.as<double>();
   const int gv = grid_for(n, TPB), gb = grid_for(nb, TPB), gs = bsr_grid(nb);
+  const CgGrid gu = cg_grid(nb), gd = cg_grid(n);
+  const int gm = std::min(gs, CG_MAXBLK);
+  const int nfin = gb;  // grid of the cycle's last kernel, which forms z.q
+  SolveScalars *sb = sc + 1;
+  // direction formed inside the stored product (two launches an iteration);
+  // the reliable update keeps the direction across batches, so it takes the
+  // separate launch
+  const bool merge = !use_mf && !multigrid && prm.refine == 0 && c.nbf * BS * BS <= FCG_MERGE_NNZ;
+  if (merge) PZG_TRY(dev_alloc(c.d_ps2, n * sizeof(float)));
   PZG_HIP(hipEventRecord(c.ev0, c.stream));
   hipLaunchKernelGGL(k_axpby64, dim3(gv), dim3(TPB), 0, c.stream, n, 0.0, c.d_f.as<double>(), 0.0,
                      (const double *)nullptr, c.d_u.as<double>());
@@ -1228,7 +1695,7 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
   double rel = 1.0, fnorm = 0.;
   bool conv = false;
   // a multigrid iteration costs several operator applications: short batches
-  const int batch = prm.check_every > 0 ? prm.check_every : (multigrid ? 4 : 50);
+  const int batch = ((prm.check_every > 0 ? prm.check_every : (multigrid ? 4 : 50)) + 1) / 2 * 2;
   auto true_res = [&](bool u_zero = false) -> int {
     if (u_zero)  // the starting guess: no product needed
       hipLaunchKernelGGL(k_residual_zero, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_f.as<double>(),
@@ -1363,35 +1830,67 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
       if (use_mf) PZG_TRY(mf_scale(c, c.d_ps.as<float>(), sc));
       restart = false;
     }
-    auto iter = [&]() {
-      int ga = gs;
-      if (use_mf) {
-        (void)mf_apply(c, c.d_ps.as<float>(), c.d_rs.as<float>(), c.d_qs.as<float>(), sc, part, &ga,
-                       true);
+    auto step = [&](const float *p_old, float *p_new) {
+      const bool early = multigrid && prm.refine == 0;
+      const int n1 = multigrid ? nfin : vbj ? gb : gu.blocks;
+      float *p = merge ? p_new : c.d_ps.as<float>();
+      int ga = merge ? gm : gs;
+      if (merge) {
+        hipLaunchKernelGGL(k_fcg_step32<BS>, dim3(gm), dim3(TPB), 0, c.stream, nb, c.d_fbia.as<int64_t>(),
+                           c.d_fbja.as<int32_t>(), c.d_bsr.as<float>(), (const float *)c.d_zs.as<float>(), p_old,
+                           p_new, (const float *)c.d_rs.as<float>(), c.d_qs.as<float>(), (const SolveScalars *)sc, sb,
+                           part, gu.blocks, n1);
       } else {
-        hipLaunchKernelGGL(k_fcg_spmv<BS>, dim3(gs), dim3(TPB), 0, c.stream, nb,
-                           c.d_fbia.as<int64_t>(), c.d_fbja.as<int32_t>(), c.d_bsr.as<float>(),
-                           c.d_ps.as<float>(), c.d_rs.as<float>(), c.d_qs.as<float>(), sc, part);
+        hipLaunchKernelGGL(k_fcg_dir32, dim3(gd.blocks), dim3(gd.tpb), 0, c.stream, n,
+                           (const float *)c.d_zs.as<float>(), p, use_mf ? c.d_mf_dis.as<float>() : nullptr,
+                           use_mf ? c.d_mf_pt.as<float>() : nullptr, (const SolveScalars *)sc, sb,
+                           (const double *)part, gu.blocks, n1);
+        if (use_mf)
+          (void)mf_apply(c, p, c.d_rs.as<float>(), c.d_qs.as<float>(), sb, part + 2 * MAXBLK, &ga, true);
+        else
+          hipLaunchKernelGGL(k_fcg_spmv<BS>, dim3(gs), dim3(TPB), 0, c.stream, nb, c.d_fbia.as<int64_t>(),
+                             c.d_fbja.as<int32_t>(), c.d_bsr.as<float>(), (const float *)p, c.d_rs.as<float>(),
+                             c.d_qs.as<float>(), sb, part + 2 * MAXBLK);
       }
-      hipLaunchKernelGGL(k_fin_fcg_alpha, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, ga);
-      hipLaunchKernelGGL(k_fcg_update<BS>, dim3(gb), dim3(TPB), 0, c.stream, nb,
-                         c.d_xs.as<float>(), c.d_rs.as<float>(), c.d_zs.as<float>(),
-                         c.d_ps.as<float>(), c.d_qs.as<float>(), c.d_bjinv.as<float>(), sc, part);
+      hipLaunchKernelGGL(k_fcg_update<BS>, dim3(gu.blocks), dim3(gu.tpb), 0, c.stream, nb, c.d_xs.as<float>(),
+                         c.d_rs.as<float>(), c.d_zs.as<float>(), (const float *)p, (const float *)c.d_qs.as<float>(),
+                         multigrid || vbj ? (const float *)nullptr : c.d_bjinv.as<float>(), sc,
+                         (const SolveScalars *)sb, part, ga);
       // S couples the penalty rows to the others (at the 1/sqrt(big) level):
       // keep their residual at zero rather than let it drift
       if (pen_rows) (void)pen_zero32(c, c.d_rs.as<float>());
-      const bool early = multigrid && prm.refine == 0;
-      if (early)
-        hipLaunchKernelGGL(k_fin_fcg_beta, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb, 1);
+      if (early) hipLaunchKernelGGL(k_fin_fcg_stop, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gu.blocks);
       if (multigrid)
         (void)mg_apply(c, c.d_rs.as<float>(), c.d_zs.as<float>(), nullptr, c.d_qs.as<float>(), sc, part);
       if (vbj) vbj_apply(c.d_zs.as<float>(), nullptr, c.d_qs.as<float>());
-      hipLaunchKernelGGL(k_fin_fcg_beta, dim3(1), dim3(TPB), 0, c.stream, sc, (const double *)part, gb, early ? 2 : 3);
-      hipLaunchKernelGGL(k_p_update32, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_zs.as<float>(),
-                         c.d_ps.as<float>(), sc, use_mf ? c.d_mf_dis.as<float>() : nullptr,
-                         use_mf ? c.d_mf_pt.as<float>() : nullptr);
     };
-    PZG_TRY(run_batches(c, batch, prm.use_graph != 0, iter, hs));
+    auto enqueue = [&]() {
+      float *p0 = c.d_ps.as<float>(), *p1 = merge ? c.d_ps2.as<float>() : p0;
+      for (int k = 0; k < batch; k += 2) {
+        step(p0, p1);
+        step(p1, p0);
+      }
+      hipLaunchKernelGGL(k_cg_close<true>, dim3(1), dim3(TPB), 0, c.stream, sc, sb, (const double *)part, gu.blocks,
+                         multigrid ? nfin : vbj ? gb : gu.blocks);
+    };
+    // the cycle's launches hold coefficients of this assembly: its graph is
+    // not kept beyond the solve
+    std::vector<uint64_t> key;
+    if (!multigrid) {
+      key = {32, BS, (uint64_t)batch, (uint64_t)n, (uint64_t)nb, (uint64_t)c.nbf, (uint64_t)merge, (uint64_t)use_mf,
+             (uint64_t)vbj, (uint64_t)c.nvol, (uint64_t)c.mf_nbcd, (uint64_t)c.tvol.nq};
+      double nu = c.nu;
+      uint64_t cb;
+      std::memcpy(&cb, &nu, sizeof(cb));
+      key.push_back(cb);
+      for (const DevBuf *b : {&c.d_scal, &c.d_partials, &c.d_xs, &c.d_rs, &c.d_zs, &c.d_ps, &c.d_ps2, &c.d_qs,
+                              &c.d_bjinv, &c.d_bsr, &c.d_fbia, &c.d_fbja, &c.d_vbj_eqb, &c.d_vbj_pos, &c.d_vbj_m,
+                              &c.d_vbj_off, &c.d_vbjinv32, &c.d_mf_dis, &c.d_mf_pt, &c.d_mf_blk, &c.d_mf_xe,
+                              &c.d_mf_bblk, &c.d_mf_bm, &c.d_mf_ptr, &c.d_mf_pos, &c.d_mf_bpos, &c.d_mf_tab,
+                              &c.d_mf_ye, &c.d_mf_coef, &c.d_mf_mfma, &c.d_mf_geo})
+        key.push_back((uint64_t)(uintptr_t)b->p);
+    }
+    PZG_TRY(run_batches(c, prm.use_graph != 0, key, enqueue, hs));
     total_it = hs.iter;
     // fold the FP32 correction into the FP64 solution and recompute the true residual
     hipLaunchKernelGGL(k_ir_update, dim3(gv), dim3(TPB), 0, c.stream, n, c.d_xs.as<float>(),
