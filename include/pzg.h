@@ -366,7 +366,9 @@ int pzg_scaled_apply(pzg_ctx *ctx, int32_t op, const double *x, double *y);
  * that of lattice level l (0 for a densely solved coarsest level; arrays of
  * 48 and 16 entries; any may be NULL).  The
  * levels are built on the first call after an assembly.  Exposes the mixed
- * solver's multigrid preconditioner, which has no reference counterpart. */
+ * solver's multigrid preconditioner, which has no reference counterpart; where
+ * an odd element count stops the halving above 1536 unknowns the solver has
+ * further levels in place of the polynomial. */
 #define PZG_MG_LEARNED 4
 int pzg_mg_apply(pzg_ctx *ctx, int32_t op, int32_t degree, double range, const double *r, double *z,
                  int32_t *nlev, int32_t *dims, double *lmax);

@@ -1881,9 +1881,9 @@ int pzg_mg_apply(pzg_ctx *ctx, int32_t op, int32_t degree, double range, const d
   c.mg_degree = degree > 0 ? degree : 2;
   c.mg_range = range > 0 ? range : 30.;
   const bool use_mf = op == PZG_INNER_MATFREE;
-  if (!c.mg_ready || c.mg_use_mf != use_mf || c.mg_les != learned) {
+  if (!c.mg_ready || c.mg_use_mf != use_mf || c.mg_les != learned || mg_levels(c) != c.mg_nstd) {
     c.mg_les = learned;  // level-0 smoothing: learned element smoother or block Jacobi
-    PZG_TRY(mg_setup(c, use_mf));
+    PZG_TRY(mg_setup(c, use_mf, false));
   }
   std::vector<float> h(n);
   for (int64_t i = 0; i < n; i++) h[i] = (float)r[i];
@@ -1894,8 +1894,8 @@ int pzg_mg_apply(pzg_ctx *ctx, int32_t op, int32_t degree, double range, const d
   PZG_HIP(hipMemcpyAsync(h.data(), c.d_zs.p, n * sizeof(float), hipMemcpyDeviceToHost, c.stream));
   PZG_HIP(hipStreamSynchronize(c.stream));
   for (int64_t i = 0; i < n; i++) z[i] = h[i];
-  const int nl = (int)std::min<size_t>(c.mg.size(), 15);
-  if (nlev) *nlev = (int32_t)c.mg.size();
+  const int nl = (int)std::min<size_t>(mg_levels(c), 15);
+  if (nlev) *nlev = (int32_t)mg_levels(c);
   if (dims)
     for (int l = 0; l < nl; l++)
       for (int d = 0; d < 3; d++) dims[3 * l + d] = c.mg[l].n[d];

@@ -380,6 +380,10 @@ struct Ctx {
       d_pen_sval, d_pen_sinv, d_pen_gptr, d_pen_gslot, d_pen_w, d_pen_scal;
   hipGraphExec_t pen_graph = nullptr;  // one batch of its CG iterations
   bool mg_struct = false;  // lattice, levels and buffers of the current mesh
+  // levels by halving even element counts; the solver's cycle (mg_ext) goes on
+  // below them when they stop above the dense limit (mg_levels)
+  size_t mg_nstd = 0;
+  bool mg_ext = false;
   bool mg_dense = true;    // the coarsest level has a dense inverse (else a Chebyshev solve)
   int mg_degree = 2;       // Chebyshev degree of the pre- and post-smoothing
   double mg_range = 30.;   // ratio of the smoothed interval's ends
@@ -466,7 +470,10 @@ int mf_setup(Ctx &c);
 // multigrid preconditioner: levels, operators and eigenvalue estimates of the
 // current system (use_mf: level 0 applied matrix-free); z = V-cycle(r), then
 // p = z and the z.q partials of the FCG update (when p / q are given)
-int mg_setup(Ctx &c, bool use_mf);
+// ext: with the levels below an odd element count (the solver's cycle)
+int mg_setup(Ctx &c, bool use_mf, bool ext);
+inline size_t mg_levels(const Ctx &c) { return c.mg_ext ? c.mg.size() : c.mg_nstd; }
+inline bool mg_dense_coarse(const Ctx &c) { return c.mg_dense || mg_levels(c) > c.mg_nstd; }
 int mg_apply(Ctx &c, const float *r, float *z, float *p, const float *q, SolveScalars *sc,
              double *partials);
 void mg_free(Ctx &c);

@@ -16,9 +16,10 @@
 // Galerkin product A_c = P^T A P formed on the device, while every element
 // count is even and the level is too large for the dense solve; the coarsest
 // level is solved with a dense inverse when it has at most MG_MAXDENSE
-// unknowns; a larger one (an odd element count stopped the halving) gets a
-// Chebyshev iteration of degree MG_COARSE_DEGREE from zero instead, a fixed
-// SPD polynomial in M^-1 A, so the cycle stays a fixed SPD operator.
+// unknowns.  Where an odd element count stops the halving above that, the
+// solver's cycle goes on with levels that keep the last node (fine_of);
+// pzg_mg_apply alone puts a Chebyshev iteration of degree MG_COARSE_DEGREE
+// from zero there, a fixed SPD polynomial in M^-1 A.
 //
 // Smoother: Chebyshev iteration (Saad, Iterative Methods for Sparse Linear
 // Systems, 2nd ed., Alg. 12.1) of degree m on M^-1 A, M = the diagonal
@@ -201,9 +202,38 @@ __global__ void k_stencil(Dims D, int64_t nn, const float *__restrict__ A, const
   }
 }
 
+// Trilinear transfer along one direction with nf fine and nc coarse nodes: nc
+// == nf leaves the direction as it is (1 or 2 nodes); an odd number of
+// elements (nf even) keeps the last fine node as a coarse node of its own, at
+// half the distance of the others.
+// fine node of coarse node I at offset dx in {-1,0,1} and its weight
+__device__ inline bool fine_of(int I, int dx, int nc, int nf, int &i, float &w) {
+  i = 2 * I + dx;
+  w = dx ? 0.5f : 1.f;
+  if (nc == nf) {
+    i = I;
+    return dx == 0;
+  }
+  if (!(nf & 1)) {
+    if (I == nc - 1) {
+      i = nf - 1;
+      return dx == 0;
+    }
+    if (i == nf - 1) return false;
+  }
+  return i >= 0 && i < nf;
+}
+// first coarse node of fine node i and their number (two: weight 1/2 each)
+__device__ inline int coarse_of(int i, int nc, int nf, int &n) {
+  n = 1;
+  if (nc == nf) return i;
+  if (!(nf & 1) && i == nf - 1) return nc - 1;
+  n = (i & 1) ? 2 : 1;
+  return i >> 1;
+}
+
 // trilinear restriction of the residual r_f - t_f (the pre-smoothing leaves
-// its last product t_f unsubtracted): b_c(N) = sum over the fine nodes
-// 2N + d, d in {-1,0,1}^3, of prod_i (1 - |d_i|/2) (r_f - t_f)
+// its last product t_f unsubtracted)
 template <int BS>
 __global__ void k_restrict(Dims C, Dims F, const float *__restrict__ rf, const float *__restrict__ tf,
                            float *__restrict__ bc, const SolveScalars *sc) {
@@ -217,15 +247,18 @@ __global__ void k_restrict(Dims C, Dims F, const float *__restrict__ rf, const f
 #pragma unroll
     for (int e = 0; e < BS; e++) acc[e] = 0.f;
     for (int dz = -1; dz <= 1; dz++) {
-      const int k = 2 * K + dz;
-      if (k < 0 || k >= F.n[2]) continue;
+      int k;
+      float wk;
+      if (!fine_of(K, dz, C.n[2], F.n[2], k, wk)) continue;
       for (int dy = -1; dy <= 1; dy++) {
-        const int j = 2 * J + dy;
-        if (j < 0 || j >= F.n[1]) continue;
+        int j;
+        float wj;
+        if (!fine_of(J, dy, C.n[1], F.n[1], j, wj)) continue;
         for (int dx = -1; dx <= 1; dx++) {
-          const int i = 2 * I + dx;
-          if (i < 0 || i >= F.n[0]) continue;
-          const float w = (dx ? 0.5f : 1.f) * (dy ? 0.5f : 1.f) * (dz ? 0.5f : 1.f);
+          int i;
+          float wi;
+          if (!fine_of(I, dx, C.n[0], F.n[0], i, wi)) continue;
+          const float w = wi * wj * wk;
           const int64_t f = node_id(F, i, j, k);
 #pragma unroll
           for (int e = 0; e < BS; e++) acc[e] += w * (rf[f * BS + e] - tf[f * BS + e]);
@@ -247,9 +280,10 @@ __global__ void k_prolong(Dims C, Dims F, const float *__restrict__ xc, float *_
        v += (int64_t)gridDim.x * blockDim.x) {
     int i, j, k;
     node_ijk(F, v, i, j, k);
-    const int i0 = i >> 1, j0 = j >> 1, k0 = k >> 1;
-    const int ni = (i & 1) ? 2 : 1, nj = (j & 1) ? 2 : 1, nk = (k & 1) ? 2 : 1;
-    const float wi = (i & 1) ? 0.5f : 1.f, wj = (j & 1) ? 0.5f : 1.f, wk = (k & 1) ? 0.5f : 1.f;
+    int ni, nj, nk;
+    const int i0 = coarse_of(i, C.n[0], F.n[0], ni), j0 = coarse_of(j, C.n[1], F.n[1], nj),
+              k0 = coarse_of(k, C.n[2], F.n[2], nk);
+    const float wi = ni == 2 ? 0.5f : 1.f, wj = nj == 2 ? 0.5f : 1.f, wk = nk == 2 ? 0.5f : 1.f;
     float acc[BS];
 #pragma unroll
     for (int e = 0; e < BS; e++) acc[e] = 0.f;
@@ -378,10 +412,9 @@ __global__ void k_mg_zero(int64_t n, float *__restrict__ x) {
 }
 
 // Galerkin product A_c = P^T A_f P for trilinear P, one thread per coarse
-// (node, stencil entry).  Along each direction the fine node f = 2N + a
-// (a in {-1,0,1}, weight 1 - |a|/2) couples to the fine node g = 2M + b of
-// the neighbour M = N + o when |g - f| <= 1; the pairs (a, b) are enumerated
-// per direction.
+// (node, stencil entry).  Along each direction the fine nodes f of N (fine_of)
+// couple to the fine nodes g of the neighbour M = N + o when |g - f| <= 1; the
+// pairs are enumerated per direction.
 template <int BS>
 __global__ void k_mg_rap(Dims C, Dims F, const float *__restrict__ Af, float *__restrict__ Ac) {
   const int64_t nc = (int64_t)C.n[0] * C.n[1] * C.n[2];
@@ -406,14 +439,14 @@ __global__ void k_mg_rap(Dims C, Dims F, const float *__restrict__ Af, float *__
       np[d] = 0;
       const int M = N[d] + o[d];
       for (int a = -1; a <= 1; a++) {
-        const int f = 2 * N[d] + a;
-        if (f < 0 || f >= F.n[d]) continue;
+        int f, g;
+        float wf, wg;
+        if (!fine_of(N[d], a, C.n[d], F.n[d], f, wf)) continue;
         for (int b = -1; b <= 1; b++) {
-          const int g = 2 * M + b;
-          if (g < 0 || g >= F.n[d] || g - f < -1 || g - f > 1) continue;
+          if (!fine_of(M, b, C.n[d], F.n[d], g, wg) || g - f < -1 || g - f > 1) continue;
           pf[d][np[d]] = f;
           pg[d][np[d]] = g - f;
-          pw[d][np[d]] = (a ? 0.5f : 1.f) * (b ? 0.5f : 1.f);
+          pw[d][np[d]] = wf * wg;
           np[d]++;
         }
       }
@@ -897,6 +930,24 @@ int structure_impl(Ctx &c) {
     c.mg.push_back(std::move(l));
   }
   c.mg_dense = c.mg.back().nn * BS <= MG_MAXDENSE;
+  c.mg_nstd = c.mg.size();
+  // the solver's cycle goes on where an odd count stopped the halving above
+  // the dense limit: every direction with more than one element is coarsened,
+  // an odd count keeping its last node (fine_of).  A 255^2 lattice (256^2
+  // nodes) with the polynomial in place of these levels took 205 FCG
+  // iterations, with them as many as its even neighbour.
+  while (!c.mg_dense && c.mg.back().nn * BS > MG_DENSE) {
+    const MgLevel &f = c.mg.back();
+    MgLevel l;
+    bool less = false;
+    for (int d = 0; d < 3; d++) {
+      l.n[d] = f.n[d] <= 2 ? f.n[d] : f.n[d] / 2 + 1;  // (odd n: (n - 1)/2 + 1)
+      less |= l.n[d] < f.n[d];
+    }
+    if (!less) break;
+    l.nn = (int64_t)l.n[0] * l.n[1] * l.n[2];
+    c.mg.push_back(std::move(l));
+  }
   // device arrays
   PZG_TRY(dev_upload(c.d_mg_vmap, vmap.data(), vmap.size(), c.stream));
   {
@@ -931,19 +982,22 @@ int setup_impl(Ctx &c) {
                      c.d_mg_vmap.as<int32_t>(), c.d_mg_vinv.as<int32_t>(), c.d_ia.as<int64_t>(),
                      c.d_a.as<double>(), c.d_ubia.as<int64_t>(), c.d_ubja.as<int32_t>(), c.mg[0].A.as<float>());
   PZG_HIP(hipGetLastError());
-  for (size_t k = 1; k < c.mg.size(); k++) {
+  const size_t nl = mg_levels(c);
+  const bool dense = mg_dense_coarse(c);
+  for (size_t k = 1; k < nl; k++) {
     hipLaunchKernelGGL(k_mg_rap<BS>, dim3(gridx(27 * BS * BS * c.mg[k].nn)), dim3(TPB), 0, c.stream, dims_of(c.mg[k]),
                        dims_of(c.mg[k - 1]), c.mg[k - 1].A.as<float>(), c.mg[k].A.as<float>());
     PZG_HIP(hipGetLastError());
   }
-  for (MgLevel &l : c.mg) {
+  for (size_t k = 0; k < nl; k++) {
+    MgLevel &l = c.mg[k];
     hipLaunchKernelGGL(k_mg_minv<BS>, dim3(gridx(l.nn)), dim3(TPB), 0, c.stream, l.nn, l.A.as<float>(),
                        l.minv.as<float>());
     PZG_HIP(hipGetLastError());
   }
   // dense inverse of the coarsest level
-  if (c.mg_dense) {
-    const MgLevel &l = c.mg.back();
+  if (dense) {
+    const MgLevel &l = c.mg[nl - 1];
     const int nd = (int)(l.nn * BS);
     std::vector<float> h((size_t)27 * BS * BS * l.nn);
     PZG_HIP(hipMemcpyAsync(h.data(), l.A.p, h.size() * sizeof(float), hipMemcpyDeviceToHost, c.stream));
@@ -1007,7 +1061,7 @@ int setup_impl(Ctx &c) {
                              c.d_mg_d0.as<float>(), c.d_mg_t0.as<float>(), c.d_mg_w0.as<float>(), op,
                              c.mg_lmax0, c.mg_les));
   }
-  for (size_t k = 0; k + (c.mg_dense ? 1 : 0) < c.mg.size(); k++) {
+  for (size_t k = 0; k + (dense ? 1 : 0) < nl; k++) {
     MgLevel &l = c.mg[k];
     auto op = [&](const float *x, float *y) { return op_lattice<BS>(c, l, x, y, nullptr); };
     PZG_TRY(lanczos_lmax<BS>(c, l.nn, l.minv.as<float>(), 1, l.nn, l.x.as<float>(), l.b.as<float>(),
@@ -1025,7 +1079,7 @@ int apply_impl(Ctx &c, const float *r, float *z, float *p, const float *q, Solve
                double *partials) {
   const LevelView L0 = view0(c);
   auto op_0 = [&](const float *x, float *y, bool ps) { return op0(c, x, y, sc, ps); };
-  const int nl = (int)c.mg.size();
+  const int nl = (int)mg_levels(c);
   PZG_TRY(smooth_pre<BS>(c, L0, r, z, op_0, sc));
   hipLaunchKernelGGL(k_restrict0<BS>, dim3(grid1(c.mg[0].nn)), dim3(TPB), 0, c.stream, c.mg[0].nn,
                      c.d_mg_vmap.as<int32_t>(), c.d_mg_dsq.as<float>(), L0.r, L0.t, c.mg[0].b.as<float>(), sc);
@@ -1039,12 +1093,12 @@ int apply_impl(Ctx &c, const float *r, float *z, float *p, const float *q, Solve
                        dims_of(c.mg[k + 1]), dims_of(l), V.r, V.t, c.mg[k + 1].b.as<float>(), sc);
     PZG_HIP(hipGetLastError());
   }
-  if (c.mg_dense) {
+  if (mg_dense_coarse(c)) {
     hipLaunchKernelGGL(k_dense, dim3(gridx(c.mg_ncoarse * 64)), dim3(TPB), 0, c.stream, (int)c.mg_ncoarse,
-                       c.d_mg_cinv.as<float>(), c.mg.back().b.as<float>(), c.mg.back().x.as<float>(), sc);
+                       c.d_mg_cinv.as<float>(), c.mg[nl - 1].b.as<float>(), c.mg[nl - 1].x.as<float>(), sc);
     PZG_HIP(hipGetLastError());
   } else {  // x = q(M^-1 A) M^-1 b, a Chebyshev iteration from zero
-    MgLevel &l = c.mg.back();
+    MgLevel &l = c.mg[nl - 1];
     LevelView V = view_l(c, l);
     V.ch = cheb_coeffs(l.lmax, MG_COARSE_RANGE, MG_COARSE_DEGREE);
     auto op = [&](const float *x, float *y, bool) { return op_lattice<BS>(c, l, x, y, sc); };
@@ -1087,9 +1141,10 @@ void mg_free(Ctx &c) {
   c.mg_ready = false;
 }
 
-int mg_setup(Ctx &c, bool use_mf) {
+int mg_setup(Ctx &c, bool use_mf, bool ext) {
   c.mg_ready = false;
   c.mg_use_mf = use_mf;
+  c.mg_ext = ext;
   if (c.mg_degree < 1 || c.mg_degree > 8 || !(c.mg_range > 1.)) {
     set_error("multigrid preconditioner: degree must be 1..8 and the range above 1");
     return PZG_EINVAL;

@@ -1756,9 +1756,9 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
     // per step at 60 against 152 ms at 30, the same at 100)
     c.mg_degree = prm.mg_degree > 0 ? prm.mg_degree : 2;
     c.mg_range = prm.mg_range > 0 ? prm.mg_range : les ? 60. : 30.;
-    if (!c.mg_ready || c.mg_use_mf != use_mf || c.mg_les != les) {
+    if (!c.mg_ready || c.mg_use_mf != use_mf || c.mg_les != les || (!c.mg_ext && mg_levels(c) < c.mg.size())) {
       c.mg_les = les;
-      PZG_TRY(mg_setup(c, use_mf));
+      PZG_TRY(mg_setup(c, use_mf, true));
     }
     if (les && !c.pen_ready) PZG_TRY(pen_setup(c));
   }
