@@ -166,40 +166,15 @@ __global__ void k_les_res(int64_t n, int mode, const float *__restrict__ b, cons
 struct Dims {
   int n[3];
 };
+// (lattices hold at most INT32_MAX nodes: 32-bit divisions)
 __device__ inline void node_ijk(const Dims &D, int64_t v, int &i, int &j, int &k) {
-  i = (int)(v % D.n[0]);
-  const int64_t q = v / D.n[0];
-  j = (int)(q % D.n[1]);
-  k = (int)(q / D.n[1]);
+  const uint32_t u = (uint32_t)v, q = u / (uint32_t)D.n[0];
+  i = (int)(u - q * (uint32_t)D.n[0]);
+  k = (int)(q / (uint32_t)D.n[1]);
+  j = (int)(q - (uint32_t)k * (uint32_t)D.n[1]);
 }
 __device__ inline int64_t node_id(const Dims &D, int i, int j, int k) {
   return i + (int64_t)D.n[0] * (j + (int64_t)D.n[1] * k);
-}
-
-// y = A x over the 27-point block stencil; stencil entry s = (dz+1)*9 +
-// (dy+1)*3 + (dx+1), value (s, e) of node v at A[(s*BS*BS + e)*nn + v].
-// One thread per (node, row component a), node fastest: the small levels
-// are latency-bound and take BS times the threads.
-template <int BS>
-__global__ void k_stencil(Dims D, int64_t nn, const float *__restrict__ A, const float *__restrict__ x,
-                          float *__restrict__ y, const SolveScalars *sc) {
-  if (stopped(sc)) return;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nn * BS;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t v = t % nn;
-    const int a = (int)(t / nn);
-    int i, j, k;
-    node_ijk(D, v, i, j, k);
-    float acc = 0.f;
-    for (int s = 0; s < 27; s++) {
-      const int ii = i + s % 3 - 1, jj = j + (s / 3) % 3 - 1, kk = k + s / 9 - 1;
-      if (ii < 0 || jj < 0 || kk < 0 || ii >= D.n[0] || jj >= D.n[1] || kk >= D.n[2]) continue;
-      const int64_t w = node_id(D, ii, jj, kk);
-#pragma unroll
-      for (int b = 0; b < BS; b++) acc += A[((int64_t)s * BS * BS + a * BS + b) * nn + v] * x[w * BS + b];
-    }
-    y[v * BS + a] = acc;
-  }
 }
 
 // Trilinear transfer along one direction with nf fine and nc coarse nodes: nc
@@ -232,88 +207,323 @@ __device__ inline int coarse_of(int i, int nc, int nf, int &n) {
   return i >> 1;
 }
 
-// trilinear restriction of the residual r_f - t_f (the pre-smoothing leaves
-// its last product t_f unsubtracted)
+// The steps of a lattice level (one Chebyshev step before and after the coarse
+// correction).  The start d = c0 M^-1 b comes from the kernel that forms b, so a
+// level is: residual b - A d, restriction (which starts the coarser level),
+// then x = d + P x_c and x + c0 M^-1 (b - A x).  On planes the last two are one
+// kernel (a row reads 9 neighbours, their x formed on the way); on
+// three-dimensional levels the sum is its own kernel (27 neighbours of up to 8
+// coarse nodes each).  Three or four launches a level instead of six, and no
+// r, t vectors.
+
+// Entries off the lattice hold zeros, so the 9 neighbours of a plane of nodes
+// are read at clamped indices without a branch: their loads are in flight
+// together.  With a branch per neighbour (serialised loads): residual at 49^3
+// nodes and below 20.3 us on average, now 13.7; the tails below 39 us on
+// planes and 47 us from 7^3 nodes x 3, now 25.5 and 31.6.
+
+// (A x)(v, a) over the block stencil; xf(w, i, j, k, b): entry b of node w =
+// (i, j, k)
+template <int BS, class X>
+__device__ inline float stencil_row(const Dims &D, int64_t nn, const float *__restrict__ A, int64_t v, int a, X xf) {
+  int i, j, k;
+  node_ijk(D, v, i, j, k);
+  float acc = 0.f;
+#pragma unroll 1
+  for (int dz = -1; dz <= 1; dz++) {
+    const int kk = k + dz;
+    if (kk < 0 || kk >= D.n[2]) continue;
+    float av[9][BS], xv[9][BS];
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+      const int ii = min(max(i + t % 3 - 1, 0), D.n[0] - 1), jj = min(max(j + t / 3 - 1, 0), D.n[1] - 1);
+      const int64_t w = node_id(D, ii, jj, kk);
+      const float *ap = A + ((int64_t)((dz + 1) * 9 + t) * BS * BS + a * BS) * nn + v;
+#pragma unroll
+      for (int b = 0; b < BS; b++) {
+        av[t][b] = ap[b * nn];
+        xv[t][b] = xf(w, ii, jj, kk, b);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+      for (int b = 0; b < BS; b++) acc += av[t][b] * xv[t][b];
+  }
+  return acc;
+}
+
+// P^T r at coarse node v
+template <int BS, class R>
+__device__ inline void restrict_node(const Dims &C, const Dims &F, int64_t v, R rf, float (&acc)[BS]) {
+  int I, J, K;
+  node_ijk(C, v, I, J, K);
+#pragma unroll
+  for (int e = 0; e < BS; e++) acc[e] = 0.f;
+  int fi[3], fj[3];
+  float wi[3], wj[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    if (!fine_of(I, d - 1, C.n[0], F.n[0], fi[d], wi[d])) fi[d] = min(2 * I, F.n[0] - 1), wi[d] = 0.f;
+    if (!fine_of(J, d - 1, C.n[1], F.n[1], fj[d], wj[d])) fj[d] = min(2 * J, F.n[1] - 1), wj[d] = 0.f;
+  }
+#pragma unroll 1
+  for (int dz = -1; dz <= 1; dz++) {
+    int k;
+    float wk;
+    if (!fine_of(K, dz, C.n[2], F.n[2], k, wk)) continue;
+    float rv[9][BS];
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+      const int64_t f = node_id(F, fi[t % 3], fj[t / 3], k);
+#pragma unroll
+      for (int e = 0; e < BS; e++) rv[t][e] = rf(f, e);
+    }
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+      const float w = wi[t % 3] * wj[t / 3] * wk;
+#pragma unroll
+      for (int e = 0; e < BS; e++) acc[e] += w * rv[t][e];
+    }
+  }
+}
+
+// (P x_c) at fine node (i, j, k), entry e: both coarse neighbours of every
+// direction, the second with weight 0 where the node lies on the first
+template <class X>
+__device__ inline float prolong_value(const Dims &C, const Dims &F, int i, int j, int k, int e, X xc) {
+  int ni, nj, nk;
+  const int i0 = coarse_of(i, C.n[0], F.n[0], ni), j0 = coarse_of(j, C.n[1], F.n[1], nj),
+            k0 = coarse_of(k, C.n[2], F.n[2], nk);
+  const int i1 = i0 + ni - 1, j1 = j0 + nj - 1;
+  const float a0 = ni == 2 ? 0.5f : 1.f, a1 = 1.f - a0, b0 = nj == 2 ? 0.5f : 1.f, b1 = 1.f - b0;
+  float acc = 0.f;
+  for (int c = 0; c < nk; c++) {
+    const float v00 = xc(node_id(C, i0, j0, k0 + c), e), v10 = xc(node_id(C, i1, j0, k0 + c), e),
+                v01 = xc(node_id(C, i0, j1, k0 + c), e), v11 = xc(node_id(C, i1, j1, k0 + c), e);
+    acc += b0 * (a0 * v00 + a1 * v10) + b1 * (a0 * v01 + a1 * v11);
+  }
+  return nk == 2 ? 0.5f * acc : acc;
+}
+
+// y = A x over the 27-point block stencil (set-up and the polynomial coarse
+// solve); stencil entry s = (dz+1)*9 + (dy+1)*3 + (dx+1), value (s, e) of node v
+// at A[(s*BS*BS + e)*nn + v].  One thread per (node, row component a on
+// grid y): the small levels are latency-bound and take BS times the threads.
 template <int BS>
-__global__ void k_restrict(Dims C, Dims F, const float *__restrict__ rf, const float *__restrict__ tf,
-                           float *__restrict__ bc, const SolveScalars *sc) {
+__global__ void k_stencil(Dims D, int64_t nn, const float *__restrict__ A, const float *__restrict__ x,
+                          float *__restrict__ y, const SolveScalars *sc) {
+  if (stopped(sc)) return;
+  const int a = blockIdx.y;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nn; v += (int64_t)gridDim.x * blockDim.x)
+    y[v * BS + a] = stencil_row<BS>(D, nn, A, v, a, [x](int64_t w, int, int, int, int e) { return x[w * BS + e]; });
+}
+
+// r = b - A d, one thread per (node, component), component on grid y
+template <int BS>
+__global__ void k_lat_res(Dims D, int64_t nn, const float *__restrict__ A, const float *__restrict__ b,
+                          const float *__restrict__ d, float *__restrict__ r, const SolveScalars *sc) {
+  if (stopped(sc)) return;
+  const int a = blockIdx.y;
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nn; v += (int64_t)gridDim.x * blockDim.x)
+    r[v * BS + a] = b[v * BS + a] - stencil_row<BS>(D, nn, A, v, a, [d](int64_t w, int, int, int, int e) { return d[w * BS + e]; });
+}
+
+// b_c = P^T r; with m: d_c = c0 M_c^-1 b_c
+template <int BS>
+__global__ void k_lat_restrict(Dims C, Dims F, const float *__restrict__ r, float *__restrict__ bc,
+                               const float *__restrict__ m, float c0, float *__restrict__ dc,
+                               const SolveScalars *sc) {
   if (stopped(sc)) return;
   const int64_t nc = (int64_t)C.n[0] * C.n[1] * C.n[2];
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nc;
        v += (int64_t)gridDim.x * blockDim.x) {
-    int I, J, K;
-    node_ijk(C, v, I, J, K);
-    float acc[BS];
-#pragma unroll
-    for (int e = 0; e < BS; e++) acc[e] = 0.f;
-    for (int dz = -1; dz <= 1; dz++) {
-      int k;
-      float wk;
-      if (!fine_of(K, dz, C.n[2], F.n[2], k, wk)) continue;
-      for (int dy = -1; dy <= 1; dy++) {
-        int j;
-        float wj;
-        if (!fine_of(J, dy, C.n[1], F.n[1], j, wj)) continue;
-        for (int dx = -1; dx <= 1; dx++) {
-          int i;
-          float wi;
-          if (!fine_of(I, dx, C.n[0], F.n[0], i, wi)) continue;
-          const float w = wi * wj * wk;
-          const int64_t f = node_id(F, i, j, k);
-#pragma unroll
-          for (int e = 0; e < BS; e++) acc[e] += w * (rf[f * BS + e] - tf[f * BS + e]);
-        }
-      }
-    }
+    float acc[BS], y[BS];
+    restrict_node<BS>(C, F, v, [r](int64_t f, int e) { return r[f * BS + e]; }, acc);
 #pragma unroll
     for (int e = 0; e < BS; e++) bc[v * BS + e] = acc[e];
+    if (!m) continue;
+    minv_mul<BS>(m, 1, nc, v, acc, y);
+#pragma unroll
+    for (int e = 0; e < BS; e++) dc[v * BS + e] = c0 * y[e];
   }
 }
 
-// trilinear prolongation, added: x_f += P x_c
+// x += P x_c (x holds d), one thread per (node, component)
 template <int BS>
-__global__ void k_prolong(Dims C, Dims F, const float *__restrict__ xc, float *__restrict__ xf,
-                          const SolveScalars *sc) {
+__global__ void k_lat_prolong(Dims C, Dims F, const float *__restrict__ xc, float *__restrict__ x,
+                              const SolveScalars *sc) {
   if (stopped(sc)) return;
-  const int64_t nf = (int64_t)F.n[0] * F.n[1] * F.n[2];
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nf;
-       v += (int64_t)gridDim.x * blockDim.x) {
+  const int64_t n = (int64_t)F.n[0] * F.n[1] * F.n[2] * BS;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t v = t / BS;
     int i, j, k;
     node_ijk(F, v, i, j, k);
-    int ni, nj, nk;
-    const int i0 = coarse_of(i, C.n[0], F.n[0], ni), j0 = coarse_of(j, C.n[1], F.n[1], nj),
-              k0 = coarse_of(k, C.n[2], F.n[2], nk);
-    const float wi = ni == 2 ? 0.5f : 1.f, wj = nj == 2 ? 0.5f : 1.f, wk = nk == 2 ? 0.5f : 1.f;
-    float acc[BS];
-#pragma unroll
-    for (int e = 0; e < BS; e++) acc[e] = 0.f;
-    for (int c = 0; c < nk; c++)
-      for (int b = 0; b < nj; b++)
-        for (int a = 0; a < ni; a++) {
-          const int64_t w = node_id(C, i0 + a, j0 + b, k0 + c);
-#pragma unroll
-          for (int e = 0; e < BS; e++) acc[e] += xc[w * BS + e];
-        }
-    const float s = wi * wj * wk;
-#pragma unroll
-    for (int e = 0; e < BS; e++) xf[v * BS + e] += s * acc[e];
+    x[t] += prolong_value(C, F, i, j, k, (int)(t - v * BS), [xc](int64_t w, int e) { return xc[w * BS + e]; });
   }
 }
 
-// level 0 <-> level 1: b1(v) = D^1/2 (r0 - t0) at the vertex block vmap[v];
-// x0(vmap[v]) += D^1/2 x1(v)
+// out = x + c0 M^-1 (b - A x); xc: x = d + P x_c formed on the way (planes), else
+// x = d as given.  A workgroup takes LAT_NT nodes, wavefronts of one component
+// each (coalesced stencil reads), the residual's components exchanged through
+// LDS.  With vmap (the first lattice level): the correction goes straight to
+// level 0, x0(vmap[v]) += D^1/2 out.
+template <int BS> constexpr int lat_nt() { return BS == 1 ? 256 : 64; }
+template <int BS>
+__global__ __launch_bounds__(lat_nt<BS>() * BS) void k_lat_post(Dims D, int64_t nn, const float *__restrict__ A,
+                                                                const float *__restrict__ m,
+                                                                const float *__restrict__ b,
+                                                                const float *__restrict__ d, Dims C,
+                                                                const float *__restrict__ xc, float c0,
+                                                                float *__restrict__ out,
+                                                                const int32_t *__restrict__ vmap,
+                                                                const float *__restrict__ dsq,
+                                                                float *__restrict__ x0, const SolveScalars *sc) {
+  if (stopped(sc)) return;
+  constexpr int NT = lat_nt<BS>();
+  __shared__ float sr[BS][NT];
+  const int l = threadIdx.x % NT, a = threadIdx.x / NT;
+  for (int64_t v0 = (int64_t)blockIdx.x * NT; v0 < nn; v0 += (int64_t)gridDim.x * NT) {
+    const int64_t v = v0 + l;
+    auto xf = [&](int64_t w, int i, int j, int k, int e) {
+      return d[w * BS + e] + (xc ? prolong_value(C, D, i, j, k, e, [xc](int64_t q, int f) { return xc[q * BS + f]; }) : 0.f);
+    };
+    float res = 0.f, y = 0.f;
+    if (v < nn) res = b[v * BS + a] - stencil_row<BS>(D, nn, A, v, a, xf);
+    if (BS > 1) {
+      __syncthreads();
+      sr[a][l] = res;
+      __syncthreads();
+    }
+    if (v >= nn) continue;
+#pragma unroll
+    for (int e = 0; e < BS; e++) y += m[(int64_t)(a * BS + e) * nn + v] * (BS > 1 ? sr[e][l] : res);
+    int i, j, k;
+    node_ijk(D, v, i, j, k);
+    const float x = xf(v, i, j, k, a) + c0 * y;
+    if (vmap) x0[(int64_t)vmap[v] * BS + a] += dsq[v * BS + a] * x;
+    else out[v * BS + a] = x;
+  }
+}
+
+// The levels from the first whose stencil is at most MG_TAIL_BYTES down to the
+// dense solve, in one workgroup: every vector in LDS, the stencils and the
+// inverse read through the L2, barriers in place of launches.  Bound by that
+// CU's L2 reads and the barriers: 25.5 us from 65^2 nodes down (10 launches of
+// about 3.5 us apart), 15.5 us from 5^3 x 3 (7 launches), 31.6 us from 7^3 x 3
+// with a dense solve of 192 (6 launches).
+constexpr int MG_TAIL_MAX = 12;
+constexpr int64_t MG_TAIL_BYTES = 400 * 1024;
+constexpr int64_t MG_TAIL_LDS = 100 * 1024;
+constexpr int MG_TAIL_TPB = 1024;
+struct TailArgs {
+  int nl;  // levels, the last one dense
+  int n[MG_TAIL_MAX][3];
+  int off[MG_TAIL_MAX];  // first of the level's three vectors in LDS (floats)
+  const float *A[MG_TAIL_MAX], *m[MG_TAIL_MAX];
+  float c0[MG_TAIL_MAX];
+  const float *cinv, *b, *d;
+  float *x;
+};
+template <int BS>
+__global__ __launch_bounds__(MG_TAIL_TPB) void k_lat_tail(TailArgs t, const SolveScalars *sc) {
+  extern __shared__ float tl[];
+  if (stopped(sc)) return;
+  const int tid = threadIdx.x;
+  auto dims = [&](int k) { return Dims{{t.n[k][0], t.n[k][1], t.n[k][2]}}; };
+  auto count = [&](int k) { return t.n[k][0] * t.n[k][1] * t.n[k][2]; };
+  // vectors of level k: b, d (then x), r
+  const int n0 = count(0) * BS;
+  for (int i = tid; i < n0; i += MG_TAIL_TPB) {
+    tl[t.off[0] + i] = t.b[i];
+    if (t.nl > 1) tl[t.off[0] + n0 + i] = t.d[i];
+  }
+  __syncthreads();
+  for (int k = 0; k + 1 < t.nl; k++) {
+    const Dims D = dims(k), C = dims(k + 1);
+    const int nn = count(k), nc = count(k + 1);
+    float *b = tl + t.off[k], *d = b + nn * BS, *r = d + nn * BS;
+    float *bc = tl + t.off[k + 1], *dc = bc + nc * BS;
+    for (int i = tid; i < nn * BS; i += MG_TAIL_TPB) {
+      const int v = i % nn, a = i / nn;
+      r[v * BS + a] = b[v * BS + a] - stencil_row<BS>(D, nn, t.A[k], v, a, [d](int64_t w, int, int, int, int e) { return d[w * BS + e]; });
+    }
+    __syncthreads();
+    const bool start = k + 2 < t.nl;
+    for (int v = tid; v < nc; v += MG_TAIL_TPB) {
+      float acc[BS], y[BS];
+      restrict_node<BS>(C, D, v, [r](int64_t f, int e) { return r[f * BS + e]; }, acc);
+      for (int e = 0; e < BS; e++) bc[v * BS + e] = acc[e];
+      if (!start) continue;
+      minv_mul<BS>(t.m[k + 1], 1, nc, v, acc, y);
+      for (int e = 0; e < BS; e++) dc[v * BS + e] = t.c0[k + 1] * y[e];
+    }
+    __syncthreads();
+  }
+  {  // dense solve: 16 lanes a row
+    const int k = t.nl - 1, nd = count(k) * BS;
+    const float *b = tl + t.off[k];
+    float *x = tl + t.off[k] + nd;
+    const int lane = tid & 15;
+    for (int i0 = 0; i0 < nd; i0 += MG_TAIL_TPB / 16) {
+      const int i = i0 + (tid >> 4);
+      float s = 0.f;
+      if (i < nd)
+        for (int j = lane; j < nd; j += 16) s += t.cinv[(int64_t)i * nd + j] * b[j];
+      s = row16_sum(s);
+      if (i < nd && lane == 0) x[i] = s;
+    }
+    __syncthreads();
+  }
+  for (int k = t.nl - 2; k >= 0; k--) {
+    const Dims D = dims(k), C = dims(k + 1);
+    const int nn = count(k), nc = count(k + 1);
+    float *b = tl + t.off[k], *d = b + nn * BS, *r = d + nn * BS;
+    const float *xc = tl + t.off[k + 1] + nc * BS;
+    for (int u = tid; u < nn * BS; u += MG_TAIL_TPB) {
+      int i, j, l;
+      node_ijk(D, u / BS, i, j, l);
+      d[u] += prolong_value(C, D, i, j, l, u % BS, [xc](int64_t w, int e) { return xc[w * BS + e]; });
+    }
+    __syncthreads();
+    for (int i = tid; i < nn * BS; i += MG_TAIL_TPB) {
+      const int v = i % nn, a = i / nn;
+      r[v * BS + a] = b[v * BS + a] - stencil_row<BS>(D, nn, t.A[k], v, a, [d](int64_t w, int, int, int, int e) { return d[w * BS + e]; });
+    }
+    __syncthreads();
+    for (int i = tid; i < nn * BS; i += MG_TAIL_TPB) {
+      const int v = i % nn, a = i / nn;
+      float y = 0.f;
+      for (int e = 0; e < BS; e++) y += t.m[k][(int64_t)(a * BS + e) * nn + v] * r[v * BS + e];
+      d[v * BS + a] += t.c0[k] * y;
+    }
+    __syncthreads();
+  }
+  for (int i = tid; i < n0; i += MG_TAIL_TPB) t.x[i] = tl[t.off[0] + n0 + i];
+}
+
+// level 0 -> level 1: b1(v) = D^1/2 (r0 - t0) at the vertex block vmap[v]; with
+// m: d1 = c0 M^-1 b1
 template <int BS>
 __global__ void k_restrict0(int64_t nn, const int32_t *__restrict__ vmap, const float *__restrict__ dsq,
                             const float *__restrict__ r0, const float *__restrict__ t0,
-                            float *__restrict__ b1, const SolveScalars *sc) {
+                            float *__restrict__ b1, const float *__restrict__ m, float c0,
+                            float *__restrict__ d1, const SolveScalars *sc) {
   if (stopped(sc)) return;
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nn;
        v += (int64_t)gridDim.x * blockDim.x) {
     const int64_t A = vmap[v];
+    float bv[BS], y[BS];
 #pragma unroll
-    for (int e = 0; e < BS; e++) b1[v * BS + e] = dsq[v * BS + e] * (r0[A * BS + e] - t0[A * BS + e]);
+    for (int e = 0; e < BS; e++) b1[v * BS + e] = bv[e] = dsq[v * BS + e] * (r0[A * BS + e] - t0[A * BS + e]);
+    if (!m) continue;
+    minv_mul<BS>(m, 1, nn, v, bv, y);
+#pragma unroll
+    for (int e = 0; e < BS; e++) d1[v * BS + e] = c0 * y[e];
   }
 }
+// x0(vmap[v]) += D^1/2 x1(v) (a hierarchy whose first lattice level is the
+// coarsest or inside the tail; else k_lat_post does it)
 template <int BS>
 __global__ void k_prolong0(int64_t nn, const int32_t *__restrict__ vmap, const float *__restrict__ dsq,
                            const float *__restrict__ x1, float *__restrict__ x0, const SolveScalars *sc) {
@@ -471,7 +681,7 @@ __global__ void k_mg_minv(int64_t nn, const float *__restrict__ A, float *__rest
   double a[BS * BS];
   for (int e = 0; e < BS * BS; e++) a[e] = A[((int64_t)13 * BS * BS + e) * nn + v];
   double r[BS * BS];
-  if (BS == 1) {
+  if constexpr (BS == 1) {
     r[0] = a[0] != 0. ? 1. / a[0] : 0.;
   } else {
     const double c00 = a[4] * a[8] - a[5] * a[7], c01 = a[5] * a[6] - a[3] * a[8],
@@ -615,7 +825,7 @@ int op0(Ctx &c, const float *x, float *y, const SolveScalars *sc, bool prescaled
 
 template <int BS>
 int op_lattice(Ctx &c, const MgLevel &l, const float *x, float *y, const SolveScalars *sc) {
-  hipLaunchKernelGGL(k_stencil<BS>, dim3(grid1(l.nn * BS)), dim3(TPB), 0, c.stream, dims_of(l), l.nn,
+  hipLaunchKernelGGL(k_stencil<BS>, dim3(grid1(l.nn), BS), dim3(TPB), 0, c.stream, dims_of(l), l.nn,
                      l.A.as<float>(), x, y, sc);
   PZG_HIP(hipGetLastError());
   return PZG_OK;
@@ -964,6 +1174,8 @@ int structure_impl(Ctx &c) {
     PZG_TRY(dev_alloc(l.minv, sizeof(float) * BS * BS * l.nn));
     for (DevBuf *b : {&l.x, &l.b, &l.r, &l.d, &l.t}) PZG_TRY(dev_alloc(*b, sizeof(float) * BS * l.nn));
   }
+  PZG_HIP(hipFuncSetAttribute((const void *)k_lat_tail<BS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)MG_TAIL_LDS));
   c.mg_struct = true;
   return PZG_OK;
 }
@@ -1080,42 +1292,90 @@ int apply_impl(Ctx &c, const float *r, float *z, float *p, const float *q, Solve
   const LevelView L0 = view0(c);
   auto op_0 = [&](const float *x, float *y, bool ps) { return op0(c, x, y, sc, ps); };
   const int nl = (int)mg_levels(c);
+  const bool dense = mg_dense_coarse(c);
+  std::vector<LevelView> V(nl);
+  for (int k = 0; k < nl; k++) V[k] = view_l(c, c.mg[k]);
+  // first level of the tail (nl: none)
+  int kt = nl;
+  if (dense) {
+    int64_t fl = 0;
+    while (kt > 0 && nl - (kt - 1) <= MG_TAIL_MAX) {
+      const MgLevel &l = c.mg[kt - 1];
+      const int64_t by = l.nn * BS * BS * 4 * (l.n[2] == 1 ? 9 : 27), f = 3 * l.nn * BS;
+      // (the coarsest level is read as its inverse, not as a stencil)
+      if ((kt < nl ? by > MG_TAIL_BYTES : c.mg_ncoarse * c.mg_ncoarse * 4 > MG_TAIL_BYTES) ||
+          (fl + f) * 4 > MG_TAIL_LDS)
+        break;
+      fl += f;
+      kt--;
+    }
+    if (nl - kt < 2) kt = nl;  // the dense solve alone is a launch either way
+  }
+  auto first = [&](int k) { return k < nl - 1 || !dense ? V[k].m : (const float *)nullptr; };  // smoothed levels
   PZG_TRY(smooth_pre<BS>(c, L0, r, z, op_0, sc));
   hipLaunchKernelGGL(k_restrict0<BS>, dim3(grid1(c.mg[0].nn)), dim3(TPB), 0, c.stream, c.mg[0].nn,
-                     c.d_mg_vmap.as<int32_t>(), c.d_mg_dsq.as<float>(), L0.r, L0.t, c.mg[0].b.as<float>(), sc);
+                     c.d_mg_vmap.as<int32_t>(), c.d_mg_dsq.as<float>(), L0.r, L0.t, c.mg[0].b.as<float>(), first(0),
+                     V[0].ch.c0, c.mg[0].d.as<float>(), sc);
   PZG_HIP(hipGetLastError());
-  for (int k = 0; k + 1 < nl; k++) {
-    MgLevel &l = c.mg[k];
-    const LevelView V = view_l(c, l);
-    auto op = [&](const float *x, float *y, bool) { return op_lattice<BS>(c, l, x, y, sc); };
-    PZG_TRY(smooth_pre<BS>(c, V, l.b.as<float>(), l.x.as<float>(), op, sc));
-    hipLaunchKernelGGL(k_restrict<BS>, dim3(grid1(c.mg[k + 1].nn)), dim3(TPB), 0, c.stream,
-                       dims_of(c.mg[k + 1]), dims_of(l), V.r, V.t, c.mg[k + 1].b.as<float>(), sc);
+  for (int k = 0; k + 1 < nl && k < kt; k++) {
+    MgLevel &l = c.mg[k], &q = c.mg[k + 1];
+    hipLaunchKernelGGL(k_lat_res<BS>, dim3(grid1(l.nn), BS), dim3(TPB), 0, c.stream, dims_of(l), l.nn,
+                       l.A.as<float>(), l.b.as<float>(), l.d.as<float>(), l.r.as<float>(), sc);
+    hipLaunchKernelGGL(k_lat_restrict<BS>, dim3(grid1(q.nn)), dim3(TPB), 0, c.stream, dims_of(q), dims_of(l),
+                       l.r.as<float>(), q.b.as<float>(), first(k + 1), V[k + 1].ch.c0, q.d.as<float>(), sc);
     PZG_HIP(hipGetLastError());
   }
-  if (mg_dense_coarse(c)) {
+  if (kt < nl) {
+    TailArgs t;
+    std::memset(&t, 0, sizeof(t));
+    t.nl = nl - kt;
+    int off = 0;
+    for (int k = kt; k < nl; k++) {
+      const MgLevel &l = c.mg[k];
+      for (int d = 0; d < 3; d++) t.n[k - kt][d] = l.n[d];
+      t.off[k - kt] = off;
+      off += (int)(3 * l.nn * BS);
+      t.A[k - kt] = l.A.as<float>();
+      t.m[k - kt] = l.minv.as<float>();
+      t.c0[k - kt] = V[k].ch.c0;
+    }
+    t.cinv = c.d_mg_cinv.as<float>();
+    t.b = c.mg[kt].b.as<float>();
+    t.d = c.mg[kt].d.as<float>();
+    t.x = c.mg[kt].x.as<float>();
+    hipLaunchKernelGGL(k_lat_tail<BS>, dim3(1), dim3(MG_TAIL_TPB), sizeof(float) * off, c.stream, t, sc);
+    PZG_HIP(hipGetLastError());
+  } else if (dense) {
     hipLaunchKernelGGL(k_dense, dim3(gridx(c.mg_ncoarse * 64)), dim3(TPB), 0, c.stream, (int)c.mg_ncoarse,
                        c.d_mg_cinv.as<float>(), c.mg[nl - 1].b.as<float>(), c.mg[nl - 1].x.as<float>(), sc);
     PZG_HIP(hipGetLastError());
   } else {  // x = q(M^-1 A) M^-1 b, a Chebyshev iteration from zero
     MgLevel &l = c.mg[nl - 1];
-    LevelView V = view_l(c, l);
-    V.ch = cheb_coeffs(l.lmax, MG_COARSE_RANGE, MG_COARSE_DEGREE);
+    LevelView W = V[nl - 1];
+    W.ch = cheb_coeffs(l.lmax, MG_COARSE_RANGE, MG_COARSE_DEGREE);
     auto op = [&](const float *x, float *y, bool) { return op_lattice<BS>(c, l, x, y, sc); };
-    PZG_TRY(smooth_pre<BS>(c, V, l.b.as<float>(), l.x.as<float>(), op, sc));
+    PZG_TRY(smooth_pre<BS>(c, W, l.b.as<float>(), l.x.as<float>(), op, sc));
   }
-  for (int k = nl - 2; k >= 0; k--) {
-    MgLevel &l = c.mg[k];
-    hipLaunchKernelGGL(k_prolong<BS>, dim3(grid1(l.nn)), dim3(TPB), 0, c.stream, dims_of(c.mg[k + 1]),
-                       dims_of(l), c.mg[k + 1].x.as<float>(), l.x.as<float>(), sc);
+  const int kup = std::min(nl - 1, kt);  // levels above the one just solved
+  for (int k = kup - 1; k >= 0; k--) {
+    MgLevel &l = c.mg[k], &q = c.mg[k + 1];
+    const bool plane = l.n[2] == 1;
+    if (!plane)
+      hipLaunchKernelGGL(k_lat_prolong<BS>, dim3(grid1(l.nn * BS)), dim3(TPB), 0, c.stream, dims_of(q), dims_of(l),
+                         q.x.as<float>(), l.d.as<float>(), sc);
+    constexpr int NT = lat_nt<BS>();
+    hipLaunchKernelGGL(k_lat_post<BS>, dim3((unsigned)std::max<int64_t>(1, (l.nn + NT - 1) / NT)), dim3(NT * BS), 0,
+                       c.stream, dims_of(l), l.nn, l.A.as<float>(), l.minv.as<float>(), l.b.as<float>(),
+                       l.d.as<float>(), dims_of(q), plane ? q.x.as<float>() : (const float *)nullptr, V[k].ch.c0,
+                       l.x.as<float>(), k == 0 ? c.d_mg_vmap.as<int32_t>() : (const int32_t *)nullptr,
+                       c.d_mg_dsq.as<float>(), z, sc);
     PZG_HIP(hipGetLastError());
-    const LevelView V = view_l(c, l);
-    auto op = [&](const float *x, float *y, bool) { return op_lattice<BS>(c, l, x, y, sc); };
-    PZG_TRY(smooth_post<BS>(c, V, l.b.as<float>(), l.x.as<float>(), op, sc));
   }
-  hipLaunchKernelGGL(k_prolong0<BS>, dim3(grid1(c.mg[0].nn)), dim3(TPB), 0, c.stream, c.mg[0].nn,
-                     c.d_mg_vmap.as<int32_t>(), c.d_mg_dsq.as<float>(), c.mg[0].x.as<float>(), z, sc);
-  PZG_HIP(hipGetLastError());
+  if (kup == 0) {
+    hipLaunchKernelGGL(k_prolong0<BS>, dim3(grid1(c.mg[0].nn)), dim3(TPB), 0, c.stream, c.mg[0].nn,
+                       c.d_mg_vmap.as<int32_t>(), c.d_mg_dsq.as<float>(), c.mg[0].x.as<float>(), z, sc);
+    PZG_HIP(hipGetLastError());
+  }
   PZG_TRY(smooth_post<BS>(c, L0, r, z, op_0, sc));
   // the learned path leaves the penalty rows to the FP64 refinement
   if ((p || q) && c.mg_les) PZG_TRY(pen_zero32(c, z));
