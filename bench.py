@@ -451,7 +451,15 @@ def main():
     mf_used = args.inner_op != "bsr" and mf_ok
     # the counter summary covers the default workload only
     counted = args.config == "C5" and not args.n and args.seed == 0
-    if mf_used:
+    # lattices of p = 2 boxes (every 3-D elasticity workload here): sum
+    # factorisation in tiles, bound by memory and not by arithmetic
+    tiled = mf_used and pb.dim == 3 and pb.p == 2 and pb.nstate == 3 and pb.el_porder is None and not pb.simplex
+    if tiled:
+        roofline = {"bound": "hbm", "kernel": "k_mft_tile<0> + k_mft_halo<0> (matrix-free FP32 operator)",
+                    "achieved": mf_gbs, "peak": 8000.0, "unit": "GB/s", "frac": mf_gbs / 8000.0,
+                    "launch_ms": mf_ms, "flops_per_launch": el_flops,
+                    "traffic": traffic_of("k_mft_tile<0>") if counted else None}
+    elif mf_used:
         kname = (f"k_mf_hex27_mfma<{sizes['bs']}>" if pb.dim == 3 and pb.p == 2
                  else "k_mf_vol") + " (matrix-free FP32 element operator)"
         tf = el_flops / (el_ms * 1e-3) / 1e12

@@ -332,8 +332,10 @@ int pzg_true_residual_noalloc(pzg_ctx *ctx, double *rel);
  * of the SpMV kernel of the given format: 0 = FP64 full CSR (plain PCG path),
  * 1 = FP32 block CSR of the mixed path, 2 = element assembly (whole pass),
  * 3 = matrix-free FP32 operator (element, boundary and row-sum kernels),
- * 4 = its volume element kernel alone, for which *bytes receives the
- * algorithmic flops of one launch instead of bytes. */
+ * 4 = its volume element kernel alone (on lattices of p = 2 boxes, where
+ * element work and row sums are one kernel, the operator without the scaling
+ * of its input), for which *bytes receives the algorithmic flops of one launch
+ * instead of bytes. */
 int pzg_time_kernel(pzg_ctx *ctx, int32_t which, int32_t nrep, double *avg_ms, double *bytes);
 
 /* No counterpart in the reference (measurement): the choices of the

@@ -60,7 +60,7 @@ static void free_all(Ctx &c) {
                     &c.d_fa, &c.d_bsr, &c.d_dinvsqrt, &c.d_bjinv, &c.d_xyz, &c.d_vnodes,
                     &c.d_vconn, &c.d_vcoef, &c.d_bnodes, &c.d_bconn, &c.d_bcid, &c.d_bctype,
                     &c.d_bcval, &c.d_bccoef, &c.d_bcvec, &c.d_aidx, &c.d_bumps, &c.d_vmap, &c.d_bmap, &c.d_tvol,
-                    &c.d_tbc, &c.d_vcolor_list, &c.d_vol_R, &c.d_blk_iptr, &c.d_blk_inc, &c.d_blk_kref, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab, &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_vbj_pos, &c.d_vbj_m, &c.d_vbj_off, &c.d_vbj_eqb, &c.d_vbjinv64, &c.d_vbjinv32, &c.d_bcolor_list, &c.d_x, &c.d_r, &c.d_z,
+                    &c.d_tbc, &c.d_vcolor_list, &c.d_vol_R, &c.d_blk_iptr, &c.d_blk_inc, &c.d_blk_kref, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab, &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_mt_cmap, &c.d_mt_tmap, &c.d_mt_part, &c.d_mt_coef, &c.d_mt_hfine, &c.d_mt_hblk, &c.d_mt_pt2, &c.d_vbj_pos, &c.d_vbj_m, &c.d_vbj_off, &c.d_vbj_eqb, &c.d_vbjinv64, &c.d_vbjinv32, &c.d_bcolor_list, &c.d_x, &c.d_r, &c.d_z,
                     &c.d_p, &c.d_p2, &c.d_q, &c.d_u, &c.d_f, &c.d_w, &c.d_xs, &c.d_rs,
                     &c.d_zs, &c.d_ps, &c.d_ps2, &c.d_qs, &c.d_bs, &c.d_scal, &c.d_partials,
                     &c.d_counter, &c.d_res2, &c.d_les_th, &c.d_les_m, &c.d_les_v, &c.d_les_g,
@@ -1784,12 +1784,19 @@ int pzg_time_kernel(pzg_ctx *ctx, int32_t which, int32_t nrep, double *avg_ms, d
     const int64_t nsh = c.tvol.nsh;
     b = (double)c.nvol * (nsh * 8.0 + c.vol_ncorner * 12.0 + 40.0 + 4.0) +
         2.0 * c.mf_nout * c.nstate * 4.0 + (double)(c.nb + 1) * 8.0 + 7.0 * n * 4.0;
+    if (c.mf_tile) {
+      // tiles: node map, coefficients, the shared nodes' partial sums written and
+      // read, their lists; vectors p read, D^-1/2 twice, pt written and read, q written
+      const double nt = (double)c.mt_nt[0] * c.mt_nt[1] * c.mt_nt[2], box = 729. * nt;
+      b = box * 4.0 + 64. * nt * 4.0 + 2.0 * (box - (double)(c.nb - c.mt_nh)) * 12.0 + c.mt_nh * 8.0 + 6.0 * n * 4.0;
+    }
   } else if (which == 4) {
     if (!mf_available(c)) {
       set_error("pzg_time_kernel: matrix-free operator needs a mesh-built system");
       return PZG_ESTATE;
     }
     PZG_TRY(mf_prepare(c));
+    PZG_TRY(dev_alloc(c.d_qs, n * sizeof(float)));
     PZG_TRY(mf_launch_vol(c, nullptr));
     PZG_HIP(hipEventRecord(c.ev0, c.stream));
     for (int i = 0; i < nrep; i++) PZG_TRY(mf_launch_vol(c, nullptr));
@@ -1800,6 +1807,9 @@ int pzg_time_kernel(pzg_ctx *ctx, int32_t which, int32_t nrep, double *avg_ms, d
     const double nq = c.tvol.nq, nsh = c.tvol.nsh, dim = c.dim, ns = c.nstate;
     const double law = ns == 3 ? 24.0 : 3.0;
     b = (double)c.nvol * (2.0 * (2.0 * nq * nsh * dim * ns) + nq * (2.0 * (2.0 * ns * dim * dim) + law));
+    // tiles: per component 54 lines of 4, the 27 modes times their diagonal (27) and
+    // 48 multiply-adds with the other components (96), the coefficient (27)
+    if (c.mf_tile) b = (double)c.nvol * 3.0 * (54. * 4. + 27. + 96. + 27.);
   } else if (which == 2) {
     if (c.external_csr) {
       set_error("pzg_time_kernel: no mesh to assemble");

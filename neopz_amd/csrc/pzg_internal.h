@@ -329,6 +329,13 @@ struct Ctx {
   int64_t mf_nbcd = 0;     // Dirichlet boundary elements
   DevBuf d_mf_blk, d_mf_xe, d_mf_bblk, d_mf_bm, d_mf_ptr, d_mf_pos, d_mf_bpos, d_mf_tab, d_mf_ye;
   int64_t mf_nout = 0;     // element contributions (entries of the row lists)
+  // lattice of identical boxes (k_mft_tile): J^-1 diagonal and |det J|, cells,
+  // tiles and fine nodes per direction, shared nodes
+  bool mf_tile = false;
+  double mf_box_inv[3] = {0, 0, 0}, mf_box_det = 0.;
+  int mt_n[3] = {0, 0, 0}, mt_nt[3] = {0, 0, 0}, mt_fn[3] = {0, 0, 0};
+  int64_t mt_nh = 0;
+  DevBuf d_mt_cmap, d_mt_tmap, d_mt_part, d_mt_coef, d_mt_hfine, d_mt_hblk, d_mt_pt2;
   int mf_resident = 0;     // workgroups of the element kernel resident at once
   DevBuf d_mf_coef, d_mf_dis, d_mf_mfma, d_mf_geo, d_mf_pt;
 
@@ -487,6 +494,22 @@ int mf_scale(Ctx &c, const float *p, const SolveScalars *sc);
 // q = S p; scaled_ready: pt already holds D^-1/2 p (fused into the p update)
 int mf_apply(Ctx &c, const float *p, const float *r, float *q, const SolveScalars *sc,
              double *partials, int *gather_grid, bool scaled_ready = false);
+// Rows of the tiled operator (c.mf_tile), v = S p with D^-1/2 p in pin (d_mf_pt
+// when null), finished in the same pass: MF_OUT_Q t = v, with partials p.v and p.r
+// (slots 0 and 1); MF_OUT_RES rout = rin - v; MF_OUT_CHEB that and the Chebyshev
+// step with the diagonal blocks: d' = c1 d + c2 minv (rin - v), x += d' and, with
+// pt, d = d', pt = D^-1/2 d'.  rout may be null with MF_OUT_CHEB; d is not read
+// when c1 = 0; pt is not pin (rows read pin while others are finished).
+enum { MF_OUT_Q = 0, MF_OUT_RES = 1, MF_OUT_CHEB = 2 };
+struct MfOut {
+  int mode = 0;
+  float c1 = 0.f, c2 = 0.f;
+  const float *pin = nullptr;
+  const float *dis = nullptr, *p = nullptr, *r = nullptr, *rin = nullptr, *minv = nullptr;
+  float *t = nullptr, *rout = nullptr, *d = nullptr, *x = nullptr, *pt = nullptr;
+  double *partials = nullptr;
+};
+int mf_apply_out(Ctx &c, const MfOut &o, const SolveScalars *sc);
 // the matrix-free operator reproduces the assembled K (mesh-built, no AddKel extras)
 inline bool mf_available(const Ctx &c) {
   return c.has_mesh && c.has_struct && !c.external_csr && !c.kel_added && c.assembled && !c.has_dep &&
@@ -502,6 +525,8 @@ inline bool mf_available(const Ctx &c) {
 enum { KF_AXPBY = 0, KF_DOT = 1, KF_RESIDUAL = 2 };
 constexpr int64_t KF_SPLIT_TILES = 4096;  // fewer element tiles of 16: three wavefronts per tile
 bool kf_usable(const Ctx &c);
+bool kf_usable_mesh(const Ctx &c);  // its mesh part: faces and blocks by row can be listed
+int kf_setup_mesh(Ctx &c);
 int kf_prepare(Ctx &c, bool *ok);
 int kf_rows_grid(const Ctx &c);
 int kf_apply(Ctx &c, int mode, const double *x, const double *f, double alpha, double beta, double *out,

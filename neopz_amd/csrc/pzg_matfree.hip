@@ -19,7 +19,8 @@
 //             element matrices depend on geometry only and are stored.
 // Element outputs go to a per-(element, shape) buffer; a second kernel sums
 // them per block row in a fixed order (no atomics: the result is
-// deterministic) and fuses the dot products of the flexible CG step.
+// deterministic) and fuses the dot products of the flexible CG step.  Lattices
+// of identical p = 2 elasticity boxes take tiles instead (k_mft_tile).
 //
 // The operator is an FP32 approximation of S of the same order as the stored
 // FP32 block CSR; the FP64 true residual of the refinement loop (CSR, FP64)
@@ -481,6 +482,391 @@ __global__ __launch_bounds__(MFK_TPB) void k_mf_hex27_mfma(MfArgs a, const MfMfm
   }
 }
 
+// ---- elasticity on a lattice of identical boxes, p = 2 ----------------------
+// The whole product (element matrices, row sums, Dirichlet faces and what the
+// caller does with a row) in two launches, for lattices of identical
+// axis-aligned hexahedra: k_mft_tile takes tiles of 4^3 cells, k_mft_halo the nodes
+// that tiles share.
+//
+// Elements: four lanes each, one component per lane and one idle, in Legendre
+// modes (box_element): about 370 operations per component against the 9,720
+// multiply-adds of the dense contractions on the matrix cores
+// (k_mf_hex27_mfma, which stays for every other p = 2 hexahedral mesh).  Lane k
+// runs its element with the axes rotated by k (axis 0 = direction k), so the
+// components differ in the addresses they read, not in the code, and exchange
+// modes by quad permutes.  Error against FP64 at random vectors, 12^3 and 16^3
+// cells: 1.40e-7 and 1.20e-7, the dense contractions 1.37e-7 and 1.38e-7.
+//
+// Memory: the tile's 9^3 nodes are staged in LDS once (the element-major gathers
+// read every node up to 8 times from memory, in 12-byte pieces that the address
+// units and not the arithmetic bound), element outputs are summed per node there
+// in a fixed order; nodes inside the tile are finished by the same kernel, the
+// others leave as partial sums that the halo kernel adds in tile order.
+//
+// Bound by LDS and memory latency at four wavefronts per SIMD (128 registers; 96
+// or 80 spill: 95 and 141 us).  Operator with its scaling pass, 64^3 / 48^3 / 24^3
+// / 12^3 / 4^3 cells: 75.6 / 41.8 / 17.2 / 15.3 / 13.4 us; element-major kernels
+// 197.5 / 87.3 / 25.2 / 22.5 / 19.8 us: faster from one tile up, so the rule is
+// the mesh alone.
+//
+// Grids: four workgroups per CU (what the registers hold; with three, 64^3 and
+// 48^3 cells took 115 and 60 us instead of 110 and 54, in an earlier form of the
+// kernel); the partial sums of both
+// kernels together fill at most MAXBLK slots.
+constexpr int MT_TILE_GRID = 1024, MT_HALO_GRID = 1024;
+constexpr int MT_TC = 4, MT_BN = 9, MT_NB = MT_BN * MT_BN * MT_BN, MT_W = 8;
+static_assert(MT_TILE_GRID + MT_HALO_GRID <= MAXBLK, "partial-sum slots");
+
+// side of the hexahedron that owns the function (kx, ky, kz), k = 0, 1: linear,
+// 2: bubble, at kx + 3 ky + 9 kz (Topology/tpzcube.h side order)
+constexpr int8_t MT_SIDE[27] = {0, 1, 8, 3, 2, 10, 11, 9, 20, 4, 5, 16, 7, 6, 18, 19, 17, 25,
+                                           12, 13, 21, 15, 14, 23, 24, 22, 26};
+
+struct MtArgs {
+  int nt[3], fn[3];
+  const int32_t *tmap;   // per tile and box node: block (-1 outside the lattice)
+  const float *tcoef;    // per tile and cell: coefficient (0: no element)
+  float *part;           // per tile and box node: partial sums of the shared nodes
+  const float *pt;       // input D^-1/2 p
+  int64_t nh;            // shared nodes: fine lattice index and block
+  const int32_t *hfine, *hblk;
+  const int32_t *pidx, *pptr, *psrc, *bblk;  // Dirichlet faces by block row
+  const float *bm;
+  // rows by component k, in rotated order: diagonal stress a[k][j] of the
+  // derivatives of k, k+1, k+2 along their own axes; mixed b1[k][j] of k along
+  // axis k+j, b2[k][j] of component k+j along axis k (j = 1, 2)
+  float a[3][3], b1[3][3], b2[3][3];
+};
+
+// what becomes of a row v = (S p)_i (MfOut::mode)
+template <int MODE>
+__device__ inline void mt_out(const MfOut &o, int64_t B, const float (&acc)[3], double &s0, double &s1) {
+  float v[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) v[k] = acc[k] * o.dis[B * 3 + k];
+  if (MODE == MF_OUT_Q) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const int64_t i = B * 3 + k;
+      o.t[i] = v[k];
+      if (o.partials) {
+        const float p = o.p[i];
+        s0 += (double)v[k] * p;
+        s1 += (double)p * o.r[i];
+      }
+    }
+    return;
+  }
+  float rv[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    rv[k] = o.rin[B * 3 + k] - v[k];
+    if (o.rout) o.rout[B * 3 + k] = rv[k];
+  }
+  if (MODE == MF_OUT_CHEB) {
+    float y[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      y[k] = o.minv[B * 9 + 3 * k] * rv[0] + o.minv[B * 9 + 3 * k + 1] * rv[1] + o.minv[B * 9 + 3 * k + 2] * rv[2];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const int64_t i = B * 3 + k;
+      const float dv = o.c1 != 0.f ? o.c1 * o.d[i] + o.c2 * y[k] : o.c2 * y[k];
+      o.x[i] += dv;
+      if (o.pt) {
+        o.d[i] = dv;
+        o.pt[i] = dv * o.dis[i];
+      }
+    }
+  }
+}
+
+// One component of S_e u on a box in Legendre modes.  c: the 27 values of the
+// lane's component in its rotated axes, index i + 3 j + 9 l by function (0, 1:
+// the ends, 2: the bubble); replaced by the element's output.
+//
+// Along an axis u0 (1-x)/2 + u1 (1+x)/2 + u2 (1-x^2) = (u0 + u1 + 4/3 u2)/2 P0 +
+// (u1 - u0)/2 P1 - 2/3 u2 P2.  In the modes (u0 + u1 + 4/3 u2, u1 - u0, u2) the
+// integrals that the 3-point rule takes exactly are: f g diagonal (BM), f' g'
+// diagonal (BE), f' g from mode n to n + 1 (BX).  So a component acts on itself
+// by a diagonal and on another one by 24 entries; nothing is evaluated at points.
+constexpr float BM[3] = {1.f / 2, 1.f / 6, 8.f / 45}, BE[3] = {0.f, 1.f / 2, 8.f / 3}, BX[2] = {1.f / 2, -2.f / 3};
+struct BoxCoef {
+  float a0, a1, a2, b11, b12, b21, b22;
+};
+__device__ inline void box_element(float (&c)[27], const BoxCoef &g) {
+#pragma unroll
+  for (int st = 1; st < 27; st *= 3)
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+      const int t = q % st + q / st * (3 * st);
+      const float u0 = c[t], u1 = c[t + st];
+      c[t] = fmaf(4.f / 3, c[t + 2 * st], u0 + u1);
+      c[t + st] = u1 - u0;
+    }
+  float y[27];
+#pragma unroll
+  for (int t = 0; t < 27; t++) {
+    const int i = t % 3, j = t / 3 % 3, l = t / 9;
+    y[t] = fmaf(g.a0, BE[i] * BM[j] * BM[l], fmaf(g.b11, BM[i] * BE[j] * BM[l], g.b12 * (BM[i] * BM[j] * BE[l]))) * c[t];
+  }
+  // component k + 1 (quad permute 0xC9; its axes (k+1, k+2, k)), then k + 2
+  // (0xD2; (k+2, k, k+1))
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int l = 0; l < 3; l++) {
+        const float f = BX[i] * BX[j] * BM[l];
+        const int t1 = i + 1 + 3 * j + 9 * l, t2 = i + 3 * (j + 1) + 9 * l;
+        y[t1] = fmaf(g.a1 * f, dpp_move<0xC9>(c[(j + 1) + 3 * l + 9 * i]), y[t1]);
+        y[t2] = fmaf(g.b21 * f, dpp_move<0xC9>(c[j + 3 * l + 9 * (i + 1)]), y[t2]);
+        const int t3 = i + 1 + 3 * l + 9 * j, t4 = i + 3 * l + 9 * (j + 1);
+        y[t3] = fmaf(g.a2 * f, dpp_move<0xD2>(c[(j + 1) + 3 * i + 9 * l]), y[t3]);
+        y[t4] = fmaf(g.b22 * f, dpp_move<0xD2>(c[j + 3 * (i + 1) + 9 * l]), y[t4]);
+      }
+#pragma unroll
+  for (int st = 1; st < 27; st *= 3)
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+      const int t = q % st + q / st * (3 * st);
+      const float y0 = y[t], y1 = y[t + st];
+      y[t] = y0 - y1;
+      y[t + st] = y0 + y1;
+      y[t + 2 * st] = fmaf(4.f / 3, y0, y[t + 2 * st]);
+    }
+#pragma unroll
+  for (int t = 0; t < 27; t++) c[t] = y[t];
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256, 4) void k_mft_tile(MtArgs g, MfOut o, const SolveScalars *sc) {
+  if (sc && sc->done) return;
+  // staged input (9^3 x 3) and element outputs (64 x 81) share the array: the
+  // inputs are in registers before the outputs are written
+  __shared__ float sh[64 * 81];
+  const int tid = threadIdx.x, el = tid >> 2, kl = tid & 3, k = kl < 3 ? kl : 0;
+  const int cx = el & 3, cy = (el >> 2) & 3, cz = el >> 4;
+  // strides of the rotated axes in the staged box and in an element's outputs
+  const int st[3] = {3, 3 * MT_BN, 3 * MT_BN * MT_BN}, so[3] = {3, 9, 27};
+  int s0 = k == 0 ? st[0] : k == 1 ? st[1] : st[2], s1 = k == 0 ? st[1] : k == 1 ? st[2] : st[0],
+            s2 = k == 0 ? st[2] : k == 1 ? st[0] : st[1];
+  int q0 = k == 0 ? so[0] : k == 1 ? so[1] : so[2], q1 = k == 0 ? so[1] : k == 1 ? so[2] : so[0],
+            q2 = k == 0 ? so[2] : k == 1 ? so[0] : so[1];
+  const int base = 3 * (2 * cx + MT_BN * (2 * cy + MT_BN * 2 * cz)) + k;
+  BoxCoef bc = {g.a[k][0], g.a[k][1], g.a[k][2], g.b1[k][1], g.b1[k][2], g.b2[k][1], g.b2[k][2]};
+  // node offset of function index 0, 1 (ends), 2 (bubble)
+  constexpr int NO[3] = {0, 2, 1};
+  double dot0 = 0., dot1 = 0.;
+  int64_t lo, hi;
+  int xi, xg;
+  xcd_slab((int64_t)g.nt[0] * g.nt[1] * g.nt[2], lo, hi, xi, xg);
+  int32_t mn[3];
+  auto load_map = [&](int64_t tile) {
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int q = tid + 256 * j;
+      mn[j] = g.tmap[(tile < hi ? tile : lo) * MT_NB + (q < MT_NB ? q : 0)];
+    }
+  };
+  if (lo + xi < hi) load_map(lo + xi);
+  for (int64_t tile = lo + xi; tile < hi; tile += xg) {
+    int32_t m[3];
+    float v[3][3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      m[j] = tid + 256 * j < MT_NB ? mn[j] : -1;
+#pragma unroll
+      for (int c = 0; c < 3; c++) v[j][c] = g.pt[(int64_t)(m[j] >= 0 ? m[j] : 0) * 3 + c];
+    }
+    const float cf = g.tcoef[tile * 64 + el];
+    load_map(tile + xg);  // a tile ahead
+    __syncthreads();      // the previous tile's sums are read
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int q = tid + 256 * j;
+      if (q < MT_NB)
+#pragma unroll
+        for (int c = 0; c < 3; c++) sh[3 * q + c] = m[j] >= 0 ? v[j][c] : 0.f;
+    }
+    __syncthreads();
+    // not invariants of the loop over tiles: their 63 products and 54 addresses
+    // would be kept, and spilled, across it
+    asm volatile("" : "+v"(bc.a0), "+v"(bc.a1), "+v"(bc.a2), "+v"(bc.b11), "+v"(bc.b12), "+v"(bc.b21), "+v"(bc.b22));
+    asm volatile("" : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(q0), "+v"(q1), "+v"(q2));
+    float u[27];
+#pragma unroll
+    for (int t = 0; t < 27; t++) u[t] = sh[base + NO[t % 3] * s0 + NO[t / 3 % 3] * s1 + NO[t / 9] * s2];
+    box_element(u, bc);
+    __syncthreads();  // every input is in registers: the outputs take its place
+    if (kl < 3)
+#pragma unroll
+      for (int t = 0; t < 27; t++)
+        sh[el * 81 + k + NO[t % 3] * q0 + NO[t / 3 % 3] * q1 + NO[t / 9] * q2] = cf * u[t];
+    __syncthreads();
+    // per box node the sum over the tile's elements that hold it (z, y, x order)
+    const int tx = (int)(tile % g.nt[0]), ty = (int)(tile / g.nt[0] % g.nt[1]),
+              tz = (int)(tile / ((int64_t)g.nt[0] * g.nt[1]));
+    int tq = tid;
+    asm volatile("" : "+v"(tq));  // (as above: 24 addresses)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int q = tq + 256 * j;
+      if (q >= MT_NB || m[j] < 0) continue;
+      const int b0 = q % MT_BN, b1 = q / MT_BN % MT_BN, b2 = q / (MT_BN * MT_BN);
+      float acc[3] = {0.f, 0.f, 0.f};
+      // cells of an even node: b/2 - 1 (its local node 2) and b/2 (0); of an odd
+      // one: (b - 1)/2 (1); cells outside the tile are masked
+#pragma unroll
+      for (int z = 0; z < 2; z++)
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+          for (int x = 0; x < 2; x++) {
+            const int ex = (b0 >> 1) - 1 + x + (b0 & 1), ey = (b1 >> 1) - 1 + y + (b1 & 1), ez = (b2 >> 1) - 1 + z + (b2 & 1);
+            const bool on = !((x & b0) | (y & b1) | (z & b2)) && ex >= 0 && ex < 4 && ey >= 0 && ey < 4 && ez >= 0 &&
+                            ez < 4;
+            const int at = on ? (ex + 4 * (ey + 4 * ez)) * 81 + 3 * ((b0 - 2 * ex) + 3 * ((b1 - 2 * ey) + 3 * (b2 - 2 * ez)))
+                              : 0;
+#pragma unroll
+            for (int c = 0; c < 3; c++) acc[c] += on ? sh[at + c] : 0.f;
+          }
+      const bool inner = b0 > 0 && b0 < MT_W && b1 > 0 && b1 < MT_W && b2 > 0 && b2 < MT_W &&
+                         MT_W * tx + b0 < g.fn[0] - 1 && MT_W * ty + b1 < g.fn[1] - 1 && MT_W * tz + b2 < g.fn[2] - 1;
+      if (inner) {
+        mt_out<MODE>(o, m[j], acc, dot0, dot1);
+      } else {
+        float *pp = g.part + (tile * MT_NB + q) * 3;
+#pragma unroll
+        for (int c = 0; c < 3; c++) pp[c] = acc[c];
+      }
+    }
+  }
+  if (MODE == MF_OUT_Q && o.partials) {
+    double vv[2] = {dot0, dot1};
+    block_partials<2>(vv, o.partials);
+  }
+}
+
+// nodes shared by tiles and nodes of the lattice boundary: the tiles' partial
+// sums in tile order, the Dirichlet faces, then the row's output
+template <int MODE>
+__global__ __launch_bounds__(256) void k_mft_halo(MtArgs g, MfOut o, int part0, const SolveScalars *sc) {
+  if (sc && sc->done) return;
+  double dot0 = 0., dot1 = 0.;
+  for (int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; h < g.nh; h += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t f = g.hfine[h];
+    const int64_t B = g.hblk[h];
+    const int fc[3] = {f % g.fn[0], f / g.fn[0] % g.fn[1], f / (g.fn[0] * g.fn[1])};
+    const int32_t pr = g.pidx ? g.pidx[B] : -1;
+    float pv[8][3];
+    bool on[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      int t[3], q[3];
+      bool ok = true;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        // tiles of the node along d: the one it lies in (or ends), and before it
+        // the one it starts after when it lies on a tile face
+        const int t1 = min(fc[d] / MT_W, g.nt[d] - 1), two = fc[d] % MT_W == 0 && fc[d] > 0 && fc[d] / MT_W <= g.nt[d] - 1;
+        const int s = (u >> d) & 1;
+        ok &= s == 1 || two;
+        t[d] = s ? t1 : t1 - 1;
+        q[d] = fc[d] - MT_W * t[d];
+      }
+      on[u] = ok;
+      const int64_t at = ok ? ((((int64_t)t[2] * g.nt[1] + t[1]) * g.nt[0] + t[0]) * MT_NB +
+                               (q[0] + MT_BN * (q[1] + MT_BN * q[2]))) * 3
+                            : 0;
+#pragma unroll
+      for (int c = 0; c < 3; c++) pv[u][c] = g.part[at + c];
+    }
+    float acc[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) acc[c] += on[u] ? pv[u][c] : 0.f;
+    if (pr >= 0)
+      for (int32_t s = g.pptr[pr]; s < g.pptr[pr + 1]; s++) {
+        const int32_t slot = g.psrc[s];
+        const float *mr = g.bm + (int64_t)slot * 9;
+        const int32_t *bj = g.bblk + slot / 9 * 9;
+        float e[3] = {0.f, 0.f, 0.f};
+        for (int j = 0; j < 9; j++)
+#pragma unroll
+          for (int c = 0; c < 3; c++) e[c] += mr[j] * g.pt[(int64_t)bj[j] * 3 + c];
+#pragma unroll
+        for (int c = 0; c < 3; c++) acc[c] += e[c];
+      }
+    mt_out<MODE>(o, B, acc, dot0, dot1);
+  }
+  if (MODE == MF_OUT_Q && o.partials) {
+    double vv[2] = {dot0, dot1};
+    block_partials<2>(vv, o.partials + part0);
+  }
+}
+
+// ---- set-up of the tiles (device; once per mesh)
+__global__ void k_mft_fill(int64_t n, int32_t v, int32_t *__restrict__ x) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) x[t] = v;
+}
+// cell and fine nodes of every element; *bad when they do not form one lattice
+__global__ void k_mft_cells(int64_t nvol, const double *__restrict__ xyz, const int64_t *__restrict__ nodes, double x0,
+                            double x1, double x2, double i0, double i1, double i2, int n0, int n1, int n2,
+                            const int32_t *__restrict__ blk, int32_t *__restrict__ cmap, int32_t *__restrict__ fmap,
+                            int *bad) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nvol) return;
+  const double *x = xyz + 3 * nodes[e * 8];
+  const double r[3] = {(x[0] - x0) * i0, (x[1] - x1) * i1, (x[2] - x2) * i2};
+  const int n[3] = {n0, n1, n2};
+  int c[3];
+  for (int d = 0; d < 3; d++) {
+    c[d] = (int)rint(r[d]);
+    if (!(fabs(r[d] - c[d]) < 1e-6) || c[d] < 0 || c[d] >= n[d]) {
+      *bad = 1;
+      return;
+    }
+  }
+  if (atomicExch(&cmap[c[0] + (int64_t)n0 * (c[1] + (int64_t)n1 * c[2])], (int32_t)e) != -1) *bad = 1;
+  const int f0 = 2 * n0 + 1, f1 = 2 * n1 + 1;
+  for (int q = 0; q < 27; q++) {  // function (kx, ky, kz): node offset 0, 2, 1
+    const int NO[3] = {0, 2, 1}, kx = q % 3, ky = q / 3 % 3, kz = q / 9;
+    const int64_t f = (2 * c[0] + NO[kx]) + (int64_t)f0 * ((2 * c[1] + NO[ky]) + (int64_t)f1 * (2 * c[2] + NO[kz]));
+    const int32_t b = blk[e * 27 + MT_SIDE[q]], was = atomicCAS(&fmap[f], -1, b);
+    if (was != -1 && was != b) *bad = 1;
+  }
+}
+__global__ void k_mft_tmap(int64_t n, int nt0, int nt1, int f0, int f1, int f2, const int32_t *__restrict__ fmap,
+                           int32_t *__restrict__ tmap) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int64_t tile = t / MT_NB;
+  const int q = (int)(t - tile * MT_NB);
+  const int fx = MT_W * (int)(tile % nt0) + q % MT_BN, fy = MT_W * (int)(tile / nt0 % nt1) + q / MT_BN % MT_BN,
+            fz = MT_W * (int)(tile / ((int64_t)nt0 * nt1)) + q / (MT_BN * MT_BN);
+  tmap[t] = fx < f0 && fy < f1 && fz < f2 ? fmap[fx + (int64_t)f0 * (fy + (int64_t)f1 * fz)] : -1;
+}
+__global__ void k_mft_hblk(int64_t n, const int32_t *__restrict__ hfine, const int32_t *__restrict__ fmap,
+                           int32_t *__restrict__ hblk) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) hblk[t] = fmap[hfine[t]];
+}
+// per assembly: the coefficients in tile order
+__global__ void k_mft_coef(int64_t n, int nt0, int nt1, int n0, int n1, int n2, const int32_t *__restrict__ cmap,
+                           const float *__restrict__ coef, float *__restrict__ tcoef) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int64_t tile = t / 64;
+  const int c = (int)(t % 64);
+  const int x = MT_TC * (int)(tile % nt0) + (c & 3), y = MT_TC * (int)(tile / nt0 % nt1) + (c >> 2 & 3),
+            z = MT_TC * (int)(tile / ((int64_t)nt0 * nt1)) + (c >> 4);
+  tcoef[t] = x < n0 && y < n1 && z < n2 ? coef[cmap[x + (int64_t)n0 * (y + (int64_t)n1 * z)]] : 0.f;
+}
+
 // Dirichlet boundary elements: y_i,k = big * sum_j M_ij u_j,k with the stored
 // FP32 matrices big*M; one thread per (element, shape).
 template <int NSHB, int NS>
@@ -620,6 +1006,173 @@ int launch_vol_lpe(Ctx &c, const MfArgs &a, const SolveScalars *sc) {
 }
 
 }  // namespace
+
+// Tiles of a lattice of identical axis-aligned p = 2 boxes (k_mft_tile); leaves
+// c.mf_tile false on any other mesh.
+static int mft_setup(Ctx &c) {
+  if (!(c.blk_asm && c.aff_on && c.blk_full && c.dim == 3 && c.nstate == 3 && c.tvol.nsh == 27 && c.tvol.nq == 27 &&
+        c.nvol > 0 && kf_usable_mesh(c)))
+    return PZG_OK;
+  const double *p0 = &c.xyz[3 * c.vol_nodes[0]];
+  static const int axis_corner[3] = {1, 3, 4};
+  double h[3], lo[3], hi[3];
+  for (int j = 0; j < 3; j++) {
+    const double *x = &c.xyz[3 * c.vol_nodes[axis_corner[j]]];
+    h[j] = x[j] - p0[j];
+    for (int i = 0; i < 3; i++)
+      if (i != j && std::fabs(x[i] - p0[i]) > 1e-12 * std::fabs(h[j])) return PZG_OK;
+    if (!(h[j] > 0.)) return PZG_OK;
+    lo[j] = hi[j] = p0[j];
+  }
+  // the side order is the kernel's
+  for (int sd = 0; sd < 27; sd++) {
+    static const int bits[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0},
+                                   {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
+    int loc[8], kind[3];
+    const int nl = side_corner_list_pub(PZG_HEX, sd, loc);
+    for (int d = 0; d < 3; d++) {
+      bool same = true;
+      for (int q = 1; q < nl; q++) same &= bits[loc[q]][d] == bits[loc[0]][d];
+      kind[d] = same ? bits[loc[0]][d] : 2;
+    }
+    if (MT_SIDE[kind[0] + 3 * kind[1] + 9 * kind[2]] != sd) return PZG_OK;
+  }
+  for (int64_t e = 0; e < c.nvol; e++) {
+    const double *x = &c.xyz[3 * c.vol_nodes[e * 8]];
+    for (int d = 0; d < 3; d++) {
+      lo[d] = std::min(lo[d], x[d]);
+      hi[d] = std::max(hi[d], x[d]);
+    }
+  }
+  int n[3], fn[3], nt[3];
+  int64_t ncell = 1, nfine = 1, ntile = 1;
+  for (int d = 0; d < 3; d++) {
+    const double m = std::floor((hi[d] - lo[d]) / h[d] + 0.5) + 1.;
+    if (m > 1e6) return PZG_OK;
+    n[d] = (int)m;
+    fn[d] = 2 * n[d] + 1;
+    nt[d] = (n[d] + MT_TC - 1) / MT_TC;
+    ncell *= n[d];
+    nfine *= fn[d];
+    ntile *= nt[d];
+  }
+  if (ncell != c.nvol || nfine != c.nb || nfine >= ((int64_t)1 << 30) || ntile * MT_NB >= ((int64_t)1 << 31) / 3)
+    return PZG_OK;
+  // nodes that the halo kernel finishes: on tile faces or on the lattice boundary
+  std::vector<int32_t> hf;
+  for (int z = 0; z < fn[2]; z++)
+    for (int y = 0; y < fn[1]; y++) {
+      const int32_t row = (int32_t)(fn[0] * (y + (int64_t)fn[1] * z));
+      if (z % MT_W == 0 || z == fn[2] - 1 || y % MT_W == 0 || y == fn[1] - 1) {
+        for (int x = 0; x < fn[0]; x++) hf.push_back(row + x);
+      } else {
+        for (int x = 0; x < fn[0]; x += MT_W) hf.push_back(row + x);
+        if ((fn[0] - 1) % MT_W) hf.push_back(row + fn[0] - 1);
+      }
+    }
+  hipStream_t s = c.stream;
+  DevBuf cm, fm, bad;
+  int rc = dev_alloc(c.d_mt_cmap, sizeof(int32_t) * ncell);
+  if (rc == PZG_OK) rc = dev_alloc(fm, sizeof(int32_t) * nfine);
+  if (rc == PZG_OK) rc = dev_alloc(bad, sizeof(int));
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_tmap, sizeof(int32_t) * ntile * MT_NB);
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_part, sizeof(float) * ntile * MT_NB * 3);
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_pt2, sizeof(float) * c.nb * 3);
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_coef, sizeof(float) * ntile * 64);
+  if (rc == PZG_OK) rc = dev_upload(c.d_mt_hfine, hf.data(), hf.size(), s);
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_hblk, sizeof(int32_t) * hf.size());
+  int hbad = 1;
+  if (rc == PZG_OK) {
+    auto g = [](int64_t m) { return dim3((unsigned)((m + MF_TPB - 1) / MF_TPB)); };
+    const int64_t nh = (int64_t)hf.size();
+    hipLaunchKernelGGL(k_mft_fill, g(ncell), dim3(MF_TPB), 0, s, ncell, -1, c.d_mt_cmap.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_fill, g(nfine), dim3(MF_TPB), 0, s, nfine, -1, fm.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_fill, dim3(1), dim3(MF_TPB), 0, s, (int64_t)1, 0, bad.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_cells, g(c.nvol), dim3(MF_TPB), 0, s, c.nvol, c.d_xyz.as<double>(),
+                       c.d_vnodes.as<int64_t>(), lo[0], lo[1], lo[2], 1. / h[0], 1. / h[1], 1. / h[2], n[0], n[1], n[2],
+                       c.d_mf_blk.as<int32_t>(), c.d_mt_cmap.as<int32_t>(), fm.as<int32_t>(), bad.as<int>());
+    hipLaunchKernelGGL(k_mft_tmap, g(ntile * MT_NB), dim3(MF_TPB), 0, s, ntile * MT_NB, nt[0], nt[1], fn[0], fn[1],
+                       fn[2], fm.as<int32_t>(), c.d_mt_tmap.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_hblk, g(nh), dim3(MF_TPB), 0, s, nh, c.d_mt_hfine.as<int32_t>(), fm.as<int32_t>(),
+                       c.d_mt_hblk.as<int32_t>());
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+      set_error(std::string("matrix-free operator: tile set-up: ") + hipGetErrorString(e));
+      rc = PZG_EHIP;
+    }
+  }
+  dev_free(fm);
+  dev_free(bad);
+  dev_free(cm);
+  PZG_TRY(rc);
+  if (hbad) return PZG_OK;
+  c.mt_nh = (int64_t)hf.size();
+  c.mf_box_det = 1.;
+  for (int d = 0; d < 3; d++) {
+    c.mt_n[d] = n[d];
+    c.mt_nt[d] = nt[d];
+    c.mt_fn[d] = fn[d];
+    c.mf_box_inv[d] = 2. / h[d];
+    c.mf_box_det *= 0.5 * h[d];
+  }
+  c.mf_tile = true;
+  return PZG_OK;
+}
+
+// q-rows of S pt (pt in d_mf_pt) through the tiles, finished as o says; the
+// partials (MF_OUT_Q) fill mft_grid blocks
+static int mft_apply(Ctx &c, const MfOut &o, const SolveScalars *sc) {
+  MtArgs g;
+  std::memset(&g, 0, sizeof(g));
+  for (int d = 0; d < 3; d++) {
+    g.nt[d] = c.mt_nt[d];
+    g.fn[d] = c.mt_fn[d];
+  }
+  g.tmap = c.d_mt_tmap.as<int32_t>();
+  g.tcoef = c.d_mt_coef.as<float>();
+  g.part = c.d_mt_part.as<float>();
+  g.pt = o.pin ? o.pin : c.d_mf_pt.as<float>();
+  g.nh = c.mt_nh;
+  g.hfine = c.d_mt_hfine.as<int32_t>();
+  g.hblk = c.d_mt_hblk.as<int32_t>();
+  if (c.kf_nface) {
+    g.pidx = c.d_kf_pidx.as<int32_t>();
+    g.pptr = c.d_kf_pptr.as<int32_t>();
+    g.psrc = c.d_kf_psrc.as<int32_t>();
+    g.bblk = c.d_kf_bblk.as<int32_t>();
+    g.bm = c.d_mf_bm.as<float>();
+  }
+  const double C1 = 1. / (2. + 2. * c.nu), den = -1. + c.nu + 2. * c.nu * c.nu, C2 = c.nu / den, C3 = (c.nu - 1.) / den;
+  const double *iv = c.mf_box_inv, det = c.mf_box_det;
+  for (int k = 0; k < 3; k++)
+    for (int j = 0; j < 3; j++) {
+      const int m = (k + j) % 3;
+      g.a[k][j] = (float)(j == 0 ? det * C3 * iv[k] * iv[k] : -det * C2 * iv[k] * iv[m]);
+      g.b1[k][j] = (float)(det * C1 * iv[m] * iv[m]);
+      g.b2[k][j] = (float)(det * C1 * iv[k] * iv[m]);
+    }
+  const int64_t ntile = (int64_t)g.nt[0] * g.nt[1] * g.nt[2];
+  const int gt = (int)std::min<int64_t>(ntile, MT_TILE_GRID);
+  const int gh = (int)std::max<int64_t>(1, std::min<int64_t>((g.nh + 255) / 256, MT_HALO_GRID));
+#define MFT(MODE)                                                                          \
+  do {                                                                                     \
+    hipLaunchKernelGGL(k_mft_tile<MODE>, dim3(gt), dim3(256), 0, c.stream, g, o, sc);      \
+    hipLaunchKernelGGL(k_mft_halo<MODE>, dim3(gh), dim3(256), 0, c.stream, g, o, gt, sc);  \
+  } while (0)
+  if (o.mode == MF_OUT_Q) MFT(MF_OUT_Q);
+  else if (o.mode == MF_OUT_RES) MFT(MF_OUT_RES);
+  else MFT(MF_OUT_CHEB);
+#undef MFT
+  PZG_HIP(hipGetLastError());
+  return PZG_OK;
+}
+static int mft_grid(const Ctx &c) {
+  const int64_t ntile = (int64_t)c.mt_nt[0] * c.mt_nt[1] * c.mt_nt[2];
+  return (int)std::min<int64_t>(ntile, MT_TILE_GRID) +
+         (int)std::max<int64_t>(1, std::min<int64_t>((c.mt_nh + 255) / 256, MT_HALO_GRID));
+}
 
 // Geometry-dependent set-up: element block maps, corner coordinates, float
 // tables, Dirichlet boundary element matrices, row incidence lists.
@@ -791,6 +1344,8 @@ int mf_setup(Ctx &c) {
   PZG_HIP(hipStreamSynchronize(s));
   c.mf_nbcd = nbcd;
   c.mf_nout = ptr[nb];
+  c.mf_tile = false;
+  PZG_TRY(mft_setup(c));
   c.mf_ready = true;
   c.mf_vals_valid = false;
   return PZG_OK;
@@ -814,6 +1369,14 @@ int mf_prepare(Ctx &c) {
                        c.d_dinvsqrt.as<double>(), c.d_mf_dis.as<float>());
     PZG_HIP(hipGetLastError());
   }
+  if (c.mf_tile) {
+    PZG_TRY(kf_setup_mesh(c));  // the Dirichlet faces by row
+    const int64_t n = (int64_t)c.mt_nt[0] * c.mt_nt[1] * c.mt_nt[2] * 64;
+    hipLaunchKernelGGL(k_mft_coef, dim3((unsigned)((n + MF_TPB - 1) / MF_TPB)), dim3(MF_TPB), 0, c.stream, n,
+                       c.mt_nt[0], c.mt_nt[1], c.mt_n[0], c.mt_n[1], c.mt_n[2], c.d_mt_cmap.as<int32_t>(),
+                       c.d_mf_coef.as<float>(), c.d_mt_coef.as<float>());
+    PZG_HIP(hipGetLastError());
+  }
   PZG_HIP(hipStreamSynchronize(c.stream));
   c.mf_vals_valid = true;
   return PZG_OK;
@@ -832,6 +1395,12 @@ int mf_scale(Ctx &c, const float *p, const SolveScalars *sc) {
 
 // Volume element kernel only (K_e pt_e into the row lists).
 int mf_launch_vol(Ctx &c, const SolveScalars *sc) {
+  if (c.mf_tile) {  // the element work and the row sums are one kernel (and the shared nodes)
+    MfOut o;
+    o.dis = c.d_mf_dis.as<float>();
+    o.t = c.d_qs.as<float>();
+    return mft_apply(c, o, sc);
+  }
   MfArgs a;
   a.nvol = c.nvol;
   a.nq = c.tvol.nq;
@@ -898,6 +1467,17 @@ int mf_apply(Ctx &c, const float *p, const float *r, float *q, const SolveScalar
              double *partials, int *gather_grid, bool scaled_ready) {
   const float *dis = c.d_mf_dis.as<float>();
   if (!scaled_ready) PZG_TRY(mf_scale(c, p, sc));
+  if (c.mf_tile) {
+    MfOut o;
+    o.mode = MF_OUT_Q;
+    o.dis = dis;
+    o.t = q;
+    o.p = p;
+    o.r = r;
+    o.partials = partials;
+    if (gather_grid) *gather_grid = mft_grid(c);
+    return mft_apply(c, o, sc);
+  }
   PZG_TRY(mf_launch_vol(c, sc));
   const int nsh = c.tvol.nsh;
   const int64_t nbcd = c.mf_nbcd;
@@ -942,5 +1522,7 @@ int mf_apply(Ctx &c, const float *p, const float *r, float *q, const SolveScalar
   if (gather_grid) *gather_grid = grid;
   return PZG_OK;
 }
+
+int mf_apply_out(Ctx &c, const MfOut &o, const SolveScalars *sc) { return mft_apply(c, o, sc); }
 
 }  // namespace pzg

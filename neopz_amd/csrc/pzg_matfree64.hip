@@ -356,13 +356,16 @@ void launch_elem(Ctx &c, const double *x, const SolveScalars *sc) {
 
 }  // namespace
 
-// The products below stand for those of the block CSR on this system
-bool kf_usable(const Ctx &c) {
-  return c.has_mesh && c.has_struct && c.assembled && !c.external_csr && !c.kel_added && !c.has_dep && !c.filt &&
-         c.blk_asm && c.aff_on && c.blk_full && c.bc_mf_ok && c.vol_rules.size() == 1 && c.bc_rules.size() <= 1 &&
-         c.dim == 3 && c.tvol.nsh == KF_NSH && (c.nbc == 0 || (c.tbc.nsh == KF_NSHB && c.bc_ncorner == 4)) &&
-         c.bs == c.nstate && c.nvol * KF_NSH < INT32_MAX && c.nbc * KF_NSHB < INT32_MAX && c.nb < INT32_MAX;
+bool kf_usable_mesh(const Ctx &c) {
+  return c.has_mesh && c.has_struct && !c.external_csr && !c.has_dep && !c.filt && c.blk_asm && c.aff_on &&
+         c.blk_full && c.bc_mf_ok && c.vol_rules.size() == 1 && c.bc_rules.size() <= 1 && c.dim == 3 &&
+         c.tvol.nsh == KF_NSH && (c.nbc == 0 || (c.tbc.nsh == KF_NSHB && c.bc_ncorner == 4)) && c.bs == c.nstate &&
+         c.nvol * KF_NSH < INT32_MAX && c.nbc * KF_NSHB < INT32_MAX && c.nb < INT32_MAX;
 }
+int kf_setup_mesh(Ctx &c) { return kf_setup(c); }
+
+// The products below stand for those of the block CSR on this system
+bool kf_usable(const Ctx &c) { return kf_usable_mesh(c) && c.assembled && !c.kel_added; }
 
 int kf_prepare(Ctx &c, bool *ok) {
   *ok = c.kf_valid;

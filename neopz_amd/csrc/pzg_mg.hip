@@ -749,6 +749,7 @@ struct LevelView {
   float *r, *d, *t;        // work vectors
   const float *dis = nullptr;  // level 0, matrix-free: D^-1/2 and the operator's
   float *pt = nullptr;         // pre-scaled input, written with each new d
+  float *pt2 = nullptr;        // level 0, tiled operator: the second such buffer
   float *y = nullptr;          // level 0, learned smoother: M r (else the blocks m)
   Cheb ch;
 };
@@ -762,6 +763,31 @@ int smooth_les(Ctx &c, const LevelView &L, const float *b, float *x, Op op, cons
   const int64_t n = L.nb * BS;
   const int g = grid1(n);
   const bool ps = L.pt != nullptr;
+  if (L.pt2) {
+    // the residual update in the operator's own pass (at 64^3 elements 15 us a
+    // step for k_les_res and t)
+    MfOut o;
+    o.mode = MF_OUT_RES;
+    o.dis = L.dis;
+    o.rin = b;
+    o.rout = L.r;
+    if (!pre) {
+      PZG_TRY(mf_scale(c, x, sc));
+      PZG_TRY(mf_apply_out(c, o, sc));
+      o.rin = L.r;
+    } else if (L.ch.c1.empty()) {  // the restriction reads r
+      hipLaunchKernelGGL(k_les_res, dim3(g), dim3(TPB), 0, c.stream, n, 0, b, (const float *)nullptr, L.r, sc);
+    }
+    LesCheb ch{pre ? 0 : 1, 0.f, (float)L.ch.c0, L.d, x, L.pt, L.dis};
+    PZG_TRY(les_apply(c, o.rin, nullptr, sc, &ch));
+    for (size_t j = 0; j < L.ch.c1.size(); j++) {
+      PZG_TRY(mf_apply_out(c, o, sc));
+      o.rin = L.r;
+      LesCheb chj{2, (float)L.ch.c1[j], (float)L.ch.c2[j], L.d, x, L.pt, L.dis};
+      PZG_TRY(les_apply(c, L.r, nullptr, sc, &chj));
+    }
+    return pre ? op(L.d, L.t, ps) : PZG_OK;
+  }
   if (pre) {
     hipLaunchKernelGGL(k_les_res, dim3(g), dim3(TPB), 0, c.stream, n, 0, b, (const float *)nullptr, L.r, sc);
   } else {
@@ -779,6 +805,35 @@ int smooth_les(Ctx &c, const LevelView &L, const float *b, float *x, Op op, cons
   return pre ? op(L.d, L.t, ps) : PZG_OK;
 }
 
+// The Chebyshev steps in the tiled operator's own passes: with restart (x += c0 M
+// (b - S x) first) or after k_cheb_init; keep: d and pt are needed afterwards, and
+// *pin then is the buffer that holds D^-1/2 d.
+int steps_tiled(Ctx &c, const LevelView &L, const float *b, float *x, const SolveScalars *sc, bool restart,
+                const float **pin) {
+  MfOut o;
+  o.mode = MF_OUT_CHEB;
+  o.dis = L.dis;
+  o.minv = L.m;
+  o.d = L.d;
+  o.x = x;
+  o.rout = L.r;
+  float *from = L.pt, *to = L.pt2;
+  const size_t m = L.ch.c1.size();
+  for (size_t j = restart ? 0 : 1; j <= m; j++) {
+    const bool last = j == m && !pin;  // nothing after it reads r, d or pt
+    o.rin = j == 0 ? b : L.r;
+    o.rout = last ? nullptr : L.r;
+    o.c1 = j == 0 ? 0.f : (float)L.ch.c1[j - 1];
+    o.c2 = j == 0 ? L.ch.c0 : (float)L.ch.c2[j - 1];
+    o.pin = from;
+    o.pt = last ? nullptr : to;
+    PZG_TRY(mf_apply_out(c, o, sc));
+    std::swap(from, to);
+  }
+  if (pin) *pin = from;
+  return PZG_OK;
+}
+
 template <int BS, class Op>
 int smooth_pre(Ctx &c, const LevelView &L, const float *b, float *x, Op op, const SolveScalars *sc) {
   if (L.y) return smooth_les<BS>(c, L, b, x, op, sc, true);
@@ -787,6 +842,13 @@ int smooth_pre(Ctx &c, const LevelView &L, const float *b, float *x, Op op, cons
   hipLaunchKernelGGL(k_cheb_init<BS>, dim3(g), dim3(TPB), 0, c.stream, L.nb, L.m, L.sa, L.sk, b, x, L.r,
                      L.d, L.ch.c0, L.dis, L.pt, sc);
   PZG_HIP(hipGetLastError());
+  if (L.pt2) {
+    MfOut o;
+    o.dis = L.dis;
+    o.t = L.t;
+    PZG_TRY(steps_tiled(c, L, b, x, sc, false, &o.pin));
+    return mf_apply_out(c, o, sc);
+  }
   for (size_t j = 0; j < L.ch.c1.size(); j++) {
     PZG_TRY(op(L.d, L.t, ps));
     hipLaunchKernelGGL(k_cheb_step<BS>, dim3(g), dim3(TPB), 0, c.stream, L.nb, L.m, L.sa, L.sk, L.t, L.r,
@@ -801,6 +863,10 @@ int smooth_post(Ctx &c, const LevelView &L, const float *b, float *x, Op op, con
   if (L.y) return smooth_les<BS>(c, L, b, x, op, sc, false);
   const int g = grid1(L.nb);
   const bool ps = L.pt != nullptr;
+  if (L.pt2) {
+    PZG_TRY(mf_scale(c, x, sc));
+    return steps_tiled(c, L, b, x, sc, true, nullptr);
+  }
   PZG_TRY(op(x, L.t, false));
   hipLaunchKernelGGL(k_cheb_restart<BS>, dim3(g), dim3(TPB), 0, c.stream, L.nb, L.m, L.sa, L.sk, b, L.t, x,
                      L.r, L.d, L.ch.c0, L.dis, L.pt, sc);
@@ -843,6 +909,7 @@ LevelView view0(Ctx &c) {
   if (c.mg_use_mf) {
     v.dis = c.d_mf_dis.as<float>();
     v.pt = c.d_mf_pt.as<float>();
+    if (c.mf_tile) v.pt2 = c.d_mt_pt2.as<float>();
   }
   if (c.mg_les) v.y = c.d_mg_y0.as<float>();
   v.ch = cheb_coeffs(c.mg_lmax0, c.mg_range, c.mg_degree);
