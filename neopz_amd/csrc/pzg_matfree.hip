@@ -505,7 +505,7 @@ __global__ __launch_bounds__(MFK_TPB) void k_mf_hex27_mfma(MfArgs a, const MfMfm
 //
 // Bound by LDS and memory latency at four wavefronts per SIMD (128 registers; 96
 // or 80 spill: 95 and 141 us).  Operator with its scaling pass, 64^3 / 48^3 / 24^3
-// / 12^3 / 4^3 cells: 75.6 / 41.8 / 17.2 / 15.3 / 13.4 us; element-major kernels
+// / 12^3 / 4^3 cells: 71.8 / 39.8 / 17.2 / 15.3 / 13.4 us; element-major kernels
 // 197.5 / 87.3 / 25.2 / 22.5 / 19.8 us: faster from one tile up, so the rule is
 // the mesh alone.
 //
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(MFK_TPB) void k_mf_hex27_mfma(MfArgs a, const MfMfm
 // 48^3 cells took 115 and 60 us instead of 110 and 54, in an earlier form of the
 // kernel); the partial sums of both
 // kernels together fill at most MAXBLK slots.
-constexpr int MT_TILE_GRID = 1024, MT_HALO_GRID = 1024;
+constexpr int MT_TILE_GRID = 1024, MT_HALO_GRID = 1024, MT_HALO_FREE = 1 << 20;
 constexpr int MT_TC = 4, MT_BN = 9, MT_NB = MT_BN * MT_BN * MT_BN, MT_W = 8;
 static_assert(MT_TILE_GRID + MT_HALO_GRID <= MAXBLK, "partial-sum slots");
 
@@ -538,48 +538,54 @@ struct MtArgs {
   float a[3][3], b1[3][3], b2[3][3];
 };
 
-// what becomes of a row v = (S p)_i (MfOut::mode)
-template <int MODE>
-__device__ inline void mt_out(const MfOut &o, int64_t B, const float (&acc)[3], double &s0, double &s1) {
-  float v[3];
+// What becomes of a row v = (S p)_i (MfOut::mode).  load() first: its loads are
+// in flight while the row's terms are summed.
+template <int MODE> struct MtRow {
+  float dis[3], a[3], b[3], m[9];
+  __device__ void load(const MfOut &o, int64_t B) {
 #pragma unroll
-  for (int k = 0; k < 3; k++) v[k] = acc[k] * o.dis[B * 3 + k];
-  if (MODE == MF_OUT_Q) {
+    for (int k = 0; k < 3; k++) dis[k] = o.dis[B * 3 + k];
+    if (MODE != MF_OUT_Q)
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const int64_t i = B * 3 + k;
-      o.t[i] = v[k];
-      if (o.partials) {
-        const float p = o.p[i];
-        s0 += (double)v[k] * p;
-        s1 += (double)p * o.r[i];
-      }
-    }
-    return;
-  }
-  float rv[3];
+      for (int k = 0; k < 3; k++) a[k] = o.rin[B * 3 + k];
+    if (MODE == MF_OUT_CHEB) {
 #pragma unroll
-  for (int k = 0; k < 3; k++) {
-    rv[k] = o.rin[B * 3 + k] - v[k];
-    if (o.rout) o.rout[B * 3 + k] = rv[k];
-  }
-  if (MODE == MF_OUT_CHEB) {
-    float y[3];
+      for (int k = 0; k < 9; k++) m[k] = o.minv[B * 9 + k];
 #pragma unroll
-    for (int k = 0; k < 3; k++)
-      y[k] = o.minv[B * 9 + 3 * k] * rv[0] + o.minv[B * 9 + 3 * k + 1] * rv[1] + o.minv[B * 9 + 3 * k + 2] * rv[2];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const int64_t i = B * 3 + k;
-      const float dv = o.c1 != 0.f ? o.c1 * o.d[i] + o.c2 * y[k] : o.c2 * y[k];
-      o.x[i] += dv;
-      if (o.pt) {
-        o.d[i] = dv;
-        o.pt[i] = dv * o.dis[i];
-      }
+      for (int k = 0; k < 3; k++) b[k] = o.c1 != 0.f ? o.d[B * 3 + k] : 0.f;
     }
   }
-}
+  __device__ void out(const MfOut &o, int64_t B, const float (&acc)[3], double &s0, double &s1) const {
+    float rv[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const float v = acc[k] * dis[k];
+      if (MODE == MF_OUT_Q) {
+        o.t[B * 3 + k] = v;
+        if (o.partials) {
+          const float p = o.p[B * 3 + k];  // (held from load() on, they spill in k_mft_tile)
+          s0 += (double)v * p;
+          s1 += (double)p * o.r[B * 3 + k];
+        }
+      } else {
+        rv[k] = a[k] - v;
+        if (o.rout) o.rout[B * 3 + k] = rv[k];
+      }
+    }
+    if (MODE == MF_OUT_CHEB)
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const int64_t i = B * 3 + k;
+        const float y = m[3 * k] * rv[0] + m[3 * k + 1] * rv[1] + m[3 * k + 2] * rv[2];
+        const float dv = o.c1 != 0.f ? o.c1 * b[k] + o.c2 * y : o.c2 * y;
+        o.x[i] += dv;
+        if (o.pt) {
+          o.d[i] = dv;
+          o.pt[i] = dv * dis[k];
+        }
+      }
+  }
+};
 
 // One component of S_e u on a box in Legendre modes.  c: the 27 values of the
 // lane's component in its rotated axes, index i + 3 j + 9 l by function (0, 1:
@@ -715,6 +721,8 @@ __global__ __launch_bounds__(256, 4) void k_mft_tile(MtArgs g, MfOut o, const So
       const int q = tq + 256 * j;
       if (q >= MT_NB || m[j] < 0) continue;
       const int b0 = q % MT_BN, b1 = q / MT_BN % MT_BN, b2 = q / (MT_BN * MT_BN);
+      const bool inner = b0 > 0 && b0 < MT_W && b1 > 0 && b1 < MT_W && b2 > 0 && b2 < MT_W &&
+                         MT_W * tx + b0 < g.fn[0] - 1 && MT_W * ty + b1 < g.fn[1] - 1 && MT_W * tz + b2 < g.fn[2] - 1;
       float acc[3] = {0.f, 0.f, 0.f};
       // cells of an even node: b/2 - 1 (its local node 2) and b/2 (0); of an odd
       // one: (b - 1)/2 (1); cells outside the tile are masked
@@ -732,10 +740,10 @@ __global__ __launch_bounds__(256, 4) void k_mft_tile(MtArgs g, MfOut o, const So
 #pragma unroll
             for (int c = 0; c < 3; c++) acc[c] += on ? sh[at + c] : 0.f;
           }
-      const bool inner = b0 > 0 && b0 < MT_W && b1 > 0 && b1 < MT_W && b2 > 0 && b2 < MT_W &&
-                         MT_W * tx + b0 < g.fn[0] - 1 && MT_W * ty + b1 < g.fn[1] - 1 && MT_W * tz + b2 < g.fn[2] - 1;
       if (inner) {
-        mt_out<MODE>(o, m[j], acc, dot0, dot1);
+        MtRow<MODE> row;  // (loaded before the sums, for three nodes at once, it spills)
+        row.load(o, m[j]);
+        row.out(o, m[j], acc, dot0, dot1);
       } else {
         float *pp = g.part + (tile * MT_NB + q) * 3;
 #pragma unroll
@@ -750,7 +758,10 @@ __global__ __launch_bounds__(256, 4) void k_mft_tile(MtArgs g, MfOut o, const So
 }
 
 // nodes shared by tiles and nodes of the lattice boundary: the tiles' partial
-// sums in tile order, the Dirichlet faces, then the row's output
+// sums in tile order, the Dirichlet faces, then the row's output.  Bound by its
+// scattered 12-byte pieces: nodes go in the order of their blocks, so that the
+// vectors at least are read in runs, and a row's loads are issued before its sum
+// (48^3 cells, Chebyshev step: 21.1 us; in lattice order, loads last: 46.9).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_mft_halo(MtArgs g, MfOut o, int part0, const SolveScalars *sc) {
   if (sc && sc->done) return;
@@ -760,6 +771,8 @@ __global__ __launch_bounds__(256) void k_mft_halo(MtArgs g, MfOut o, int part0, 
     const int64_t B = g.hblk[h];
     const int fc[3] = {f % g.fn[0], f / g.fn[0] % g.fn[1], f / (g.fn[0] * g.fn[1])};
     const int32_t pr = g.pidx ? g.pidx[B] : -1;
+    MtRow<MODE> row;
+    row.load(o, B);
     float pv[8][3];
     bool on[8];
 #pragma unroll
@@ -800,7 +813,7 @@ __global__ __launch_bounds__(256) void k_mft_halo(MtArgs g, MfOut o, int part0, 
 #pragma unroll
         for (int c = 0; c < 3; c++) acc[c] += e[c];
       }
-    mt_out<MODE>(o, B, acc, dot0, dot1);
+    row.out(o, B, acc, dot0, dot1);
   }
   if (MODE == MF_OUT_Q && o.partials) {
     double vv[2] = {dot0, dot1};
@@ -850,10 +863,55 @@ __global__ void k_mft_tmap(int64_t n, int nt0, int nt1, int f0, int f1, int f2, 
             fz = MT_W * (int)(tile / ((int64_t)nt0 * nt1)) + q / (MT_BN * MT_BN);
   tmap[t] = fx < f0 && fy < f1 && fz < f2 ? fmap[fx + (int64_t)f0 * (fy + (int64_t)f1 * fz)] : -1;
 }
-__global__ void k_mft_hblk(int64_t n, const int32_t *__restrict__ hfine, const int32_t *__restrict__ fmap,
-                           int32_t *__restrict__ hblk) {
+// fine node of every block; *bad when a block has two
+__global__ void k_mft_inv(int64_t n, const int32_t *__restrict__ fmap, int32_t *__restrict__ bf, int *bad) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) hblk[t] = fmap[hfine[t]];
+  if (t >= n) return;
+  const int32_t b = fmap[t];
+  if (b < 0 || b >= n || atomicExch(&bf[b], (int32_t)t) != -1) *bad = 1;
+}
+// Shared nodes in the order of their blocks (rows of the vectors next to each
+// other are next to each other in the list): per workgroup of 256 blocks their
+// number (hblk null) or, from its first place first[workgroup], the list.
+__global__ __launch_bounds__(256) void k_mft_halo_list(int64_t n, int f0, int f1, int f2, const int32_t *__restrict__ bf,
+                                                       int32_t *__restrict__ first, int64_t nh,
+                                                       int32_t *__restrict__ hfine, int32_t *__restrict__ hblk) {
+  __shared__ int wc[4];
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int32_t f = t < n ? bf[t] : -1;
+  const int x = f % f0, y = f / f0 % f1, z = f / (f0 * f1);
+  const bool h = f >= 0 && (x % MT_W == 0 || x == f0 - 1 || y % MT_W == 0 || y == f1 - 1 || z % MT_W == 0 || z == f2 - 1);
+  const uint64_t mask = __ballot(h);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (lane == 0) wc[w] = __popcll(mask);
+  __syncthreads();
+  if (!hblk) {
+    if (threadIdx.x == 0) first[blockIdx.x] = wc[0] + wc[1] + wc[2] + wc[3];
+    return;
+  }
+  if (!h) return;
+  int64_t at = first[blockIdx.x] + __popcll(mask & ((1ull << lane) - 1));
+  for (int k = 0; k < w; k++) at += wc[k];
+  if (at < nh) {
+    hfine[at] = f;
+    hblk[at] = (int32_t)t;
+  }
+}
+// counts to first places, one workgroup
+__global__ __launch_bounds__(256) void k_mft_scan(int n, int32_t *__restrict__ x) {
+  __shared__ int part[256];
+  const int per = (n + 255) / 256, lo = threadIdx.x * per, hi = min(n, lo + per);
+  int s = 0;
+  for (int i = lo; i < hi; i++) s += x[i];
+  part[threadIdx.x] = s;
+  __syncthreads();
+  int at = 0;
+  for (int i = 0; i < (int)threadIdx.x; i++) at += part[i];
+  for (int i = lo; i < hi; i++) {
+    const int v = x[i];
+    x[i] = at;
+    at += v;
+  }
 }
 // per assembly: the coefficients in tile order
 __global__ void k_mft_coef(int64_t n, int nt0, int nt1, int n0, int n1, int n2, const int32_t *__restrict__ cmap,
@@ -1059,19 +1117,15 @@ static int mft_setup(Ctx &c) {
   if (ncell != c.nvol || nfine != c.nb || nfine >= ((int64_t)1 << 30) || ntile * MT_NB >= ((int64_t)1 << 31) / 3)
     return PZG_OK;
   // nodes that the halo kernel finishes: on tile faces or on the lattice boundary
-  std::vector<int32_t> hf;
-  for (int z = 0; z < fn[2]; z++)
-    for (int y = 0; y < fn[1]; y++) {
-      const int32_t row = (int32_t)(fn[0] * (y + (int64_t)fn[1] * z));
-      if (z % MT_W == 0 || z == fn[2] - 1 || y % MT_W == 0 || y == fn[1] - 1) {
-        for (int x = 0; x < fn[0]; x++) hf.push_back(row + x);
-      } else {
-        for (int x = 0; x < fn[0]; x += MT_W) hf.push_back(row + x);
-        if ((fn[0] - 1) % MT_W) hf.push_back(row + fn[0] - 1);
-      }
-    }
+  int64_t inside = 1;
+  for (int d = 0; d < 3; d++) {
+    const int faces = (fn[d] - 1) / MT_W + 1 + ((fn[d] - 1) % MT_W ? 1 : 0);
+    inside *= fn[d] - faces;
+  }
+  const int64_t nh = nfine - inside;
   hipStream_t s = c.stream;
-  DevBuf cm, fm, bad;
+  DevBuf fm, bf, first, bad;
+  const int ngrp = (int)((nfine + 255) / 256);
   int rc = dev_alloc(c.d_mt_cmap, sizeof(int32_t) * ncell);
   if (rc == PZG_OK) rc = dev_alloc(fm, sizeof(int32_t) * nfine);
   if (rc == PZG_OK) rc = dev_alloc(bad, sizeof(int));
@@ -1079,12 +1133,13 @@ static int mft_setup(Ctx &c) {
   if (rc == PZG_OK) rc = dev_alloc(c.d_mt_part, sizeof(float) * ntile * MT_NB * 3);
   if (rc == PZG_OK) rc = dev_alloc(c.d_mt_pt2, sizeof(float) * c.nb * 3);
   if (rc == PZG_OK) rc = dev_alloc(c.d_mt_coef, sizeof(float) * ntile * 64);
-  if (rc == PZG_OK) rc = dev_upload(c.d_mt_hfine, hf.data(), hf.size(), s);
-  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_hblk, sizeof(int32_t) * hf.size());
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_hfine, sizeof(int32_t) * nh);
+  if (rc == PZG_OK) rc = dev_alloc(c.d_mt_hblk, sizeof(int32_t) * nh);
+  if (rc == PZG_OK) rc = dev_alloc(bf, sizeof(int32_t) * nfine);
+  if (rc == PZG_OK) rc = dev_alloc(first, sizeof(int32_t) * ngrp);
   int hbad = 1;
   if (rc == PZG_OK) {
     auto g = [](int64_t m) { return dim3((unsigned)((m + MF_TPB - 1) / MF_TPB)); };
-    const int64_t nh = (int64_t)hf.size();
     hipLaunchKernelGGL(k_mft_fill, g(ncell), dim3(MF_TPB), 0, s, ncell, -1, c.d_mt_cmap.as<int32_t>());
     hipLaunchKernelGGL(k_mft_fill, g(nfine), dim3(MF_TPB), 0, s, nfine, -1, fm.as<int32_t>());
     hipLaunchKernelGGL(k_mft_fill, dim3(1), dim3(MF_TPB), 0, s, (int64_t)1, 0, bad.as<int32_t>());
@@ -1093,8 +1148,13 @@ static int mft_setup(Ctx &c) {
                        c.d_mf_blk.as<int32_t>(), c.d_mt_cmap.as<int32_t>(), fm.as<int32_t>(), bad.as<int>());
     hipLaunchKernelGGL(k_mft_tmap, g(ntile * MT_NB), dim3(MF_TPB), 0, s, ntile * MT_NB, nt[0], nt[1], fn[0], fn[1],
                        fn[2], fm.as<int32_t>(), c.d_mt_tmap.as<int32_t>());
-    hipLaunchKernelGGL(k_mft_hblk, g(nh), dim3(MF_TPB), 0, s, nh, c.d_mt_hfine.as<int32_t>(), fm.as<int32_t>(),
-                       c.d_mt_hblk.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_fill, g(nfine), dim3(MF_TPB), 0, s, nfine, -1, bf.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_inv, g(nfine), dim3(MF_TPB), 0, s, nfine, fm.as<int32_t>(), bf.as<int32_t>(), bad.as<int>());
+    hipLaunchKernelGGL(k_mft_halo_list, dim3((unsigned)ngrp), dim3(256), 0, s, nfine, fn[0], fn[1], fn[2], bf.as<int32_t>(),
+                       first.as<int32_t>(), nh, (int32_t *)nullptr, (int32_t *)nullptr);
+    hipLaunchKernelGGL(k_mft_scan, dim3(1), dim3(256), 0, s, ngrp, first.as<int32_t>());
+    hipLaunchKernelGGL(k_mft_halo_list, dim3((unsigned)ngrp), dim3(256), 0, s, nfine, fn[0], fn[1], fn[2], bf.as<int32_t>(),
+                       first.as<int32_t>(), nh, c.d_mt_hfine.as<int32_t>(), c.d_mt_hblk.as<int32_t>());
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1105,10 +1165,11 @@ static int mft_setup(Ctx &c) {
   }
   dev_free(fm);
   dev_free(bad);
-  dev_free(cm);
+  dev_free(bf);
+  dev_free(first);
   PZG_TRY(rc);
   if (hbad) return PZG_OK;
-  c.mt_nh = (int64_t)hf.size();
+  c.mt_nh = nh;
   c.mf_box_det = 1.;
   for (int d = 0; d < 3; d++) {
     c.mt_n[d] = n[d];
@@ -1155,7 +1216,8 @@ static int mft_apply(Ctx &c, const MfOut &o, const SolveScalars *sc) {
     }
   const int64_t ntile = (int64_t)g.nt[0] * g.nt[1] * g.nt[2];
   const int gt = (int)std::min<int64_t>(ntile, MT_TILE_GRID);
-  const int gh = (int)std::max<int64_t>(1, std::min<int64_t>((g.nh + 255) / 256, MT_HALO_GRID));
+  const int gh = (int)std::max<int64_t>(1, std::min<int64_t>((g.nh + 255) / 256,
+                                                                   o.partials ? MT_HALO_GRID : MT_HALO_FREE));
 #define MFT(MODE)                                                                          \
   do {                                                                                     \
     hipLaunchKernelGGL(k_mft_tile<MODE>, dim3(gt), dim3(256), 0, c.stream, g, o, sc);      \
