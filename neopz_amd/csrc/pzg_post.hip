@@ -4,11 +4,11 @@
 //    EvaluateError (Mesh/pzinterpolationspace.cpp:1108-1207): per volume
 //    element the weighted sum over the error rule's points of the material's
 //    Errors values, then its square root.  A group of G lanes (G = the power
-//    of two >= the rule's point count, at most 64) takes one element: the
-//    element's solution coefficients, table columns and corner coordinates
-//    go to LDS, each lane walks the points q = lane, lane + G, ... of tables
-//    stored point-fastest (coalesced loads), and the group adds its lanes'
-//    sums with cross-lane shuffles.  With POINTS = true the kernel writes the
+//    of two >= the rule's point count, at most 64) takes EB elements: their
+//    solution coefficients, table columns and corner coordinates go to LDS
+//    (sides without equations are left out), each lane walks the points q =
+//    lane, lane + G, ... of tables stored point-fastest (coalesced loads), and
+//    the group adds its lanes' sums with cross-lane shuffles.  With POINTS = true the kernel writes the
 //    physical coordinates of the points instead (the points at which a
 //    caller evaluates its exact-solution function).
 //
@@ -137,143 +137,266 @@ __device__ inline void err_values(const PostArgs &a, double coef, const double (
   }
 }
 
-template <int NS, bool POINTS>
+// g = (gradient in x, y, z) of the reference gradient gr, and |det J| (the element's
+// volume / area / length measure) (Axes2XYZ of the axes gradient); dim 3: ji[d][i]
+// = d xi_d / d x_i
+__device__ inline double jac_inverse(const double (&J)[3][3], double (&ji)[3][3]) {
+  const double det = -J[0][2] * J[1][1] * J[2][0] + J[0][1] * J[1][2] * J[2][0] + J[0][2] * J[1][0] * J[2][1] -
+                     J[0][0] * J[1][2] * J[2][1] - J[0][1] * J[1][0] * J[2][2] + J[0][0] * J[1][1] * J[2][2];
+  ji[0][0] = (-J[1][2] * J[2][1] + J[1][1] * J[2][2]) / det;
+  ji[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det;
+  ji[0][2] = (-J[0][2] * J[1][1] + J[0][1] * J[1][2]) / det;
+  ji[1][0] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) / det;
+  ji[1][1] = (-J[0][2] * J[2][0] + J[0][0] * J[2][2]) / det;
+  ji[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det;
+  ji[2][0] = (-J[1][1] * J[2][0] + J[1][0] * J[2][1]) / det;
+  ji[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det;
+  ji[2][2] = (-J[0][1] * J[1][0] + J[0][0] * J[1][1]) / det;
+  return det;
+}
+
+// EB elements per group of lanes share every table value it loads; AFF:
+// tetrahedra, whose Jacobian is the same at every point (the corner derivatives
+// are -1, 0, 1) and is inverted once per element.
+//
+// One element per group was bound by the L1: four table values for four
+// multiply-adds, over all 56 sides of an order-5 element whatever its order.
+// 82,944 tetrahedra of orders 1 to 5, 512 points each: 8.57 ms then; 2.76 ms with
+// EB = 4 (247 registers, two wavefronts per SIMD), 2.84 ms with EB = 2.  What is
+// left is arithmetic: the exact solution's sines and the multiply-adds.
+template <int NS, bool POINTS, int EB, bool AFF>
 __global__ __launch_bounds__(PTPB) void k_post(const PostArgs a) {
   extern __shared__ double s_mem[];
   const int G = a.G, ngrp = PTPB / G;
   const int gl = threadIdx.x / G, lq = threadIdx.x - gl * G;
-  const int64_t gi = (int64_t)blockIdx.x * ngrp + gl;
-  const bool live = gi < a.nlist;
-  const int64_t e = live ? a.list[gi] : 0;
-  double *s_u = s_mem + (size_t)gl * a.nslot * NS;
-  double *s_x = s_mem + (size_t)ngrp * a.nslot * NS + gl * 24;
-  int *s_col = reinterpret_cast<int *>(s_mem + (size_t)ngrp * (a.nslot * NS + 24)) + gl * a.nslot;
+  const int64_t g0 = ((int64_t)blockIdx.x * ngrp + gl) * EB;
+  const bool live = g0 < a.nlist;
+  int64_t e[EB];
+#pragma unroll
+  for (int j = 0; j < EB; j++) e[j] = live ? a.list[g0 + j < a.nlist ? g0 + j : a.nlist - 1] : 0;
+  const int gsz = a.nslot * NS * EB + (24 + (AFF ? 10 : 0)) * EB;
+  double *s_u = s_mem + (size_t)gl * gsz;  // [slot][state][element]
+  double *s_x = s_u + a.nslot * NS * EB;   // corners, then det and ji
+  double *s_j = s_x + 24 * EB;
+  int *s_col = reinterpret_cast<int *>(s_mem + (size_t)ngrp * gsz) + gl * a.nslot * EB;
+  const int nc = a.nc, dim = a.dim, nq = a.nq, ncol = a.ncol;
+  const double *W = a.tab, *PH = W + nq, *DPH = PH + (size_t)ncol * nq;
+  const double *CP = DPH + (size_t)dim * ncol * nq, *CD = CP + (size_t)nc * nq;
+  int nact = 0;  // slots with a value in one of the elements
   if (live) {
-    int64_t id[4] = {0, 0, 0, 0};
-    if (a.hp)
-      for (int k = 0; k < a.nc; k++) id[k] = a.nodes[e * a.nc + k];
-    for (int i = lq; i < a.nslot; i += G) {
-      s_col[i] = a.hp ? a.slot[i] + hp_variant(a.tet, a.slot[HP_MAXSH + i], id) : i;
-      if (!POINTS) {
-        // a constrained connect's value follows from the connects it depends
-        // on (TPZCompMesh::LoadSolution expands the solution)
-        const int64_t cc = a.conn[e * a.nsv + i], b = a.aidx[cc];
-        for (int k = 0; k < NS; k++) {
-          double v = 0.;
-          if (b >= 0) v = a.u[b * a.bs + k];
-          else if (a.dep_ptr)
-            for (int64_t d = a.dep_ptr[cc]; d < a.dep_ptr[cc + 1]; d++)
-              if (a.dep_blk[d] >= 0) v += a.dep_coef[d] * a.u[a.dep_blk[d] * a.bs + k];
-          s_u[i * NS + k] = v;
+    const int sh = threadIdx.x & 63 & ~(G - 1);
+    const uint64_t below = (1ull << lq) - 1, mine = G < 64 ? (1ull << G) - 1 : ~0ull;
+    if (!POINTS)
+      for (int i0 = 0; i0 < a.nslot; i0 += G) {
+        const int i = i0 + lq;
+        double v[EB][NS];
+        int col[EB], c0 = 0;
+        bool any = false, differ = false;
+#pragma unroll
+        for (int j = 0; j < EB; j++) {
+          col[j] = 0;
+#pragma unroll
+          for (int k = 0; k < NS; k++) v[j][k] = 0.;
+          if (i >= a.nslot) continue;
+          // a constrained connect's value follows from the connects it depends
+          // on (TPZCompMesh::LoadSolution expands the solution)
+          const int64_t cc = a.conn[e[j] * a.nsv + i], b = a.aidx[cc];
+          const bool has = b >= 0 || a.dep_ptr;
+          if (!has) continue;  // no equations: no term
+          for (int k = 0; k < NS; k++) {
+            if (b >= 0) v[j][k] = a.u[b * a.bs + k];
+            else
+              for (int64_t d = a.dep_ptr[cc]; d < a.dep_ptr[cc + 1]; d++)
+                if (a.dep_blk[d] >= 0) v[j][k] += a.dep_coef[d] * a.u[a.dep_blk[d] * a.bs + k];
+          }
+          col[j] = i;
+          if (a.hp) {
+            int64_t id[4] = {0, 0, 0, 0};
+            for (int k = 0; k < nc; k++) id[k] = a.nodes[e[j] * nc + k];
+            col[j] = a.slot[i] + hp_variant(a.tet, a.slot[HP_MAXSH + i], id);
+          }
+          if (!any) c0 = col[j];
+          else differ |= col[j] != c0;
+          any = true;
+        }
+        const uint64_t m = (__ballot(any) >> sh) & mine;
+        if (any) {
+          const int at = nact + __popcll(m & below);
+#pragma unroll
+          for (int j = 0; j < EB; j++) {
+#pragma unroll
+            for (int k = 0; k < NS; k++) s_u[(at * NS + k) * EB + j] = v[j][k];
+            // negative: the elements' columns differ
+            if (j > 0 || !differ) s_col[at * EB + j] = differ ? col[j] : c0;
+          }
+          if (differ) s_col[at * EB] = -1 - col[0];
+        }
+        nact += __popcll(m);
+      }
+#pragma unroll
+    for (int j = 0; j < EB; j++)
+      for (int k = lq; k < nc * 3; k += G) s_x[j * 24 + k] = a.xyz[3 * a.nodes[e[j] * nc + k / 3] + k % 3];
+  }
+  __syncthreads();
+  if (AFF) {
+    for (int j = lq; live && j < EB; j += G) {
+      double J[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}}, ji[3][3];
+      for (int n = 0; n < nc; n++)
+        for (int d = 0; d < 3; d++) {
+          const double cd = CD[((size_t)d * nc + n) * nq];
+          for (int i = 0; i < 3; i++) J[i][d] += cd * s_x[j * 24 + 3 * n + i];
+        }
+      s_j[j * 10] = jac_inverse(J, ji);
+      for (int d = 0; d < 3; d++)
+        for (int i = 0; i < 3; i++) s_j[j * 10 + 1 + 3 * d + i] = ji[d][i];
+    }
+    __syncthreads();
+  }
+  if (!live) return;
+
+  double acc[EB][MAXERR];
+#pragma unroll
+  for (int j = 0; j < EB; j++)
+#pragma unroll
+    for (int m = 0; m < MAXERR; m++) acc[j][m] = 0.;
+  for (int q = lq; q < nq; q += G) {
+    // discrete value and reference gradient (TPZInterpolationSpace::
+    // ComputeSolution)
+    double u[EB][NS], gr[EB][3][NS];
+#pragma unroll
+    for (int j = 0; j < EB; j++)
+#pragma unroll
+      for (int k = 0; k < NS; k++) {
+        u[j][k] = 0.;
+        for (int d = 0; d < 3; d++) gr[j][d][k] = 0.;
+      }
+    for (int i = 0; i < nact; i++) {
+      const int col = s_col[i * EB];
+      if (EB == 1 || col >= 0) {
+        const double ph = PH[(size_t)col * nq + q];
+        double dp[3] = {0., 0., 0.};
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+          if (d < dim) dp[d] = DPH[((size_t)d * ncol + col) * nq + q];
+#pragma unroll
+        for (int k = 0; k < NS; k++)
+#pragma unroll
+          for (int j = 0; j < EB; j++) {
+            const double cf = s_u[(i * NS + k) * EB + j];
+            u[j][k] += ph * cf;
+#pragma unroll
+            for (int d = 0; d < 3; d++) gr[j][d][k] += dp[d] * cf;
+          }
+      } else {
+#pragma unroll
+        for (int j = 0; j < EB; j++) {
+          const int cj = j == 0 ? -1 - col : s_col[i * EB + j];
+          const double ph = PH[(size_t)cj * nq + q];
+          double dp[3] = {0., 0., 0.};
+#pragma unroll
+          for (int d = 0; d < 3; d++)
+            if (d < dim) dp[d] = DPH[((size_t)d * ncol + cj) * nq + q];
+#pragma unroll
+          for (int k = 0; k < NS; k++) {
+            const double cf = s_u[(i * NS + k) * EB + j];
+            u[j][k] += ph * cf;
+#pragma unroll
+            for (int d = 0; d < 3; d++) gr[j][d][k] += dp[d] * cf;
+          }
         }
       }
     }
-    for (int k = lq; k < a.nc * 3; k += G) s_x[k] = a.xyz[3 * a.nodes[e * a.nc + k / 3] + k % 3];
-  }
-  __syncthreads();
-  if (!live) return;
-
-  const int nq = a.nq, dim = a.dim, nc = a.nc, ncol = a.ncol;
-  const double *W = a.tab, *PH = W + nq, *DPH = PH + (size_t)ncol * nq;
-  const double *CP = DPH + (size_t)dim * ncol * nq, *CD = CP + (size_t)nc * nq;
-  const double coef = a.coef ? a.coef[e] : (a.material == PZG_MAT_ELAST3D ? a.E : a.kconst);
-  double acc[MAXERR] = {0., 0., 0., 0., 0., 0.};
-  for (int q = lq; q < nq; q += G) {
-    // geometric map: x and J[i][j] = d x_i / d xi_j (TPZGeoEl::X / GradX)
-    double x[3] = {0., 0., 0.}, J[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
-    for (int n = 0; n < nc; n++) {
-      const double cp = CP[(size_t)n * nq + q];
-      for (int i = 0; i < 3; i++) x[i] += cp * s_x[3 * n + i];
-      for (int j = 0; j < dim; j++) {
-        const double cd = CD[((size_t)j * nc + n) * nq + q];
-        for (int i = 0; i < 3; i++) J[i][j] += cd * s_x[3 * n + i];
+#pragma unroll
+    for (int j = 0; j < EB; j++) {
+      // geometric map: x and J[i][d] = d x_i / d xi_d (TPZGeoEl::X / GradX)
+      double x[3] = {0., 0., 0.}, J[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
+      for (int n = 0; n < nc; n++) {
+        const double cp = CP[(size_t)n * nq + q];
+#pragma unroll
+        for (int i = 0; i < 3; i++) x[i] += cp * s_x[j * 24 + 3 * n + i];
+        if (!AFF)
+#pragma unroll
+          for (int d = 0; d < 3; d++)
+            if (d < dim) {
+              const double cd = CD[((size_t)d * nc + n) * nq + q];
+#pragma unroll
+              for (int i = 0; i < 3; i++) J[i][d] += cd * s_x[j * 24 + 3 * n + i];
+            }
       }
-    }
-    if constexpr (POINTS) {
-      const int64_t p = a.off[e] + q;
-      for (int i = 0; i < 3; i++) a.xq[p * 3 + i] = x[i];
-      continue;
-    }
-    // discrete value and reference gradient (TPZInterpolationSpace::
-    // ComputeSolution)
-    double u[NS], gr[3][NS];
-    for (int k = 0; k < NS; k++) {
-      u[k] = 0.;
-      for (int d = 0; d < 3; d++) gr[d][k] = 0.;
-    }
-    for (int i = 0; i < a.nslot; i++) {
-      const int col = s_col[i];
-      const double ph = PH[(size_t)col * nq + q];
-      double dp[3] = {0., 0., 0.};
-      for (int d = 0; d < dim; d++) dp[d] = DPH[((size_t)d * ncol + col) * nq + q];
-      for (int k = 0; k < NS; k++) {
-        const double cf = s_u[i * NS + k];
-        u[k] += ph * cf;
-        for (int d = 0; d < 3; d++) gr[d][k] += dp[d] * cf;
+      if constexpr (POINTS) {
+        const int64_t p = a.off[e[j]] + q;
+        for (int i = 0; i < 3; i++) a.xq[p * 3 + i] = x[i];
+        continue;
       }
-    }
-    // physical gradient (Axes2XYZ of the axes gradient, i.e. the gradient in
-    // x, y, z) and |det J| (the element's volume / area / length measure)
-    double g[3][NS], det;
-    if (dim == 3) {
-      det = -J[0][2] * J[1][1] * J[2][0] + J[0][1] * J[1][2] * J[2][0] + J[0][2] * J[1][0] * J[2][1] -
-            J[0][0] * J[1][2] * J[2][1] - J[0][1] * J[1][0] * J[2][2] + J[0][0] * J[1][1] * J[2][2];
-      double ji[3][3];  // inverse of J: ji[d][i] = d xi_d / d x_i
-      ji[0][0] = (-J[1][2] * J[2][1] + J[1][1] * J[2][2]) / det;
-      ji[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) / det;
-      ji[0][2] = (-J[0][2] * J[1][1] + J[0][1] * J[1][2]) / det;
-      ji[1][0] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) / det;
-      ji[1][1] = (-J[0][2] * J[2][0] + J[0][0] * J[2][2]) / det;
-      ji[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) / det;
-      ji[2][0] = (-J[1][1] * J[2][0] + J[1][0] * J[2][1]) / det;
-      ji[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) / det;
-      ji[2][2] = (-J[0][1] * J[1][0] + J[0][0] * J[1][1]) / det;
-      for (int i = 0; i < 3; i++)
-        for (int k = 0; k < NS; k++) g[i][k] = ji[0][i] * gr[0][k] + ji[1][i] * gr[1][k] + ji[2][i] * gr[2][k];
-    } else if (dim == 2) {
-      // surface element: g = J (J^T J)^-1 grad_xi, det = sqrt(det J^T J)
-      const double g11 = J[0][0] * J[0][0] + J[1][0] * J[1][0] + J[2][0] * J[2][0];
-      const double g12 = J[0][0] * J[0][1] + J[1][0] * J[1][1] + J[2][0] * J[2][1];
-      const double g22 = J[0][1] * J[0][1] + J[1][1] * J[1][1] + J[2][1] * J[2][1];
-      const double dg = g11 * g22 - g12 * g12;
-      det = sqrt(dg);
-      for (int k = 0; k < NS; k++) {
-        const double h0 = (g22 * gr[0][k] - g12 * gr[1][k]) / dg;
-        const double h1 = (-g12 * gr[0][k] + g11 * gr[1][k]) / dg;
-        for (int i = 0; i < 3; i++) g[i][k] = J[i][0] * h0 + J[i][1] * h1;
+      double g[3][NS], det;
+      if (AFF || dim == 3) {
+        double ji[3][3];
+        if (AFF) {
+          det = s_j[j * 10];
+#pragma unroll
+          for (int d = 0; d < 9; d++) ji[d / 3][d % 3] = s_j[j * 10 + 1 + d];
+        } else {
+          det = jac_inverse(J, ji);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+          for (int k = 0; k < NS; k++)
+            g[i][k] = ji[0][i] * gr[j][0][k] + ji[1][i] * gr[j][1][k] + ji[2][i] * gr[j][2][k];
+      } else if (dim == 2) {
+        // surface element: g = J (J^T J)^-1 grad_xi, det = sqrt(det J^T J)
+        const double g11 = J[0][0] * J[0][0] + J[1][0] * J[1][0] + J[2][0] * J[2][0];
+        const double g12 = J[0][0] * J[0][1] + J[1][0] * J[1][1] + J[2][0] * J[2][1];
+        const double g22 = J[0][1] * J[0][1] + J[1][1] * J[1][1] + J[2][1] * J[2][1];
+        const double dg = g11 * g22 - g12 * g12;
+        det = sqrt(dg);
+        for (int k = 0; k < NS; k++) {
+          const double h0 = (g22 * gr[j][0][k] - g12 * gr[j][1][k]) / dg;
+          const double h1 = (-g12 * gr[j][0][k] + g11 * gr[j][1][k]) / dg;
+          for (int i = 0; i < 3; i++) g[i][k] = J[i][0] * h0 + J[i][1] * h1;
+        }
+      } else {
+        const double l2 = J[0][0] * J[0][0] + J[1][0] * J[1][0] + J[2][0] * J[2][0];
+        det = sqrt(l2);
+        for (int k = 0; k < NS; k++)
+          for (int i = 0; i < 3; i++) g[i][k] = J[i][0] * gr[j][0][k] / l2;
       }
-    } else {
-      const double l2 = J[0][0] * J[0][0] + J[1][0] * J[1][0] + J[2][0] * J[2][0];
-      det = sqrt(l2);
-      for (int k = 0; k < NS; k++)
-        for (int i = 0; i < 3; i++) g[i][k] = J[i][0] * gr[0][k] / l2;
-    }
-    // exact solution at x
-    double ue[NS], ge[3][NS];
-    if (a.kind == PZG_EXACT_POINTS) {
-      const int64_t p = a.off[e] + q;
-      for (int k = 0; k < NS; k++) {
-        ue[k] = a.uq[p * NS + k];
-        for (int d = 0; d < 3; d++) ge[d][k] = d < dim ? a.duq[(p * dim + d) * NS + k] : 0.;
+      // exact solution at x
+      double ue[NS], ge[3][NS];
+      if (a.kind == PZG_EXACT_POINTS) {
+        const int64_t p = a.off[e[j]] + q;
+        for (int k = 0; k < NS; k++) {
+          ue[k] = a.uq[p * NS + k];
+          for (int d = 0; d < 3; d++) ge[d][k] = d < dim ? a.duq[(p * dim + d) * NS + k] : 0.;
+        }
+      } else {
+        double g1[3], u1;
+        exact_dev(a, x, u1, g1);
+        for (int k = 0; k < NS; k++) {
+          ue[k] = u1;
+          for (int d = 0; d < 3; d++) ge[d][k] = g1[d];
+        }
       }
-    } else {
-      double g1[3], u1;
-      exact_dev(a, x, u1, g1);
-      for (int k = 0; k < NS; k++) {
-        ue[k] = u1;
-        for (int d = 0; d < 3; d++) ge[d][k] = g1[d];
-      }
+      const double coef = a.coef ? a.coef[e[j]] : (a.material == PZG_MAT_ELAST3D ? a.E : a.kconst);
+      double v[MAXERR];
+      err_values<NS>(a, coef, u[j], g, ue, ge, v);
+      const double wdet = W[q] * fabs(det);
+#pragma unroll
+      for (int m = 0; m < MAXERR; m++) acc[j][m] += wdet * v[m];
+      __builtin_amdgcn_sched_barrier(0);  // one element at a time (else 256 registers for four)
     }
-    double v[MAXERR];
-    err_values<NS>(a, coef, u, g, ue, ge, v);
-    const double wdet = W[q] * fabs(det);
-    for (int m = 0; m < MAXERR; m++) acc[m] += wdet * v[m];
   }
   if constexpr (POINTS) return;
-  for (int o = G >> 1; o > 0; o >>= 1)
-    for (int m = 0; m < MAXERR; m++) acc[m] += __shfl_xor(acc[m], o, 64);
-  if (lq == 0)
-    for (int m = 0; m < a.nerr; m++) a.out[e * a.nerr + m] = sqrt(acc[m]);
+#pragma unroll
+  for (int j = 0; j < EB; j++) {
+    for (int o = G >> 1; o > 0; o >>= 1)
+#pragma unroll
+      for (int m = 0; m < MAXERR; m++) acc[j][m] += __shfl_xor(acc[j][m], o, 64);
+    if (lq == 0 && g0 + j < a.nlist)
+#pragma unroll
+      for (int m = 0; m < MAXERR; m++)
+        if (m < a.nerr) a.out[e[j] * a.nerr + m] = sqrt(acc[j][m]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -322,7 +445,26 @@ static int post_prepare(Ctx &c, int porder) {
   std::vector<int32_t> list(c.nvol);
   {
     std::vector<int64_t> fill(c.post_lptr.begin(), c.post_lptr.end() - 1);
-    for (int64_t e = 0; e < c.nvol; e++) list[fill[c.vol_bucket[e]]++] = (int32_t)e;
+    if (hp) {
+      // elements whose vertex ids are in the same order have the same table
+      // columns and come next to each other
+      std::vector<uint8_t> key(c.nvol);
+      int64_t cnt[257] = {0};
+      for (int64_t e = 0; e < c.nvol; e++) {
+        const int64_t *id = &c.vol_nodes[e * c.vol_ncorner];
+        int k = 0;
+        for (int i = 0; i < c.vol_ncorner; i++)
+          for (int j = 0; j < i; j++) k = 2 * k + (id[j] < id[i] ? 1 : 0);
+        key[e] = (uint8_t)k;  // at most 6 comparisons
+        cnt[k + 1]++;
+      }
+      for (int k = 0; k < 256; k++) cnt[k + 1] += cnt[k];
+      std::vector<int32_t> byk(c.nvol);
+      for (int64_t e = 0; e < c.nvol; e++) byk[cnt[key[e]]++] = (int32_t)e;
+      for (int64_t k = 0; k < c.nvol; k++) list[fill[c.vol_bucket[byk[k]]]++] = byk[k];
+    } else {
+      for (int64_t e = 0; e < c.nvol; e++) list[fill[c.vol_bucket[e]]++] = (int32_t)e;
+    }
   }
   hipStream_t s = c.stream;
   PZG_TRY(dev_upload(c.d_post_tab, tab.data(), tab.size(), s));
@@ -351,26 +493,34 @@ static int post_launch(Ctx &c, PostArgs a) {
     a.nslot = hp ? t.nsh : (t.ncol < c.vol_nsides ? t.ncol : c.vol_nsides);
     // G lanes per element (a power of two up to a wavefront), enough for the
     // element's points, and enough for the workgroup's elements to fit in LDS
-    const int ns = POINTS ? 0 : c.nstate;
-    auto lds_of = [&](int g) {
-      return (size_t)(PTPB / g) * ((size_t)a.nslot * (ns ? ns : 1) * 8 + 24 * 8 + a.nslot * 4);
+    const bool aff = c.vol_etype == PZG_TET;
+    auto lds_of = [&](int g, int eb) {
+      return (size_t)(PTPB / g) * eb * ((size_t)a.nslot * (POINTS ? 1 : c.nstate) * 8 + (24 + 10) * 8 + a.nslot * 4);
     };
-    int G = 1;
-    while (G < 64 && (G < t.nq || lds_of(G) > 65536)) G <<= 1;
+    auto group = [&](int eb) {
+      int G = 1;
+      while (G < 64 && (G < t.nq || lds_of(G, eb) > 65536)) G <<= 1;
+      return G;
+    };
+    // elements per group: as many as registers hold, when that still leaves two
+    // workgroups per CU (below it, fewer elements per group fill the chip better)
+    int eb = POINTS ? 1 : c.nstate == 1 && aff ? 4 : 2;
+    if (eb > 1 && (a.nlist < (int64_t)512 * eb * (PTPB / group(eb)) || lds_of(group(eb), eb) > 65536)) eb = 1;
+    const int G = group(eb);
     a.G = G;
-    const int ngrp = PTPB / G;
-    const size_t lds = lds_of(G);
+    const size_t lds = lds_of(G, eb);
     if (lds > 65536) {
       set_error("post-processing: element too large for the error kernel");
       return PZG_EUNSUP;
     }
-    const dim3 grid((unsigned)((a.nlist + ngrp - 1) / ngrp));
-    if (POINTS)
-      hipLaunchKernelGGL((k_post<1, true>), grid, dim3(PTPB), lds, c.stream, a);
-    else if (c.nstate == 1)
-      hipLaunchKernelGGL((k_post<1, false>), grid, dim3(PTPB), lds, c.stream, a);
-    else
-      hipLaunchKernelGGL((k_post<3, false>), grid, dim3(PTPB), lds, c.stream, a);
+    const int64_t per = (int64_t)(PTPB / G) * eb;
+    const dim3 grid((unsigned)((a.nlist + per - 1) / per));
+    if (POINTS) hipLaunchKernelGGL((k_post<1, true, 1, false>), grid, dim3(PTPB), lds, c.stream, a);
+    else if (c.nstate == 1 && eb == 4) hipLaunchKernelGGL((k_post<1, false, 4, true>), grid, dim3(PTPB), lds, c.stream, a);
+    else if (c.nstate == 1 && eb == 2) hipLaunchKernelGGL((k_post<1, false, 2, false>), grid, dim3(PTPB), lds, c.stream, a);
+    else if (c.nstate == 1) hipLaunchKernelGGL((k_post<1, false, 1, false>), grid, dim3(PTPB), lds, c.stream, a);
+    else if (eb == 2) hipLaunchKernelGGL((k_post<3, false, 2, false>), grid, dim3(PTPB), lds, c.stream, a);
+    else hipLaunchKernelGGL((k_post<3, false, 1, false>), grid, dim3(PTPB), lds, c.stream, a);
     PZG_HIP(hipGetLastError());
   }
   return PZG_OK;
