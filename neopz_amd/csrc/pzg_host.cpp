@@ -1952,7 +1952,9 @@ int pzg_learned_train(pzg_ctx *ctx, int32_t steps, double lr, double *loss_first
   double l = 0.;
   PZG_TRY(les_fit_G(c));  // G: least squares on every pair collected so far
   for (int t = 0; t < steps; t++) {
-    PZG_TRY(les_loss_grad(c, t == 0 ? &l : nullptr));
+    // the features are those of the call; the steps train the network alone (G is
+    // the fit): no gradient of G
+    PZG_TRY(les_loss_grad(c, t == 0 ? &l : nullptr, t == 0, false));
     if (t == 0 && loss_first) *loss_first = l;
     PZG_TRY(les_adam_step(c, lr));
   }

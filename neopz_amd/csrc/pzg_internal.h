@@ -464,7 +464,7 @@ struct LesCheb {
 // z = M r (learned smoother); with ch, the Chebyshev step with y = M r instead
 int les_apply(Ctx &c, const float *r, float *z, const SolveScalars *sc, const LesCheb *ch = nullptr);
 int les_collect(Ctx &c, int nrhs, uint64_t seed);
-int les_loss_grad(Ctx &c, double *loss_out);
+int les_loss_grad(Ctx &c, double *loss_out, bool features = true, bool grad_G = true);
 int les_adam_step(Ctx &c, double lr);
 int les_fit_G(Ctx &c);  // G from the accumulated least-squares sums
 // penalty rows of the learned path (pzg_penalty.hip)

@@ -70,21 +70,6 @@ __global__ void k_nn_in(int64_t rows, const float *__restrict__ X, const float *
   H[g] = s;
 }
 
-// M[s][I] = mean_{J in N(I)} H[s][J]
-__global__ void k_nn_agg(int64_t rows, int64_t nc, const int64_t *__restrict__ cia,
-                         const int32_t *__restrict__ cja, const float *__restrict__ H,
-                         float *__restrict__ M) {
-  int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= rows * NNF) return;
-  int64_t r = g / NNF;
-  int f = (int)(g % NNF);
-  int64_t s = r / nc, I = r % nc;
-  const int64_t j0 = cia[I], j1 = cia[I + 1];
-  float acc = 0.f;
-  for (int64_t k = j0; k < j1; k++) acc += H[(s * nc + cja[k]) * NNF + f];
-  M[g] = j1 > j0 ? acc / (float)(j1 - j0) : 0.f;
-}
-
 // out[s][J] (+)= sum_{I in N(J)} Y[s][I] / deg(I)   (transpose of the mean)
 __global__ void k_nn_agg_t(int64_t rows, int64_t nc, const int64_t *__restrict__ cia,
                            const int32_t *__restrict__ cja, const float *__restrict__ Y,
@@ -102,23 +87,31 @@ __global__ void k_nn_agg_t(int64_t rows, int64_t nc, const int64_t *__restrict__
   out[g] += acc;
 }
 
-// P = H A + M B;  Hout = lrelu(P)   (weights staged in LDS)
-__global__ __launch_bounds__(TPB) void k_nn_layer(int64_t rows, const float *__restrict__ H,
-                                                  const float *__restrict__ M,
+// M[I] = mean_{J in N(I)} H[J];  P = H A + M B;  Hout = lrelu(P)   (weights and the
+// workgroup's rows of M staged in LDS)
+__global__ __launch_bounds__(TPB) void k_nn_layer(int64_t rows, const int64_t *__restrict__ cia,
+                                                  const int32_t *__restrict__ cja,
+                                                  const float *__restrict__ H, float *__restrict__ M,
                                                   const float *__restrict__ A,
                                                   const float *__restrict__ B,
                                                   float *__restrict__ P, float *__restrict__ Hout) {
-  __shared__ float sA[NNF * NNF], sB[NNF * NNF];
+  __shared__ float sA[NNF * NNF], sB[NNF * NNF], sM[TPB];
   for (int k = threadIdx.x; k < NNF * NNF; k += blockDim.x) {
     sA[k] = A[k];
     sB[k] = B[k];
   }
-  __syncthreads();
   int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= rows * NNF) return;
   int64_t r = g / NNF;
   int f = (int)(g % NNF);
-  const float *h = H + r * NNF, *m = M + r * NNF;
+  if (r < rows) {
+    const int64_t j0 = cia[r], j1 = cia[r + 1];
+    float acc = 0.f;
+    for (int64_t k = j0; k < j1; k++) acc += H[(int64_t)cja[k] * NNF + f];
+    sM[threadIdx.x] = M[g] = j1 > j0 ? acc / (float)(j1 - j0) : 0.f;
+  }
+  __syncthreads();
+  if (r >= rows) return;
+  const float *h = H + r * NNF, *m = sM + (threadIdx.x - f);
   float s = 0.f;
   for (int k = 0; k < NNF; k++) s += h[k] * sA[k * NNF + f] + m[k] * sB[k * NNF + f];
   if (P) P[g] = s;
@@ -139,27 +132,18 @@ __global__ void k_nn_out(int64_t rows, const float *__restrict__ H, const float 
 }
 
 // ---- training kernels -------------------------------------------------------
-// dH = dZ Wout^T
-template <int BS>
-__global__ void k_nn_back_out(int64_t rows, const float *__restrict__ dZ,
-                              const float *__restrict__ Wout, float *__restrict__ dH) {
-  int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= rows * NNF) return;
-  int64_t r = g / NNF;
-  int f = (int)(g % NNF);
-  float s = 0.f;
-  for (int k = 0; k < BS; k++) s += dZ[r * BS + k] * Wout[f * BS + k];
-  dH[g] = s;
-}
-
-// G = dH * lrelu'(P);  dHprev = G A^T;  GBt = G B^T
-__global__ __launch_bounds__(TPB) void k_nn_back_layer(int64_t rows, const float *__restrict__ dH,
+// One layer of the backward pass.  dH of the layer's output: dZ Wout^T (LAST, the
+// last layer) or dH plus the transposed mean of the layer above's GBt (Y);
+// G = dH * lrelu'(P);  dH = G A^T;  GBt = G B^T
+template <bool LAST>
+__global__ __launch_bounds__(TPB) void k_nn_back_layer(int64_t rows, const int64_t *__restrict__ cia,
+                                                       const int32_t *__restrict__ cja,
+                                                       const float *__restrict__ dZ, const float *__restrict__ Wout,
+                                                       const float *__restrict__ Y, float *__restrict__ dH,
                                                        const float *__restrict__ P,
                                                        const float *__restrict__ A,
                                                        const float *__restrict__ B,
-                                                       float *__restrict__ G,
-                                                       float *__restrict__ dHprev,
-                                                       float *__restrict__ GBt) {
+                                                       float *__restrict__ G, float *__restrict__ GBt) {
   __shared__ float sA[NNF * NNF], sB[NNF * NNF];
   __shared__ float sG[TPB];
   for (int k = threadIdx.x; k < NNF * NNF; k += blockDim.x) {
@@ -167,29 +151,43 @@ __global__ __launch_bounds__(TPB) void k_nn_back_layer(int64_t rows, const float
     sB[k] = B[k];
   }
   int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t r = g / NNF;
+  const int f = (int)(g % NNF);
   float gv = 0.f;
-  if (g < rows * NNF) gv = dH[g] * dlrelu(P[g]);
+  if (r < rows) {
+    float d;
+    if (LAST) {
+      d = dZ[r] * Wout[f];
+    } else {
+      float acc = 0.f;
+      for (int64_t k = cia[r]; k < cia[r + 1]; k++) {
+        const int64_t I = cja[k];
+        acc += Y[I * NNF + f] / (float)(cia[I + 1] - cia[I]);
+      }
+      d = dH[g] + acc;
+    }
+    gv = d * dlrelu(P[g]);
+  }
   sG[threadIdx.x] = gv;
   __syncthreads();
-  if (g >= rows * NNF) return;
+  if (r >= rows) return;
   G[g] = gv;
-  const int f = (int)(g % NNF);
   const float *gr = sG + (threadIdx.x - f);  // the row's 32 gradients (rows never straddle blocks)
   float sa = 0.f, sb = 0.f;
   for (int k = 0; k < NNF; k++) {
     sa += gr[k] * sA[f * NNF + k];
     sb += gr[k] * sB[f * NNF + k];
   }
-  dHprev[g] = sa;
+  dH[g] = sa;
   GBt[g] = sb;
 }
 
 // dX = dH W0^T is not needed (inputs are data); dW0 etc. via outer products.
 // partial[blk][a][b] = sum_{rows in blk} L[row][a] * R[row][b]
+// (this block's NE values at partial)
 template <int FA, int FB>
-__global__ __launch_bounds__(TPB) void k_nn_outer(int64_t rows, const float *__restrict__ Lm,
-                                                  const float *__restrict__ Rm,
-                                                  float *__restrict__ partial) {
+__device__ inline void nn_outer(int64_t rows, const float *__restrict__ Lm, const float *__restrict__ Rm,
+                                float *__restrict__ partial) {
   constexpr int NE = FA * FB;
   float acc[(NE + TPB - 1) / TPB];
   for (int k = 0; k < (NE + TPB - 1) / TPB; k++) acc[k] = 0.f;
@@ -220,8 +218,31 @@ __global__ __launch_bounds__(TPB) void k_nn_outer(int64_t rows, const float *__r
   }
   for (int k = 0; k < (NE + TPB - 1) / TPB; k++) {
     int e = threadIdx.x + k * TPB;
-    if (e < NE) partial[(int64_t)blockIdx.x * NE + e] = acc[k];
+    if (e < NE) partial[e] = acc[k];
   }
+}
+template <int FA, int FB>
+__global__ __launch_bounds__(TPB) void k_nn_outer(int64_t rows, const float *__restrict__ Lm,
+                                                  const float *__restrict__ Rm,
+                                                  float *__restrict__ partial) {
+  nn_outer<FA, FB>(rows, Lm, Rm, partial + (int64_t)blockIdx.x * FA * FB);
+}
+
+// Every weight matrix of the network in one launch (blockIdx.y: the matrix), its
+// partials at off inside the block's n parameters.  A training step of 1,728
+// elements is bound by its launches: one for the products and one for their sums
+// take 20 us, a pair per matrix took 8 x 19 us.
+constexpr int NN_MATS = 2 * NNL + 2;
+struct NnMats {
+  const float *L[NN_MATS], *R[NN_MATS];
+  int off[NN_MATS], n;
+};
+__global__ __launch_bounds__(TPB) void k_nn_outer_all(int64_t rows, NnMats a, float *__restrict__ partial) {
+  const int t = blockIdx.y;
+  float *p = partial + (int64_t)blockIdx.x * a.n + a.off[t];
+  if (t == 0) nn_outer<LES_FIN, NNF>(rows, a.L[t], a.R[t], p);
+  else if (t == NN_MATS - 1) nn_outer<NNF, 1>(rows, a.L[t], a.R[t], p);
+  else nn_outer<NNF, NNF>(rows, a.L[t], a.R[t], p);
 }
 
 // g[off + e] = sum_blk partial[blk][e]  (fixed order)
@@ -230,6 +251,7 @@ __global__ void k_nn_sum_partials(int nblk, int ne, const float *__restrict__ pa
   int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ne) return;
   double s = 0.;
+#pragma unroll 8  // (loads in flight; added in order)
   for (int b = 0; b < nblk; b++) s += partial[(int64_t)b * ne + e];
   g[e] = (float)s;
 }
@@ -911,30 +933,45 @@ __global__ __launch_bounds__(256) void k_les_solve(int ne, int nr, const double 
 // per element: y_k = G r_k, d_k = mask (s y_k - e_k); loss_e = sum |d|^2,
 // ds_e = sum d.y; Dsc = 2 s d / den (the G gradient rows).  One workgroup
 // per element.
+// G in LDS (for 81 values its row stride has no bank conflicts), four pairs at a time;
+// 1,728 elements of 81 values and 4 pairs, 53 us with G's rows read by one lane each.
 __global__ __launch_bounds__(128) void k_les_fwd(int ne, int nr, const float *__restrict__ G,
                                                  const float *__restrict__ scale,
                                                  const float *__restrict__ M, const float *__restrict__ R,
                                                  const float *__restrict__ E, double den,
                                                  float *__restrict__ Dsc, double *__restrict__ loss_e,
                                                  double *__restrict__ ds_e) {
-  __shared__ float sr[LES_MAXNE];
+  __shared__ float sG[LES_MAXNE * LES_MAXNE], sr[LES_MAXNE][4];
   __shared__ double red[2][128];
   const int64_t e = blockIdx.x;
   const int tid = threadIdx.x;
   const float s = scale[e];
   double lacc = 0., dacc = 0.;
-  for (int k = 0; k < nr; k++) {
+  for (int t = tid; t < ne * ne; t += blockDim.x) sG[t] = G[t];
+  for (int k0 = 0; k0 < nr; k0 += 4) {
     __syncthreads();
-    for (int t = tid; t < ne; t += blockDim.x) sr[t] = R[(e * nr + k) * ne + t];
+    for (int t = tid; t < 4 * ne; t += blockDim.x) {
+      const int k = t / ne;
+      sr[t - k * ne][k] = k0 + k < nr ? R[(e * nr + k0 + k) * ne + t - k * ne] : 0.f;
+    }
     __syncthreads();
     for (int i = tid; i < ne; i += blockDim.x) {
-      float y = 0.f;
-      for (int j = 0; j < ne; j++) y += G[i * ne + j] * sr[j];
+      float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int j = 0; j < ne; j++) {
+        const float gij = sG[i * ne + j];
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] += gij * sr[j][k];
+      }
       const float m = M[e * ne + i];
-      const double d = m * ((double)s * y - (double)E[(e * nr + k) * ne + i]);
-      lacc += d * d;
-      dacc += d * y;
-      Dsc[(e * nr + k) * ne + i] = (float)(2.0 * s * d / den);
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (k0 + k >= nr) continue;
+        const double d = m * ((double)s * y[k] - (double)E[(e * nr + k0 + k) * ne + i]);
+        lacc += d * d;
+        dacc += d * y[k];
+        Dsc[(e * nr + k0 + k) * ne + i] = (float)(2.0 * s * d / den);
+      }
     }
   }
   red[0][tid] = lacc;
@@ -1113,11 +1150,9 @@ static int les_forward(Ctx &c, bool keep) {
   hipLaunchKernelGGL(k_nn_in<LES_FIN>, dim3(g), dim3(TPB), 0, c.stream, rows, c.d_les_X.as<float>(),
                      th + o.w0, H);
   for (int l = 0; l < NNL; l++) {
-    hipLaunchKernelGGL(k_nn_agg, dim3(g), dim3(TPB), 0, c.stream, rows, rows, c.d_les_cia.as<int64_t>(),
-                       c.d_les_cja.as<int32_t>(), H + (int64_t)l * need, M + (int64_t)l * need);
-    hipLaunchKernelGGL(k_nn_layer, dim3(g), dim3(TPB), 0, c.stream, rows, H + (int64_t)l * need,
-                       M + (int64_t)l * need, th + o.a[l], th + o.b[l], keep ? P + (int64_t)l * need : nullptr,
-                       H + (int64_t)(l + 1) * need);
+    hipLaunchKernelGGL(k_nn_layer, dim3(g), dim3(TPB), 0, c.stream, rows, c.d_les_cia.as<int64_t>(),
+                       c.d_les_cja.as<int32_t>(), H + (int64_t)l * need, M + (int64_t)l * need, th + o.a[l],
+                       th + o.b[l], keep ? P + (int64_t)l * need : nullptr, H + (int64_t)(l + 1) * need);
   }
   hipLaunchKernelGGL(k_nn_out<1>, dim3(grid1(rows)), dim3(TPB), 0, c.stream, rows, H + (int64_t)NNL * need,
                      th + o.wout, c.d_les_z.as<float>());
@@ -1718,8 +1753,9 @@ int les_fit_G(Ctx &c) {
   return PZG_OK;
 }
 
-// loss and gradient (into d_les_g) on the stored pairs
-int les_loss_grad(Ctx &c, double *loss_out) {
+// loss and gradient (into d_les_g) on the stored pairs; features: the elements'
+// features are not in place yet; grad_G: also the gradient of G
+int les_loss_grad(Ctx &c, double *loss_out, bool features, bool grad_G) {
   if (!c.les_ready || c.les_nr == 0) {
     set_error("learned preconditioner: no training pairs (pzg_learned_collect)");
     return PZG_ESTATE;
@@ -1727,7 +1763,7 @@ int les_loss_grad(Ctx &c, double *loss_out) {
   const int ne = c.les_ne, nr = (int)c.les_nr;
   const int64_t nv = c.nvol, rows = nv, need = rows * NNF;
   LesOff o = les_offsets(ne);
-  PZG_TRY(les_features(c));
+  if (features) PZG_TRY(les_features(c));
   PZG_TRY(les_forward(c, true));
   PZG_TRY(dev_alloc(c.d_les_D, sizeof(float) * nv * nr * ne));
   PZG_TRY(dev_alloc(c.d_les_le, sizeof(double) * nv));
@@ -1735,9 +1771,9 @@ int les_loss_grad(Ctx &c, double *loss_out) {
   PZG_TRY(dev_alloc(c.d_les_loss, sizeof(double)));
   PZG_TRY(dev_alloc(c.d_nn_dZ, sizeof(float) * rows));
   PZG_TRY(dev_alloc(c.d_nn_dH, sizeof(float) * need));
-  PZG_TRY(dev_alloc(c.d_nn_G, sizeof(float) * need));
-  PZG_TRY(dev_alloc(c.d_nn_tmp, sizeof(float) * need));
-  PZG_TRY(dev_alloc(c.d_nn_part, sizeof(float) * NBLK_RED * std::max(ne * ne, NNF * NNF)));
+  PZG_TRY(dev_alloc(c.d_nn_G, sizeof(float) * need * NNL));
+  PZG_TRY(dev_alloc(c.d_nn_tmp, sizeof(float) * need * 2));
+  PZG_TRY(dev_alloc(c.d_nn_part, sizeof(float) * NBLK_RED * std::max(ne * ne, o.n - o.w0)));
   const float *th = c.d_les_th.as<float>();
   float *gr = c.d_les_g.as<float>();
   hipStream_t s = c.stream;
@@ -1769,34 +1805,40 @@ int les_loss_grad(Ctx &c, double *loss_out) {
     hipLaunchKernelGGL(k_les_sym, dim3(grid1(ne * ne)), dim3(TPB), 0, s, ne, gr + o.g);
     return PZG_OK;
   };
-  PZG_TRY(outerG());
+  if (grad_G) PZG_TRY(outerG());
   // network backward (rows = elements)
   float *H = c.d_nn_trH.as<float>(), *M = c.d_nn_trM.as<float>(), *P = c.d_nn_trP.as<float>();
   const int gnode = grid1(need);
   const int nrn = (int)std::min<int64_t>(NBLK_RED, std::max<int64_t>(1, rows / 64));
-  auto outer = [&](const float *Lm, const float *Rm, int fa, int fb, int off) {
-    float *part = c.d_nn_part.as<float>();
-    if (fa == NNF && fb == NNF)
-      hipLaunchKernelGGL((k_nn_outer<NNF, NNF>), dim3(nrn), dim3(TPB), 0, s, rows, Lm, Rm, part);
-    else if (fa == NNF && fb == 1)
-      hipLaunchKernelGGL((k_nn_outer<NNF, 1>), dim3(nrn), dim3(TPB), 0, s, rows, Lm, Rm, part);
-    else
-      hipLaunchKernelGGL((k_nn_outer<LES_FIN, NNF>), dim3(nrn), dim3(TPB), 0, s, rows, Lm, Rm, part);
-    hipLaunchKernelGGL(k_nn_sum_partials, dim3(grid1(fa * fb)), dim3(TPB), 0, s, nrn, fa * fb, part, gr + off);
-  };
-  hipLaunchKernelGGL(k_nn_back_out<1>, dim3(gnode), dim3(TPB), 0, s, rows, c.d_nn_dZ.as<float>(), th + o.wout,
-                     c.d_nn_dH.as<float>());
-  outer(H + (int64_t)NNL * need, c.d_nn_dZ.as<float>(), NNF, 1, o.wout);
+  float *dH = c.d_nn_dH.as<float>(), *G = c.d_nn_G.as<float>(), *tmp = c.d_nn_tmp.as<float>();
+  const int64_t *cia = c.d_les_cia.as<int64_t>();
+  const int32_t *cja = c.d_les_cja.as<int32_t>();
+  NnMats mats;
+  mats.n = o.n - o.w0;
+  mats.L[0] = c.d_les_X.as<float>();
+  mats.R[0] = dH;
+  mats.off[0] = 0;
+  mats.L[NN_MATS - 1] = H + (int64_t)NNL * need;
+  mats.R[NN_MATS - 1] = c.d_nn_dZ.as<float>();
+  mats.off[NN_MATS - 1] = o.wout - o.w0;
   for (int l = NNL - 1; l >= 0; l--) {
-    hipLaunchKernelGGL(k_nn_back_layer, dim3(gnode), dim3(TPB), 0, s, rows, c.d_nn_dH.as<float>(),
-                       P + (int64_t)l * need, th + o.a[l], th + o.b[l], c.d_nn_G.as<float>(),
-                       c.d_nn_dH.as<float>(), c.d_nn_tmp.as<float>());
-    outer(H + (int64_t)l * need, c.d_nn_G.as<float>(), NNF, NNF, o.a[l]);
-    outer(M + (int64_t)l * need, c.d_nn_G.as<float>(), NNF, NNF, o.b[l]);
-    hipLaunchKernelGGL(k_nn_agg_t, dim3(gnode), dim3(TPB), 0, s, rows, rows, c.d_les_cia.as<int64_t>(),
-                       c.d_les_cja.as<int32_t>(), c.d_nn_tmp.as<float>(), c.d_nn_dH.as<float>());
+    float *y0 = tmp + (l & 1 ? 0 : need), *y1 = tmp + (l & 1 ? need : 0);  // neighbours read the layer above's
+    if (l == NNL - 1)
+      hipLaunchKernelGGL(k_nn_back_layer<true>, dim3(gnode), dim3(TPB), 0, s, rows, cia, cja, c.d_nn_dZ.as<float>(),
+                         th + o.wout, y0, dH, P + (int64_t)l * need, th + o.a[l], th + o.b[l], G + (int64_t)l * need, y1);
+    else
+      hipLaunchKernelGGL(k_nn_back_layer<false>, dim3(gnode), dim3(TPB), 0, s, rows, cia, cja, c.d_nn_dZ.as<float>(),
+                         th + o.wout, y0, dH, P + (int64_t)l * need, th + o.a[l], th + o.b[l], G + (int64_t)l * need, y1);
+    for (int w = 0; w < 2; w++) {
+      mats.L[1 + 2 * l + w] = (w ? M : H) + (int64_t)l * need;
+      mats.R[1 + 2 * l + w] = G + (int64_t)l * need;
+      mats.off[1 + 2 * l + w] = (w ? o.b[l] : o.a[l]) - o.w0;
+    }
   }
-  outer(c.d_les_X.as<float>(), c.d_nn_dH.as<float>(), LES_FIN, NNF, o.w0);
+  hipLaunchKernelGGL(k_nn_agg_t, dim3(gnode), dim3(TPB), 0, s, rows, rows, cia, cja, (const float *)tmp, dH);
+  hipLaunchKernelGGL(k_nn_outer_all, dim3(nrn, NN_MATS), dim3(TPB), 0, s, rows, mats, c.d_nn_part.as<float>());
+  hipLaunchKernelGGL(k_nn_sum_partials, dim3(grid1(mats.n)), dim3(TPB), 0, s, nrn, mats.n,
+                     c.d_nn_part.as<float>(), gr + o.w0);
   PZG_HIP(hipGetLastError());
   if (loss_out) {
     PZG_HIP(hipMemcpyAsync(loss_out, c.d_les_loss.p, sizeof(double), hipMemcpyDeviceToHost, s));
