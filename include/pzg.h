@@ -318,8 +318,9 @@ int pzg_true_residual(pzg_ctx *ctx, double *rel);
 
 /* pzg_true_residual without any allocation: no counterpart in the reference;
  * for callers that cannot allocate device memory (code under HIP graph
- * capture, serving loops, harnesses that forbid hipMalloc).  The FP64 block
- * CSR and the solution must already be on the device (after a solve,
+ * capture, serving loops, harnesses that forbid hipMalloc).  The FP64
+ * operator (the block CSR or, on meshes of identical affine p = 2 hexahedra,
+ * the element products) and the solution must already be on the device (after a solve,
  * pzg_multadd or pzg_true_residual of the current assembly), else
  * PZG_ESTATE.  Reduces in a fixed per-GPU static scratch of 32.8 KB (2 x 2048
  * partial sums, the two norms, a counter), set up by pzg_create and held
