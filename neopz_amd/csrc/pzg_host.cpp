@@ -54,6 +54,12 @@ template <class F> static void parallel_for(int64_t n, F f) {
   for (auto &x : th) x.join();
 }
 
+void drop_solve_graph(Ctx &c) {
+  if (c.solve_graph) (void)hipGraphExecDestroy(c.solve_graph);
+  c.solve_graph = nullptr;
+  c.solve_key.clear();
+}
+
 static void free_all(Ctx &c) {
   DevBuf *bufs[] = {&c.d_ia, &c.d_ja, &c.d_a, &c.d_rhs, &c.d_diag, &c.d_ubia, &c.d_ubja,
                     &c.d_fbia, &c.d_fbja, &c.d_rank_fwd, &c.d_rank_bwd, &c.d_lowsrc,
@@ -78,9 +84,7 @@ static void free_all(Ctx &c) {
                     &c.cv.d_ef, &c.cb.d_cel, &c.cb.d_cslot, &c.cb.d_T, &c.cb.d_blk, &c.cb.d_n,
                     &c.cb.d_ek, &c.cb.d_ef};
   for (DevBuf *b : bufs) dev_free(*b);
-  if (c.solve_graph) (void)hipGraphExecDestroy(c.solve_graph);
-  c.solve_graph = nullptr;
-  c.solve_key.clear();
+  drop_solve_graph(c);
   mg_free(c);
 }
 
@@ -496,6 +500,7 @@ static int mesh_set(Ctx &c, const pzg_mesh_desc *m) {
     set_error("pzg_mesh_set: boundary element arrays missing");
     return PZG_EINVAL;
   }
+  drop_solve_graph(c);
   c.dim = m->dim;
   c.material = m->material;
   c.nstate = m->nstate;
@@ -873,6 +878,7 @@ static int struct_create(Ctx &c) {
     set_error("pzg_struct_create: call pzg_mesh_set first");
     return PZG_ESTATE;
   }
+  drop_solve_graph(c);
   const int64_t nb = c.nb, bs = c.bs;
   const int nsv = c.vol_nsides, nsb = c.bc_nsides;
   const int64_t nel = c.nvol + c.nbc;
@@ -1254,6 +1260,7 @@ int pzg_set_equation_filter(pzg_ctx *ctx, int64_t nactive, const int64_t *active
   }
   c.filt_keep.clear();
   c.filt_ia.clear();
+  drop_solve_graph(c);
   // the pattern belongs to the filter: pzg_struct_create builds it again
   c.has_struct = false;
   c.assembled = false;
@@ -1418,6 +1425,7 @@ int pzg_csr_set(pzg_ctx *ctx, int64_t neq, const int64_t *ia, const int64_t *ja,
         return PZG_EINVAL;
       }
   }
+  drop_solve_graph(c);
   // A caller matrix is handled as a scalar problem (block size 1), in its
   // own numbering (no equation filter).
   c.has_mesh = false;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -317,7 +318,9 @@ struct Ctx {
   DevBuf d_res2;  // |r|^2, |f|^2 of the FP64 true residual
   int reduce_blocks = 1024;
   // captured batch of the last CG/FCG iteration, reused while every pointer,
-  // size and launch shape in it (solve_key) is the same
+  // value, size and launch shape in it (solve_key: kf_key, mf_key and the
+  // solver's own) is the same, and given back with the structure it was
+  // captured on (drop_solve_graph)
   hipGraphExec_t solve_graph = nullptr;
   std::vector<uint64_t> solve_key;
   bool has_solution = false;
@@ -433,6 +436,22 @@ int launch_expand_upper_ja(Ctx &c);
 int launch_elem_maps(Ctx &c);
 int launch_assemble(Ctx &c);
 int launch_diag(Ctx &c);
+// gives back the kept CG/FCG graph: the structure it was captured on changes
+void drop_solve_graph(Ctx &c);
+// Words of a graph key: whole numbers and flags, the bits of a double, the
+// address of a buffer.
+inline uint64_t key_word(const DevBuf &b) { return (uint64_t)(uintptr_t)b.p; }
+inline uint64_t key_word(double v) {
+  uint64_t w;
+  std::memcpy(&w, &v, sizeof(w));
+  return w;
+}
+inline uint64_t key_word(int64_t v) { return (uint64_t)v; }
+inline uint64_t key_word(int v) { return (uint64_t)v; }
+inline uint64_t key_word(bool v) { return v ? 1 : 0; }
+template <class... T> inline void key_add(std::vector<uint64_t> &key, const T &...v) {
+  (key.push_back(key_word(v)), ...);
+}
 // decouples the inactive equations of the equation filter (mesh numbering)
 int launch_filter_mask(Ctx &c);
 int launch_expand_full(Ctx &c);
@@ -510,6 +529,8 @@ struct MfOut {
   double *partials = nullptr;
 };
 int mf_apply_out(Ctx &c, const MfOut &o, const SolveScalars *sc);
+// what the launches of mf_apply hold besides the caller's vectors (of a graph key)
+void mf_key(const Ctx &c, std::vector<uint64_t> &key);
 // the matrix-free operator reproduces the assembled K (mesh-built, no AddKel extras)
 inline bool mf_available(const Ctx &c) {
   return c.has_mesh && c.has_struct && !c.external_csr && !c.kel_added && c.assembled && !c.has_dep &&
@@ -531,6 +552,8 @@ int kf_prepare(Ctx &c, bool *ok);
 int kf_rows_grid(const Ctx &c);
 int kf_apply(Ctx &c, int mode, const double *x, const double *f, double alpha, double beta, double *out,
              const SolveScalars *sc, double *partials);
+// what the launches of kf_apply hold besides the caller's vectors (of a graph key)
+void kf_key(const Ctx &c, std::vector<uint64_t> &key);
 int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info);
 int solve_mixed(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info);
 int true_residual(Ctx &c, const double *u, double *rel);

@@ -1587,4 +1587,18 @@ int mf_apply(Ctx &c, const float *p, const float *r, float *q, const SolveScalar
 
 int mf_apply_out(Ctx &c, const MfOut &o, const SolveScalars *sc) { return mft_apply(c, o, sc); }
 
+// Every buffer, value and choice that mft_apply, or mf_launch_vol and the
+// boundary and row kernels, put into their launches.
+void mf_key(const Ctx &c, std::vector<uint64_t> &key) {
+  key_add(key, c.mf_tile, c.dim, c.nstate, c.neq, c.nb, c.nu, c.d_mf_dis, c.d_mf_pt, c.d_mf_bm);
+  if (c.mf_tile) {
+    for (int d = 0; d < 3; d++) key_add(key, c.mt_nt[d], c.mt_fn[d], c.mf_box_inv[d]);
+    key_add(key, c.mf_box_det, c.mt_nh, c.kf_nface, c.d_mt_tmap, c.d_mt_coef, c.d_mt_part, c.d_mt_hfine, c.d_mt_hblk,
+            c.d_kf_pidx, c.d_kf_pptr, c.d_kf_psrc, c.d_kf_bblk);
+  } else {
+    key_add(key, c.nvol, c.tvol.nq, c.tvol.nsh, c.tbc.nsh, c.mf_nbcd, c.mf_nout, c.d_mf_blk, c.d_mf_xe, c.d_mf_bblk,
+            c.d_mf_ptr, c.d_mf_pos, c.d_mf_bpos, c.d_mf_tab, c.d_mf_ye, c.d_mf_coef, c.d_mf_mfma, c.d_mf_geo);
+  }
+}
+
 }  // namespace pzg

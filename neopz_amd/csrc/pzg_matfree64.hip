@@ -376,6 +376,13 @@ int kf_prepare(Ctx &c, bool *ok) {
   return PZG_OK;
 }
 
+// Every buffer, value and choice that kf_apply puts into its launches.
+void kf_key(const Ctx &c, std::vector<uint64_t> &key) {
+  key_add(key, c.bs, c.neq, c.nvol, c.kf_nface, c.vol_coef.empty(), c.material == PZG_MAT_ELAST3D ? c.E : c.scale,
+          c.d_vcoef, c.d_kf_tab, c.d_kf_blk, c.d_kf_ye, c.d_blk_iptr, c.d_blk_inc, c.d_kf_pidx, c.d_kf_pptr,
+          c.d_kf_psrc, c.d_kf_bblk, c.d_kf_bm);
+}
+
 int kf_rows_grid(const Ctx &c) {
   return (int)std::max<int64_t>(1, std::min<int64_t>((c.neq + KF_TPB - 1) / KF_TPB, MAXBLK));
 }

@@ -1220,18 +1220,13 @@ static int pcg64_iterate(Ctx &c, const pzg_solve_params &prm, int pre, SolveScal
     }
     hipLaunchKernelGGL(k_cg_close<false>, dim3(1), dim3(TPB), 0, c.stream, A, B, (const double *)part, gu.blocks, n1);
   };
-  std::vector<uint64_t> key = {64, BS, (uint64_t)pre, (uint64_t)batch, (uint64_t)n, (uint64_t)nb, (uint64_t)c.nbf,
-                               (uint64_t)merge, (uint64_t)c.kf_valid, (uint64_t)c.nvol, (uint64_t)c.kf_nface,
-                               (uint64_t)c.vol_coef.empty()};
-  double coef0 = c.material == PZG_MAT_ELAST3D ? c.E : c.scale;
-  uint64_t cb;
-  std::memcpy(&cb, &coef0, sizeof(cb));
-  key.push_back(cb);
-  for (const DevBuf *b : {&c.d_scal, &c.d_partials, &c.d_diag, &c.d_bjinv64, &c.d_r, &c.d_z, &c.d_q, &c.d_u, &c.d_p,
-                          &c.d_p2, &c.d_fbia, &c.d_fbja, &c.d_fa, &c.d_vbj_eqb, &c.d_vbj_pos, &c.d_vbj_m,
-                          &c.d_vbj_off, &c.d_blk_iptr, &c.d_blk_inc, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab,
-                          &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_vcoef})
-    key.push_back((uint64_t)(uintptr_t)b->p);
+  std::vector<uint64_t> key;
+  key_add(key, 64, BS, pre, batch, n, nb, c.nbf, merge, c.kf_valid);
+  for (const DevBuf *b : {&c.d_scal, &c.d_partials, &c.d_r, &c.d_z, &c.d_q, &c.d_u, &c.d_p, &c.d_p2, &c.d_diag,
+                          &c.d_bjinv64, &c.d_fbia, &c.d_fbja, &c.d_fa, &c.d_vbj_eqb, &c.d_vbj_pos, &c.d_vbj_m,
+                          &c.d_vbj_off})
+    key_add(key, *b);
+  if (c.kf_valid) kf_key(c, key);
   return run_batches(c, prm.use_graph != 0, key, enqueue, hs);
 }
 
@@ -1877,18 +1872,12 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
     // not kept beyond the solve
     std::vector<uint64_t> key;
     if (!multigrid) {
-      key = {32, BS, (uint64_t)batch, (uint64_t)n, (uint64_t)nb, (uint64_t)c.nbf, (uint64_t)merge, (uint64_t)use_mf,
-             (uint64_t)vbj, (uint64_t)c.nvol, (uint64_t)c.mf_nbcd, (uint64_t)c.tvol.nq};
-      double nu = c.nu;
-      uint64_t cb;
-      std::memcpy(&cb, &nu, sizeof(cb));
-      key.push_back(cb);
+      key_add(key, 32, BS, batch, n, nb, c.nbf, merge, use_mf, vbj);
       for (const DevBuf *b : {&c.d_scal, &c.d_partials, &c.d_xs, &c.d_rs, &c.d_zs, &c.d_ps, &c.d_ps2, &c.d_qs,
                               &c.d_bjinv, &c.d_bsr, &c.d_fbia, &c.d_fbja, &c.d_vbj_eqb, &c.d_vbj_pos, &c.d_vbj_m,
-                              &c.d_vbj_off, &c.d_vbjinv32, &c.d_mf_dis, &c.d_mf_pt, &c.d_mf_blk, &c.d_mf_xe,
-                              &c.d_mf_bblk, &c.d_mf_bm, &c.d_mf_ptr, &c.d_mf_pos, &c.d_mf_bpos, &c.d_mf_tab,
-                              &c.d_mf_ye, &c.d_mf_coef, &c.d_mf_mfma, &c.d_mf_geo})
-        key.push_back((uint64_t)(uintptr_t)b->p);
+                              &c.d_vbj_off, &c.d_vbjinv32})
+        key_add(key, *b);
+      if (use_mf) mf_key(c, key);
     }
     PZG_TRY(run_batches(c, prm.use_graph != 0, key, enqueue, hs));
     total_it = hs.iter;
