@@ -870,6 +870,20 @@ __global__ void k_mft_inv(int64_t n, const int32_t *__restrict__ fmap, int32_t *
   const int32_t b = fmap[t];
   if (b < 0 || b >= n || atomicExch(&bf[b], (int32_t)t) != -1) *bad = 1;
 }
+// the node lies on a tile face or on the lattice boundary: k_mft_halo finishes it
+__device__ inline bool mft_shared(int32_t f, int f0, int f1, int f2) {
+  const int x = f % f0, y = f / f0 % f1, z = f / (f0 * f1);
+  return x % MT_W == 0 || x == f0 - 1 || y % MT_W == 0 || y == f1 - 1 || z % MT_W == 0 || z == f2 - 1;
+}
+// *bad when a Dirichlet face (blocks bblk) has a node inside a tile: k_mft_tile
+// finishes its nodes without the faces
+__global__ void k_mft_faces(int64_t n, const int32_t *__restrict__ bblk, int64_t nb, const int32_t *__restrict__ bf,
+                            int f0, int f1, int f2, int *bad) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int32_t b = bblk[t], f = b >= 0 && b < nb ? bf[b] : -1;
+  if (f < 0 || !mft_shared(f, f0, f1, f2)) *bad = 1;
+}
 // Shared nodes in the order of their blocks (rows of the vectors next to each
 // other are next to each other in the list): per workgroup of 256 blocks their
 // number (hblk null) or, from its first place first[workgroup], the list.
@@ -879,8 +893,7 @@ __global__ __launch_bounds__(256) void k_mft_halo_list(int64_t n, int f0, int f1
   __shared__ int wc[4];
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int32_t f = t < n ? bf[t] : -1;
-  const int x = f % f0, y = f / f0 % f1, z = f / (f0 * f1);
-  const bool h = f >= 0 && (x % MT_W == 0 || x == f0 - 1 || y % MT_W == 0 || y == f1 - 1 || z % MT_W == 0 || z == f2 - 1);
+  const bool h = f >= 0 && mft_shared(f, f0, f1, f2);
   const uint64_t mask = __ballot(h);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) wc[w] = __popcll(mask);
@@ -1065,8 +1078,9 @@ int launch_vol_lpe(Ctx &c, const MfArgs &a, const SolveScalars *sc) {
 
 }  // namespace
 
-// Tiles of a lattice of identical axis-aligned p = 2 boxes (k_mft_tile); leaves
-// c.mf_tile false on any other mesh.
+// Tiles of a lattice of identical axis-aligned p = 2 boxes (k_mft_tile) whose
+// Dirichlet faces lie on tile faces or on the lattice boundary (k_mft_halo adds
+// them); leaves c.mf_tile false on any other mesh.
 static int mft_setup(Ctx &c) {
   if (!(c.blk_asm && c.aff_on && c.blk_full && c.dim == 3 && c.nstate == 3 && c.tvol.nsh == 27 && c.tvol.nq == 27 &&
         c.nvol > 0 && kf_usable_mesh(c)))
@@ -1150,6 +1164,9 @@ static int mft_setup(Ctx &c) {
                        fn[2], fm.as<int32_t>(), c.d_mt_tmap.as<int32_t>());
     hipLaunchKernelGGL(k_mft_fill, g(nfine), dim3(MF_TPB), 0, s, nfine, -1, bf.as<int32_t>());
     hipLaunchKernelGGL(k_mft_inv, g(nfine), dim3(MF_TPB), 0, s, nfine, fm.as<int32_t>(), bf.as<int32_t>(), bad.as<int>());
+    if (c.mf_nbcd > 0)
+      hipLaunchKernelGGL(k_mft_faces, g(c.mf_nbcd * 9), dim3(MF_TPB), 0, s, c.mf_nbcd * 9, c.d_mf_bblk.as<int32_t>(),
+                         nfine, bf.as<int32_t>(), fn[0], fn[1], fn[2], bad.as<int>());
     hipLaunchKernelGGL(k_mft_halo_list, dim3((unsigned)ngrp), dim3(256), 0, s, nfine, fn[0], fn[1], fn[2], bf.as<int32_t>(),
                        first.as<int32_t>(), nh, (int32_t *)nullptr, (int32_t *)nullptr);
     hipLaunchKernelGGL(k_mft_scan, dim3(1), dim3(256), 0, s, ngrp, first.as<int32_t>());
