@@ -355,6 +355,10 @@ static int blk_setup(Ctx &c, const std::vector<double> &R) {
   c.blk_kref.swap(K);
   c.blk_full = iptr[c.nb] == c.nvol * NSH;
   for (int sh = 0; sh < NSH; sh++) c.blk_full &= T.shape_side[sh] == sh;
+  for (int64_t e = 0; e < c.nbc; e++)
+    if (c.bc_type[c.bc_id[e]] == PZG_BC_DIRICHLET)
+      for (int sh = 0; sh < c.tbc.nsh; sh++)
+        c.blk_full &= c.aidx[c.bc_conn[e * c.bc_nsides + c.tbc.shape_side[sh]]] >= 0;
   c.blk_asm = true;
   c.blk_grid = 0;
   return PZG_OK;

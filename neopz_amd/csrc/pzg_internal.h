@@ -250,7 +250,9 @@ struct Ctx {
   bool blk_asm = false;
   int blk_grid = 0;
   DevBuf d_blk_iptr, d_blk_inc, d_blk_kref;
-  bool blk_full = false;          // every shape of every element is active
+  // every shape of every element and of every Dirichlet face has a block (the
+  // element products' lists of blocks hold no -1)
+  bool blk_full = false;
   std::vector<double> blk_kref;   // the coefficient-1 element matrix
   // FP64 products from the element matrix (pzg_matfree64.hip): mesh part,
   // validity for the assembled system, entries dropped by AddKel for every
