@@ -547,6 +547,16 @@ inline bool mf_available(const Ctx &c) {
 // kf_rows_grid blocks.
 enum { KF_AXPBY = 0, KF_DOT = 1, KF_RESIDUAL = 2 };
 constexpr int64_t KF_SPLIT_TILES = 4096;  // fewer element tiles of 16: three wavefronts per tile
+// Meshes of fewer elements keep the block CSR: its product then is as fast or
+// faster (the element product waits for its tables and three dependent loads
+// whatever the size), and FP64 PCG has the one-workgroup and the merged
+// iteration on it.  Block CSR / element products, MultAdd of host vectors in us
+// and Jacobi-PCG solves in ms:
+//   3 unknowns a node: 3^3 elements 44 / 45, 6.1 / 7.5; 4^3 50 / 52, 6.2 / 6.4;
+//                      5^3 43 / 41, 9.1 / 8.6; 6^3 47 / 43, 9.8 / 8.2
+//   1 unknown a node:  8^3 elements 36 / 42, 4.2 / 6.7; 16^3 59 / 63, 7.9 / 8.8;
+//                      20^3 88 / 87, 11.9 / 10.5; 24^3 126 / 118, 15.5 / 10.8
+constexpr int64_t KF_MIN_EL3 = 96, KF_MIN_EL1 = 6000;
 bool kf_usable(const Ctx &c);
 bool kf_usable_mesh(const Ctx &c);  // its mesh part: faces and blocks by row can be listed
 int kf_setup_mesh(Ctx &c);

@@ -365,7 +365,9 @@ bool kf_usable_mesh(const Ctx &c) {
 int kf_setup_mesh(Ctx &c) { return kf_setup(c); }
 
 // The products below stand for those of the block CSR on this system
-bool kf_usable(const Ctx &c) { return kf_usable_mesh(c) && c.assembled && !c.kel_added; }
+bool kf_usable(const Ctx &c) {
+  return kf_usable_mesh(c) && c.assembled && !c.kel_added && c.nvol >= (c.nstate == 3 ? KF_MIN_EL3 : KF_MIN_EL1);
+}
 
 int kf_prepare(Ctx &c, bool *ok) {
   *ok = c.kf_valid;
