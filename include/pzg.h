@@ -320,12 +320,12 @@ int pzg_true_residual(pzg_ctx *ctx, double *rel);
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  The FP64
  * operator (the block CSR or, on meshes of identical affine p = 2 hexahedra,
- * the element products) and the solution must already be on the device (after a solve,
- * pzg_multadd or pzg_true_residual of the current assembly), else
- * PZG_ESTATE.  Reduces in a fixed per-GPU static scratch of 32.8 KB (2 x 2048
- * partial sums, the two norms, a counter), set up by pzg_create and held
- * until the process ends; any system size fits (the residual grid is capped
- * at 2048 workgroups).  Every context on one GPU shares that scratch: calls
+ * the element products) and the solution must already be on the device
+ * (after a solve, pzg_multadd or pzg_true_residual of the current assembly),
+ * else PZG_ESTATE.  Reduces in a fixed per-GPU static scratch of 32.8 KB (2 x 2048
+ * partial sums and the two norms), set up by pzg_create and held until the
+ * process ends; any system size fits (the residual grid is capped at 2048
+ * workgroups).  Every context on one GPU shares that scratch: calls
  * that overlap on one GPU (different streams or threads) race. */
 int pzg_true_residual_noalloc(pzg_ctx *ctx, double *rel);
 

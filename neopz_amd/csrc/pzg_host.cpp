@@ -69,7 +69,7 @@ static void free_all(Ctx &c) {
                     &c.d_tbc, &c.d_vcolor_list, &c.d_vol_R, &c.d_blk_iptr, &c.d_blk_inc, &c.d_blk_kref, &c.d_kf_blk, &c.d_kf_ye, &c.d_kf_tab, &c.d_kf_bblk, &c.d_kf_bm, &c.d_kf_pidx, &c.d_kf_pptr, &c.d_kf_psrc, &c.d_mt_cmap, &c.d_mt_tmap, &c.d_mt_part, &c.d_mt_coef, &c.d_mt_hfine, &c.d_mt_hblk, &c.d_mt_pt2, &c.d_vbj_pos, &c.d_vbj_m, &c.d_vbj_off, &c.d_vbj_eqb, &c.d_vbjinv64, &c.d_vbjinv32, &c.d_bcolor_list, &c.d_x, &c.d_r, &c.d_z,
                     &c.d_p, &c.d_p2, &c.d_q, &c.d_u, &c.d_f, &c.d_w, &c.d_xs, &c.d_rs,
                     &c.d_zs, &c.d_ps, &c.d_ps2, &c.d_qs, &c.d_bs, &c.d_scal, &c.d_partials,
-                    &c.d_counter, &c.d_res2, &c.d_les_th, &c.d_les_m, &c.d_les_v, &c.d_les_g,
+                    &c.d_flag, &c.d_res2, &c.d_les_th, &c.d_les_m, &c.d_les_v, &c.d_les_g,
                     &c.d_les_cia, &c.d_les_cja, &c.d_les_pen, &c.d_les_X, &c.d_les_z, &c.d_les_s,
                     &c.d_les_ye, &c.d_les_blkm, &c.d_les_eoff, &c.d_bjinv64, &c.d_les_cmap, &c.d_les_tmapb, &c.d_les_tmap, &c.d_les_part, &c.d_les_hmapb, &c.d_les_hmap, &c.d_les_hptr, &c.d_les_hsrc, &c.d_les_tscale, &c.d_les_Se, &c.d_les_M, &c.d_les_R, &c.d_les_E, &c.d_les_D,
                     &c.d_les_le, &c.d_les_ds, &c.d_les_loss, &c.d_les_fail, &c.d_nn_trH, &c.d_nn_trM,

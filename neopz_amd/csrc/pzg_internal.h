@@ -158,7 +158,7 @@ __host__ __device__ inline int64_t bsr_pos(int64_t b0, int64_t n, int64_t i, int
 // read by the direction; sc[1]: the reverse), so every workgroup can form the
 // scalars of a step from the partial sums itself.
 struct SolveScalars {
-  double rho, pq, alpha, beta, rr, normb, resid, tol, pr, zq;
+  double rho, pq, beta, normb, resid, tol;
   double rlast;   // mixed: scaled residual norm at the last reliable update
   double delta;   // mixed: reduction of the recursive residual that triggers an update
   int64_t iter, maxit;
@@ -316,7 +316,8 @@ struct Ctx {
   // ---- solver workspace -----------------------------------------------------
   DevBuf d_x, d_r, d_z, d_p, d_p2, d_q, d_u, d_f, d_w;        // fp64
   DevBuf d_xs, d_rs, d_zs, d_ps, d_ps2, d_qs, d_bs;          // fp32
-  DevBuf d_scal, d_partials, d_counter;
+  DevBuf d_scal, d_partials;
+  DevBuf d_flag;  // int: a connect block could not be inverted
   DevBuf d_res2;  // |r|^2, |f|^2 of the FP64 true residual
   int reduce_blocks = 1024;
   // captured batch of the last CG/FCG iteration, reused while every pointer,
@@ -402,7 +403,7 @@ struct Ctx {
   double mg_lmax0 = 0.;    // largest eigenvalue of the block-Jacobi scaled S
   int64_t mg_ncoarse = 0;  // unknowns of the coarsest level
   std::vector<MgLevel> mg;
-  DevBuf d_mg_vmap, d_mg_vinv, d_mg_dsq, d_mg_cinv, d_mg_r0, d_mg_d0, d_mg_t0, d_mg_w0, d_mg_lz, d_mg_y0;
+  DevBuf d_mg_vmap, d_mg_vinv, d_mg_dsq, d_mg_cinv, d_mg_r0, d_mg_d0, d_mg_t0, d_mg_w0, d_mg_lz;
 
   // post-processing (pzg_post.hip): error-rule tables per rule bucket for the
   // exact-solution order post_porder (-1: not built), the elements of every

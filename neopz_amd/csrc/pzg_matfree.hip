@@ -1417,7 +1417,6 @@ int mf_setup(Ctx &c) {
   PZG_TRY(dev_upload(c.d_mf_pos, pos.data(), pos.size(), s));
   PZG_TRY(dev_upload(c.d_mf_bpos, bpos.data(), bpos.size(), s));
   PZG_TRY(dev_upload(c.d_mf_tab, &tab, 1, s));
-  PZG_TRY(dev_alloc(c.d_mf_ye, sizeof(float) * std::max<int64_t>(ptr[nb], 1) * ns));
   PZG_TRY(dev_alloc(c.d_mf_coef, sizeof(float) * std::max<int64_t>(nvol, 1)));
   PZG_TRY(dev_alloc(c.d_mf_dis, sizeof(float) * std::max<int64_t>(c.neq, 1)));
   PZG_HIP(hipStreamSynchronize(s));
@@ -1425,6 +1424,8 @@ int mf_setup(Ctx &c) {
   c.mf_nout = ptr[nb];
   c.mf_tile = false;
   PZG_TRY(mft_setup(c));
+  // element outputs, which the tiles sum in LDS
+  if (!c.mf_tile) PZG_TRY(dev_alloc(c.d_mf_ye, sizeof(float) * std::max<int64_t>(ptr[nb], 1) * ns));
   c.mf_ready = true;
   c.mf_vals_valid = false;
   return PZG_OK;

@@ -750,13 +750,13 @@ struct LevelView {
   const float *dis = nullptr;  // level 0, matrix-free: D^-1/2 and the operator's
   float *pt = nullptr;         // pre-scaled input, written with each new d
   float *pt2 = nullptr;        // level 0, tiled operator: the second such buffer
-  float *y = nullptr;          // level 0, learned smoother: M r (else the blocks m)
+  bool les = false;            // level 0: M is the learned smoother (else the blocks m)
   Cheb ch;
 };
 
 // op(x, y, prescaled): y = A x; prescaled: L.pt already holds D^-1/2 x.
 // Leaves x and, as r - t, the residual b - A x (the restriction subtracts).
-// the learned smoother's steps (LevelView::y set)
+// the learned smoother's steps (LevelView::les)
 template <int BS, class Op>
 int smooth_les(Ctx &c, const LevelView &L, const float *b, float *x, Op op, const SolveScalars *sc,
                bool pre) {
@@ -836,7 +836,7 @@ int steps_tiled(Ctx &c, const LevelView &L, const float *b, float *x, const Solv
 
 template <int BS, class Op>
 int smooth_pre(Ctx &c, const LevelView &L, const float *b, float *x, Op op, const SolveScalars *sc) {
-  if (L.y) return smooth_les<BS>(c, L, b, x, op, sc, true);
+  if (L.les) return smooth_les<BS>(c, L, b, x, op, sc, true);
   const int g = grid1(L.nb);
   const bool ps = L.pt != nullptr;
   hipLaunchKernelGGL(k_cheb_init<BS>, dim3(g), dim3(TPB), 0, c.stream, L.nb, L.m, L.sa, L.sk, b, x, L.r,
@@ -860,7 +860,7 @@ int smooth_pre(Ctx &c, const LevelView &L, const float *b, float *x, Op op, cons
 
 template <int BS, class Op>
 int smooth_post(Ctx &c, const LevelView &L, const float *b, float *x, Op op, const SolveScalars *sc) {
-  if (L.y) return smooth_les<BS>(c, L, b, x, op, sc, false);
+  if (L.les) return smooth_les<BS>(c, L, b, x, op, sc, false);
   const int g = grid1(L.nb);
   const bool ps = L.pt != nullptr;
   if (L.pt2) {
@@ -911,7 +911,7 @@ LevelView view0(Ctx &c) {
     v.pt = c.d_mf_pt.as<float>();
     if (c.mf_tile) v.pt2 = c.d_mt_pt2.as<float>();
   }
-  if (c.mg_les) v.y = c.d_mg_y0.as<float>();
+  v.les = c.mg_les;
   v.ch = cheb_coeffs(c.mg_lmax0, c.mg_range, c.mg_degree);
   return v;
 }
@@ -1086,7 +1086,6 @@ int lanczos_lmax(Ctx &c, int64_t nb, const float *m, int64_t sa, int64_t sk, flo
   return PZG_OK;
 }
 
-// inverse of a symmetric positive definite matrix (Cholesky, in place)
 // In-place inverse of a symmetric positive definite matrix (FP64, n x n) by
 // Gauss-Jordan sweeps without pivoting, one pivot per launch pair: k_gj_save
 // keeps row and column k, k_gj_step applies the sweep
@@ -1331,10 +1330,7 @@ int setup_impl(Ctx &c) {
   }
   // largest eigenvalues of M^-1 A: level 0, then every smoothed lattice level
   {
-    if (c.mg_les) {  // the learned smoother of the current assembly
-      PZG_TRY(les_prepare(c));
-      PZG_TRY(dev_alloc(c.d_mg_y0, sizeof(float) * std::max<int64_t>(c.neq, 1)));
-    }
+    if (c.mg_les) PZG_TRY(les_prepare(c));  // the learned smoother of the current assembly
     auto op = [&](const float *x, float *y) { return op0(c, x, y, nullptr, false); };
     PZG_TRY(lanczos_lmax<BS>(c, c.nb, c.d_bjinv.as<float>(), (int64_t)BS * BS, 1, c.d_mg_r0.as<float>(),
                              c.d_mg_d0.as<float>(), c.d_mg_t0.as<float>(), c.d_mg_w0.as<float>(), op,
@@ -1463,7 +1459,7 @@ void mg_free(Ctx &c) {
   c.mg.clear();
   c.mg_struct = false;
   for (DevBuf *b : {&c.d_mg_vmap, &c.d_mg_vinv, &c.d_mg_dsq, &c.d_mg_cinv, &c.d_mg_r0, &c.d_mg_d0, &c.d_mg_t0, &c.d_mg_w0,
-                    &c.d_mg_lz, &c.d_mg_y0})
+                    &c.d_mg_lz})
     dev_free(*b);
   c.mg_ready = false;
 }

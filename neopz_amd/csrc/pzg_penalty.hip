@@ -363,8 +363,6 @@ __global__ void k_pen_zero32(int64_t np, const int64_t *__restrict__ idx, float 
 
 }  // namespace
 
-static int pen_fill(Ctx &c);
-
 // Structure of the penalty block, once per mesh (the full block pattern and
 // the penalty flags of the learned element graph): the penalized equations,
 // K_pp's CSR pattern, the Schwarz sets of the penalized boundary elements with

@@ -957,8 +957,7 @@ int launch_spmv64(Ctx &c, const double *x, double *y) {
 static int ensure_reduce(Ctx &c) {
   if (!c.d_partials.p) {
     PZG_TRY(dev_alloc(c.d_partials, sizeof(double) * NSLOT * MAXBLK));
-    PZG_TRY(dev_alloc(c.d_counter, sizeof(unsigned) * 16));
-    PZG_HIP(hipMemsetAsync(c.d_counter.p, 0, sizeof(unsigned) * 16, c.stream));
+    PZG_TRY(dev_alloc(c.d_flag, sizeof(int)));
   }
   PZG_TRY(dev_alloc(c.d_scal, sizeof(SolveScalars) * 2));
   PZG_TRY(dev_alloc(c.d_res2, 2 * sizeof(double)));
@@ -1025,12 +1024,13 @@ int true_residual(Ctx &c, const double *u, double *rel) {
 
 // ---- allocation-free true residual ---------------------------------------
 // Fixed device scratch of pzg_true_residual_noalloc, one copy per GPU, held
-// until the process ends: the reduction partials (2 x MAXBLK doubles, one
-// slot per workgroup of the capped residual grid) and the two sums.  32.8 KB whatever the system size, because the residual
-// kernel strides over block rows with at most MAXBLK workgroups.
+// until the process ends: the reduction partials (2 x MAXBLK doubles, one slot
+// per workgroup of the capped residual grid) and the two sums.  32.8 KB
+// whatever the system size: the residual kernels stride over the rows with at
+// most MAXBLK workgroups.
 constexpr int NOALLOC_PART = 2 * MAXBLK;           // partials, doubles
 constexpr int NOALLOC_OUT = NOALLOC_PART;          // |r|^2, |f|^2
-constexpr int NOALLOC_WORDS = NOALLOC_PART + 8;
+constexpr int NOALLOC_WORDS = NOALLOC_PART + 2;
 static __device__ __align__(256) double scratch[NOALLOC_WORDS];
 
 constexpr int NOALLOC_MAXDEV = 64;
@@ -1057,7 +1057,8 @@ int noalloc_scratch_setup(int device) {
 }
 
 // The residual of true_residual on the FP64 operator already on the device
-// (element products or full block CSR), reducing in the per-device scratch: no allocation of any kind.
+// (element products or full block CSR), reducing in the per-device scratch: no
+// allocation of any kind.
 int true_residual_noalloc(Ctx &c, double *rel) {
   if (!(c.kf_valid || (c.full_valid && c.d_fbia.p)) || !c.f_valid || !c.d_f.p) {
     set_error("pzg_true_residual_noalloc: no FP64 operator or load of the current system on the "
@@ -1307,7 +1308,7 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
       return PZG_ESTATE;
     }
     PZG_TRY(dev_alloc(c.d_bjinv64, sizeof(double) * std::max<int64_t>(c.vbj_ninv, 1)));
-    int *fail = reinterpret_cast<int *>(c.d_counter.as<unsigned>() + 8);
+    int *fail = c.d_flag.as<int>();
     PZG_HIP(hipMemsetAsync(fail, 0, sizeof(int), c.stream));
     hipLaunchKernelGGL(k_vbj_inv64, dim3((unsigned)((c.vbj_nblk + 3) / 4)), dim3(256), 0, c.stream, c.vbj_nblk,
                        c.d_vbj_pos.as<int64_t>(), c.d_vbj_m.as<int32_t>(), c.d_vbj_off.as<int64_t>(),
@@ -1326,7 +1327,7 @@ int solve_pcg64(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info) {
       return PZG_EUNSUP;
     }
     PZG_TRY(dev_alloc(c.d_bjinv64, sizeof(double) * c.nb * c.bs * c.bs));
-    int *fail = reinterpret_cast<int *>(c.d_counter.as<unsigned>() + 8);
+    int *fail = c.d_flag.as<int>();
     PZG_HIP(hipMemsetAsync(fail, 0, sizeof(int), c.stream));
     DISPATCH_BS(c.bs, hipLaunchKernelGGL(k_bj_inv64<BS>, dim3((unsigned)((c.nb + TPB - 1) / TPB)), dim3(TPB), 0,
                                          c.stream, c.nb, c.d_ia.as<int64_t>(), c.d_a.as<double>(),
@@ -1720,7 +1721,7 @@ static int mixed_impl(Ctx &c, const pzg_solve_params &prm, pzg_solve_info &info)
   if (vbj && !conv) {
     PZG_TRY(dev_alloc(c.d_vbjinv64, sizeof(double) * std::max<int64_t>(c.vbj_ninv, 1)));
     PZG_TRY(dev_alloc(c.d_vbjinv32, sizeof(float) * std::max<int64_t>(c.vbj_ninv, 1)));
-    int *fail = reinterpret_cast<int *>(c.d_counter.as<unsigned>() + 8);
+    int *fail = c.d_flag.as<int>();
     PZG_HIP(hipMemsetAsync(fail, 0, sizeof(int), c.stream));
     hipLaunchKernelGGL(k_vbj_inv64, dim3((unsigned)((c.vbj_nblk + 3) / 4)), dim3(256), 0, c.stream, c.vbj_nblk,
                        c.d_vbj_pos.as<int64_t>(), c.d_vbj_m.as<int32_t>(), c.d_vbj_off.as<int64_t>(),
