@@ -445,19 +445,19 @@ def main():
         L.check(ctx.lib.pzg_time_kernel(ctx.h, 4, 20, C.byref(avg), C.byref(nbytes)))
         el_ms, el_flops = avg.value, nbytes.value
     sizes = ctx.sizes()
-    # roofline of the dominant kernel of the measured path: the matrix-free
-    # element kernel (FP32 contractions on the matrix cores) when the inner
-    # operator is matrix-free, else the FP32 block CSR SpMV
+    # roofline of the FP32 operator of the measured path: the tiled product, the
+    # element kernel (FP32 contractions on the matrix cores) or the block CSR SpMV
     mf_used = args.inner_op != "bsr" and mf_ok
     # the counter summary covers the default workload only
     counted = args.config == "C5" and not args.n and args.seed == 0
-    # lattices of p = 2 boxes (every 3-D elasticity workload here): sum
-    # factorisation in tiles, bound by memory and not by arithmetic
+    # lattices of p = 2 boxes (every 3-D elasticity workload here): elements in
+    # Legendre modes in LDS tiles; priced against HBM, the nearest roof, held
+    # below it by LDS and memory latency
     tiled = mf_used and pb.dim == 3 and pb.p == 2 and pb.nstate == 3 and pb.el_porder is None and not pb.simplex
     if tiled:
         roofline = {"bound": "hbm", "kernel": "k_mft_tile<0> + k_mft_halo<0> (matrix-free FP32 operator)",
                     "achieved": mf_gbs, "peak": 8000.0, "unit": "GB/s", "frac": mf_gbs / 8000.0,
-                    "launch_ms": mf_ms, "flops_per_launch": el_flops,
+                    "limited_by": "LDS and memory latency", "launch_ms": mf_ms, "flops_per_launch": el_flops,
                     "traffic": traffic_of("k_mft_tile<0>") if counted else None}
     elif mf_used:
         kname = (f"k_mf_hex27_mfma<{sizes['bs']}>" if pb.dim == 3 and pb.p == 2

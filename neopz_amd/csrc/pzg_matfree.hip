@@ -511,8 +511,7 @@ __global__ __launch_bounds__(MFK_TPB) void k_mf_hex27_mfma(MfArgs a, const MfMfm
 //
 // Grids: four workgroups per CU (what the registers hold; with three, 64^3 and
 // 48^3 cells took 115 and 60 us instead of 110 and 54, in an earlier form of the
-// kernel); the partial sums of both
-// kernels together fill at most MAXBLK slots.
+// kernel); the partial sums of both kernels together fill at most MAXBLK slots.
 constexpr int MT_TILE_GRID = 1024, MT_HALO_GRID = 1024, MT_HALO_FREE = 1 << 20;
 constexpr int MT_TC = 4, MT_BN = 9, MT_NB = MT_BN * MT_BN * MT_BN, MT_W = 8;
 static_assert(MT_TILE_GRID + MT_HALO_GRID <= MAXBLK, "partial-sum slots");

@@ -161,10 +161,10 @@ __device__ inline double jac_inverse(const double (&J)[3][3], double (&ji)[3][3]
 //
 // One element per group was bound by the L1: four table values for four
 // multiply-adds, over all 56 sides of an order-5 element whatever its order.
-// 82,944 tetrahedra of orders 1 to 5, 512 points each: 8.57 ms of kernels then, 2.29
-// now with EB = 4 (247 registers, two wavefronts per SIMD); with EB = 2 the call takes
-// 2.84 ms instead of 2.76.  What is
-// left is arithmetic: the exact solution's sines and the multiply-adds.
+// 82,944 tetrahedra of orders 1 to 5, 512 points each: 8.57 ms of kernels then,
+// 2.3 now with EB = 4 (247 registers, two wavefronts per SIMD); with EB = 2 the
+// call takes 0.08 ms more.  What is left is arithmetic: the exact solution's
+// sines and the multiply-adds.
 template <int NS, bool POINTS, int EB, bool AFF>
 __global__ __launch_bounds__(PTPB) void k_post(const PostArgs a) {
   extern __shared__ double s_mem[];
