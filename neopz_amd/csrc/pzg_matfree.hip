@@ -494,8 +494,10 @@ __global__ __launch_bounds__(MFK_TPB) void k_mf_hex27_mfma(MfArgs a, const MfMfm
 // (k_mf_hex27_mfma, which stays for every other p = 2 hexahedral mesh).  Lane k
 // runs its element with the axes rotated by k (axis 0 = direction k), so the
 // components differ in the addresses they read, not in the code, and exchange
-// modes by quad permutes.  Error against FP64 at random vectors, 12^3 and 16^3
-// cells: 1.40e-7 and 1.20e-7, the dense contractions 1.37e-7 and 1.38e-7.
+// modes by quad permutes.  Error against FP64 at random vectors, 12^3 / 16^3 /
+// 48^3 cells: 1.19e-7 / 1.18e-7 / 1.18e-7, the dense contractions 1.37e-7 /
+// 1.32e-7 / 1.35e-7; at a smooth field 4.4e-7 / 5.2e-7 / 3.6e-6 against 4.9e-7 /
+// 5.6e-7 / 3.7e-6.
 //
 // Memory: the tile's 9^3 nodes are staged in LDS once (the element-major gathers
 // read every node up to 8 times from memory, in 12-byte pieces that the address
@@ -1198,6 +1200,13 @@ static int mft_setup(Ctx &c) {
   return PZG_OK;
 }
 
+// The part of an element's stiffness that goes into its FP32 coefficient: the
+// factors left for the rows (a, b1, b2) hold no edge length on cubes.  A rounded
+// edge factor in them is the same relative error in every element and does not
+// average out in the sums: 1.64e-7 on 5^3 and 1.65e-7 on 21^3 cells instead of
+// 1.24e-7 and 1.20e-7 (dense contractions 1.63e-7 and 1.46e-7).
+static double mft_unit(const Ctx &c) { return c.mf_box_det * c.mf_box_inv[0] * c.mf_box_inv[0]; }
+
 // q-rows of S pt (pt in d_mf_pt) through the tiles, finished as o says; the
 // partials (MF_OUT_Q) fill mft_grid blocks
 static int mft_apply(Ctx &c, const MfOut &o, const SolveScalars *sc) {
@@ -1222,7 +1231,7 @@ static int mft_apply(Ctx &c, const MfOut &o, const SolveScalars *sc) {
     g.bm = c.d_mf_bm.as<float>();
   }
   const double C1 = 1. / (2. + 2. * c.nu), den = -1. + c.nu + 2. * c.nu * c.nu, C2 = c.nu / den, C3 = (c.nu - 1.) / den;
-  const double *iv = c.mf_box_inv, det = c.mf_box_det;
+  const double *iv = c.mf_box_inv, det = c.mf_box_det / mft_unit(c);
   for (int k = 0; k < 3; k++)
     for (int j = 0; j < 3; j++) {
       const int m = (k + j) % 3;
@@ -1438,8 +1447,8 @@ int mf_prepare(Ctx &c) {
   if (!c.scal_valid) PZG_TRY(launch_build_bsr(c, false));
   if (c.mf_vals_valid) return PZG_OK;
   std::vector<float> coef(c.nvol);
-  const double dflt = c.material == PZG_MAT_ELAST3D ? c.E : c.scale;
-  for (int64_t e = 0; e < c.nvol; e++) coef[e] = (float)(c.vol_coef.empty() ? dflt : c.vol_coef[e]);
+  const double dflt = c.material == PZG_MAT_ELAST3D ? c.E : c.scale, unit = c.mf_tile ? mft_unit(c) : 1.;
+  for (int64_t e = 0; e < c.nvol; e++) coef[e] = (float)(unit * (c.vol_coef.empty() ? dflt : c.vol_coef[e]));
   if (c.nvol)
     PZG_HIP(hipMemcpyAsync(c.d_mf_coef.p, coef.data(), coef.size() * sizeof(float),
                            hipMemcpyHostToDevice, c.stream));

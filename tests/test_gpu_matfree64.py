@@ -1,5 +1,7 @@
-"""FP64 products with K from the element matrix (meshes of identical affine
-p = 2 hexahedra) against the oracle's assembled matrix.
+"""FP64 products on meshes of identical affine p = 2 hexahedra against the
+oracle's assembled matrix: element by element on the large mesh, by the block CSR
+on the small ones (fewer than 96 elements, 6000 with one unknown a node; both
+sides of these limits are in test_gpu_element_product_sizes.py).
 
 Bar: |K x - K_ref x| <= 1e-13 * sum_j |K_ij| |x_j| per row: both sums have at
 most a few hundred terms of that size, added in another order (64 eps = 1.4e-14
